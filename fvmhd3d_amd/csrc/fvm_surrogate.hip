@@ -8,8 +8,8 @@
 //                   V = w_n n + u_t and the MHD scaling (rho_s, c_s); the
 //                   network answers the residual over the HLL flux of the two
 //                   sides per unit normalised jump (fvm_mlp.h)
-//   training        Adam over bf16-operand MFMA GEMMs (v_mfma_f32_16x16x32_bf16,
-//                   FP32 accumulation), one kernel per GEMM / elementwise step
+//   training        Adam over bf16-operand MFMAs (v_mfma_f32_16x16x32_bf16,
+//                   FP32 accumulation), two launches a step (fvm_sg_train.h)
 //   inference       one fused kernel: each wavefront featurises 64 faces, runs
 //                   the four layers as chained MFMAs with every activation kept
 //                   in registers (the K order of each weight fragment is the
@@ -35,6 +35,7 @@
 #include "fvm_internal.h"
 #include "fvm_physics.h"
 #include "fvm_mlp.h"
+#include "fvm_sg_train.h"
 
 namespace fvm {
 namespace sg {
@@ -158,136 +159,6 @@ __global__ void k_pack_samples(int n, const int *flag, const int *pos, const flo
   const size_t i = (size_t)(base + pos[f]);
   for (int k = 0; k < NIN; k++) X[i * NIN + k] = Xs[(size_t)f * NIN + k];
   for (int k = 0; k < NOUT; k++) T[i * NOUT + k] = Ts[(size_t)f * NOUT + k];
-}
-
-// ---------------------------------------------------------------------------
-// training GEMM: C[M][N] (+)= op(A)[M][K] op(B)[K][N], op(A)[m][k] = A[m*sam + k*sak],
-// op(B)[k][n] = B[k*sbk + n*sbn]; operands rounded to bf16, FP32 accumulation.
-// 64x64 block tile, 4 wavefronts of 32x32, K step 32.
-// ---------------------------------------------------------------------------
-constexpr int GT = 64, GK = 32, GKP = GK + 8;  // LDS rows padded to 80 bytes
-
-__global__ void __launch_bounds__(256) k_gemm(int M, int N, int K, const float *__restrict__ A, long long sam,
-                                              long long sak, const float *__restrict__ B, long long sbk,
-                                              long long sbn, float *__restrict__ C, int ldc, int accumulate) {
-  __shared__ __attribute__((aligned(16))) __bf16 As[GT][GKP];
-  __shared__ __attribute__((aligned(16))) __bf16 Bs[GT][GKP];
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const int m0 = blockIdx.y * GT, n0 = blockIdx.x * GT;
-  const int wm = (w & 1) * 32, wn = (w >> 1) * 32;
-  const int g = lane >> 4, r16 = lane & 15;
-  f32x4 acc[2][2];
-  for (int i = 0; i < 2; i++)
-    for (int j = 0; j < 2; j++) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  for (int k0 = 0; k0 < K; k0 += GK) {
-    for (int q = 0; q < (GT * GK) / 256; q++) {
-      const int idx = t + 256 * q;
-      int m, k;
-      if (sak == 1) { m = idx / GK; k = idx % GK; }
-      else { m = idx % GT; k = idx / GT; }
-      const int gm = m0 + m, gk = k0 + k;
-      const float v = (gm < M && gk < K) ? A[(long long)gm * sam + (long long)gk * sak] : 0.0f;
-      As[m][k] = (__bf16)v;
-      int n;
-      if (sbn == 1) { n = idx % GT; k = idx / GT; }
-      else { n = idx / GK; k = idx % GK; }
-      const int gn = n0 + n, gk2 = k0 + k;
-      const float u = (gn < N && gk2 < K) ? B[(long long)gk2 * sbk + (long long)gn * sbn] : 0.0f;
-      Bs[n][k] = (__bf16)u;
-    }
-    __syncthreads();
-    bf16x8 a[2], b[2];
-    for (int i = 0; i < 2; i++) a[i] = *reinterpret_cast<const bf16x8 *>(&As[wm + 16 * i + r16][8 * g]);
-    for (int j = 0; j < 2; j++) b[j] = *reinterpret_cast<const bf16x8 *>(&Bs[wn + 16 * j + r16][8 * g]);
-    for (int i = 0; i < 2; i++)
-      for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
-    __syncthreads();
-  }
-  // D layout: lane holds column r16 and rows 4g..4g+3 of each 16x16 tile
-  for (int i = 0; i < 2; i++)
-    for (int j = 0; j < 2; j++) {
-      const int col = n0 + wn + 16 * j + r16;
-      for (int r = 0; r < 4; r++) {
-        const int row = m0 + wm + 16 * i + 4 * g + r;
-        if (row < M && col < N) {
-          float *p = C + (long long)row * ldc + col;
-          *p = accumulate ? *p + acc[i][j][r] : acc[i][j][r];
-        }
-      }
-    }
-}
-
-// H[r][c] = act(H[r][c] + b[c])
-__global__ void k_bias_act(float *H, const float *b, int rows, int cols, int relu) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (long long)rows * cols) return;
-  const float v = H[i] + b[i % cols];
-  H[i] = relu ? fmaxf(v, 0.0f) : v;
-}
-// D *= (H > 0)
-__global__ void k_relu_mask(float *D, const float *H, long long n) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n && !(H[i] > 0.0f)) D[i] = 0.0f;
-}
-// out[c] = sum_r D[r][c]; 64 columns per block, fixed summation order
-__global__ void __launch_bounds__(256) k_colsum(const float *D, int rows, int cols, float *out) {
-  __shared__ float part[4][64];
-  const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-  const int c = blockIdx.x * 64 + tx;
-  float s = 0.0f;
-  if (c < cols)
-    for (int r = ty; r < rows; r += 4) s += D[(long long)r * cols + c];
-  part[ty][tx] = s;
-  __syncthreads();
-  if (ty == 0 && c < cols) out[c] = (part[0][tx] + part[1][tx]) + (part[2][tx] + part[3][tx]);
-}
-// loss terms and dL/dy for a batch (outputs 0..6 fluxes weighted by w, 7 confidence)
-struct LossW {
-  float w[7];
-};
-__global__ void k_loss(const float *Y, const float *T, int B, float lam, LossW lw, float *dY, float *loss_acc) {
-  const int i = gid();
-  float l = 0.0f;
-  if (i < B) {
-    float e2 = 0.0f, d[7];
-    for (int k = 0; k < 7; k++) {
-      d[k] = Y[(size_t)i * NOUT + k] - T[(size_t)i * NOUT + k];
-      e2 += lw.w[k] * d[k] * d[k];
-    }
-    const float c = log10f(e2 + 1e-10f);
-    const float dc = Y[(size_t)i * NOUT + 7] - c;
-    const float iB = 1.0f / (float)B;
-    for (int k = 0; k < 7; k++) dY[(size_t)i * NOUT + k] = 2.0f * lw.w[k] * d[k] * iB;
-    dY[(size_t)i * NOUT + 7] = 2.0f * lam * dc * iB;
-    l = (e2 + lam * dc * dc) * iB;
-  }
-  for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o);
-  if (__lane_id() == 0) atomicAdd(loss_acc, l);
-}
-__global__ void k_adam(float *P, const float *G, float *Mm, float *Vv, int n, float lr, float b1, float b2, float eps,
-                       float c1, float c2) {
-  const int i = gid();
-  if (i >= n) return;
-  const float g = G[i];
-  const float m = b1 * Mm[i] + (1.0f - b1) * g;
-  const float v = b2 * Vv[i] + (1.0f - b2) * g * g;
-  Mm[i] = m;
-  Vv[i] = v;
-  P[i] -= lr * (m / c1) / (sqrtf(v / c2) + eps);
-}
-__device__ __forceinline__ unsigned long long splitmix(unsigned long long z) {
-  z += 0x9E3779B97F4A7C15ULL;
-  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ULL;
-  z = (z ^ (z >> 27)) * 0x94D049BB133111EBULL;
-  return z ^ (z >> 31);
-}
-__global__ void k_gather(const float *X, const float *T, long long nsamp, int B, unsigned long long seed,
-                         unsigned long long step, float *Xb, float *Tb) {
-  const int i = gid();
-  if (i >= B) return;
-  const long long s = (long long)(splitmix(seed ^ splitmix((step << 32) ^ (unsigned long long)i)) % (unsigned long long)nsamp);
-  for (int k = 0; k < NIN; k++) Xb[(size_t)i * NIN + k] = X[(size_t)s * NIN + k];
-  for (int k = 0; k < NOUT; k++) Tb[(size_t)i * NOUT + k] = T[(size_t)s * NOUT + k];
 }
 
 // ---------------------------------------------------------------------------
@@ -526,8 +397,8 @@ struct fvm_sg {
   Buf params, grads, am, av, pfrag, pbias;
   Buf X, T;
   long long nsamp = 0, cap = 0;
-  Buf xb, tb, h[3], y, dy, d[2], loss;
-  int bcap = 0;
+  Buf xb, tb, y, loss;     // fvm_sg_gradients' batch and outputs; the steps' losses
+  Buf tfrag, tops, tcols, tloss;  // training: packed weights; the tiles' operands, FP32 gradients and losses
   Buf stage, fbl, fbc;
   Buf sx, st, sflag, spos;  // sample staging of one add_faces call
   fvm::ScanScratch scan;
@@ -564,64 +435,45 @@ static int sg_ensure(fvm_sg *s, Buf &b, size_t bytes, bool keep = false) {
 }
 static unsigned nblk(long long n, int b = 256) { return (unsigned)((n + b - 1) / b); }
 
-static int gemm(fvm_sg *s, int M, int N, int K, const float *A, long long sam, long long sak, const float *B,
-                long long sbk, long long sbn, float *C, int ldc, int accumulate) {
-  dim3 grid((unsigned)((N + GT - 1) / GT), (unsigned)((M + GT - 1) / GT));
-  hipLaunchKernelGGL(k_gemm, grid, dim3(256), 0, s->stream, M, N, K, A, sam, sak, B, sbk, sbn, C, ldc, accumulate);
+// fragments of the current parameters for the training kernels; their padding
+// is cleared when they are first allocated
+static int train_pack(fvm_sg *s) {
+  if (!s->tfrag.p) {
+    int rc = sg_ensure(s, s->tfrag, sizeof(__bf16) * (size_t)T_FRAG);
+    if (rc) return rc;
+    SGCHK(s, hipMemsetAsync(s->tfrag.p, 0, s->tfrag.bytes, s->stream));
+  }
+  hipLaunchKernelGGL(k_train_pack, dim3(nblk(NPARAM)), dim3(256), 0, s->stream, (const float *)s->params.p,
+                     (__bf16 *)s->tfrag.p);
   SGCHK(s, hipGetLastError());
   return FVM_OK;
 }
-
-static int ensure_batch(fvm_sg *s, int B) {
-  if (B <= s->bcap) return FVM_OK;
+// buffers of a batch of B samples, and what both launches of a step share
+static int train_args(fvm_sg *s, int B, float lam, TrainArgs &A, GradArgs &D) {
+  const size_t nt = ((size_t)B + TS - 1) / TS;
   int rc;
-  const size_t b = (size_t)B;
-  if ((rc = sg_ensure(s, s->xb, 4 * b * NIN)) || (rc = sg_ensure(s, s->tb, 4 * b * NOUT)) ||
-      (rc = sg_ensure(s, s->h[0], 4 * b * NH)) || (rc = sg_ensure(s, s->h[1], 4 * b * NH)) ||
-      (rc = sg_ensure(s, s->h[2], 4 * b * NH)) || (rc = sg_ensure(s, s->y, 4 * b * NOUT)) ||
-      (rc = sg_ensure(s, s->dy, 4 * b * NOUT)) || (rc = sg_ensure(s, s->d[0], 4 * b * NH)) ||
-      (rc = sg_ensure(s, s->d[1], 4 * b * NH)) || (rc = sg_ensure(s, s->loss, 4 * 1024)))
+  if ((rc = train_pack(s)) || (rc = sg_ensure(s, s->tops, sizeof(__bf16) * N_OP * OP_E * nt)) ||
+      (rc = sg_ensure(s, s->tcols, sizeof(float) * N_COL * COL_E * nt)) || (rc = sg_ensure(s, s->tloss, sizeof(float) * nt)))
     return rc;
-  s->bcap = B;
-  return FVM_OK;
-}
-
-// forward + loss + backward on the batch in xb/tb; loss accumulated into loss[slot]
-static int fwd_bwd(fvm_sg *s, int B, float lam, int slot) {
-  const float *P = (const float *)s->params.p;
-  float *G = (float *)s->grads.p;
-  const float *X = (const float *)s->xb.p;
-  float *H0 = (float *)s->h[0].p, *H1 = (float *)s->h[1].p, *H2 = (float *)s->h[2].p;
-  float *Y = (float *)s->y.p, *dY = (float *)s->dy.p, *D0 = (float *)s->d[0].p, *D1 = (float *)s->d[1].p;
-  int rc;
-  const long long bh = (long long)B * NH;
-  // forward
-  if ((rc = gemm(s, B, NH, NIN, X, NIN, 1, P + OW0, NH, 1, H0, NH, 0))) return rc;
-  hipLaunchKernelGGL(k_bias_act, dim3(nblk(bh)), dim3(256), 0, s->stream, H0, P + OB0, B, NH, 1);
-  if ((rc = gemm(s, B, NH, NH, H0, NH, 1, P + OW1, NH, 1, H1, NH, 0))) return rc;
-  hipLaunchKernelGGL(k_bias_act, dim3(nblk(bh)), dim3(256), 0, s->stream, H1, P + OB1, B, NH, 1);
-  if ((rc = gemm(s, B, NH, NH, H1, NH, 1, P + OW2, NH, 1, H2, NH, 0))) return rc;
-  hipLaunchKernelGGL(k_bias_act, dim3(nblk(bh)), dim3(256), 0, s->stream, H2, P + OB2, B, NH, 1);
-  if ((rc = gemm(s, B, NOUT, NH, H2, NH, 1, P + OW3, NOUT, 1, Y, NOUT, 0))) return rc;
-  hipLaunchKernelGGL(k_bias_act, dim3(nblk((long long)B * NOUT)), dim3(256), 0, s->stream, Y, P + OB3, B, NOUT, 0);
-  hipLaunchKernelGGL(k_loss, dim3(nblk(B)), dim3(256), 0, s->stream, Y, (const float *)s->tb.p, B, lam, s->lossw, dY,
-                     (float *)s->loss.p + slot);
-  // backward
-  if ((rc = gemm(s, NH, NOUT, B, H2, 1, NH, dY, NOUT, 1, G + OW3, NOUT, 0))) return rc;
-  hipLaunchKernelGGL(k_colsum, dim3(nblk(NOUT, 64)), dim3(256), 0, s->stream, dY, B, NOUT, G + OB3);
-  if ((rc = gemm(s, B, NH, NOUT, dY, NOUT, 1, P + OW3, 1, NOUT, D0, NH, 0))) return rc;
-  hipLaunchKernelGGL(k_relu_mask, dim3(nblk(bh)), dim3(256), 0, s->stream, D0, H2, bh);
-  if ((rc = gemm(s, NH, NH, B, H1, 1, NH, D0, NH, 1, G + OW2, NH, 0))) return rc;
-  hipLaunchKernelGGL(k_colsum, dim3(nblk(NH, 64)), dim3(256), 0, s->stream, D0, B, NH, G + OB2);
-  if ((rc = gemm(s, B, NH, NH, D0, NH, 1, P + OW2, 1, NH, D1, NH, 0))) return rc;
-  hipLaunchKernelGGL(k_relu_mask, dim3(nblk(bh)), dim3(256), 0, s->stream, D1, H1, bh);
-  if ((rc = gemm(s, NH, NH, B, H0, 1, NH, D1, NH, 1, G + OW1, NH, 0))) return rc;
-  hipLaunchKernelGGL(k_colsum, dim3(nblk(NH, 64)), dim3(256), 0, s->stream, D1, B, NH, G + OB1);
-  if ((rc = gemm(s, B, NH, NH, D1, NH, 1, P + OW1, 1, NH, D0, NH, 0))) return rc;
-  hipLaunchKernelGGL(k_relu_mask, dim3(nblk(bh)), dim3(256), 0, s->stream, D0, H0, bh);
-  if ((rc = gemm(s, NIN, NH, B, X, 1, NIN, D0, NH, 1, G + OW0, NH, 0))) return rc;
-  hipLaunchKernelGGL(k_colsum, dim3(nblk(NH, 64)), dim3(256), 0, s->stream, D0, B, NH, G + OB0);
-  SGCHK(s, hipGetLastError());
+  A = TrainArgs{};
+  A.B = B;
+  A.frag = (const __bf16 *)s->tfrag.p;
+  A.P = (const float *)s->params.p;
+  A.lam = lam;
+  A.lw = s->lossw;
+  A.ops = (__bf16 *)s->tops.p;
+  A.cols = (float *)s->tcols.p;
+  A.tloss = (float *)s->tloss.p;
+  D = GradArgs{};
+  D.ntile = (int)nt;
+  D.ops = A.ops;
+  D.cols = A.cols;
+  D.tloss = A.tloss;
+  D.G = (float *)s->grads.p;
+  D.P = (float *)s->params.p;
+  D.M = (float *)s->am.p;
+  D.V = (float *)s->av.p;
+  D.frag = (__bf16 *)s->tfrag.p;
   return FVM_OK;
 }
 
@@ -705,8 +557,8 @@ int fvm_sg_create(fvm_sg **out, int device, double gamma_gas) {
 void fvm_sg_destroy(fvm_sg *s) {
   if (!s) return;
   (void)hipSetDevice(s->device);
-  for (Buf *b : {&s->params, &s->grads, &s->am, &s->av, &s->pfrag, &s->pbias, &s->X, &s->T, &s->xb, &s->tb, &s->h[0],
-                 &s->h[1], &s->h[2], &s->y, &s->dy, &s->d[0], &s->d[1], &s->loss, &s->stage, &s->fbl, &s->fbc,
+  for (Buf *b : {&s->params, &s->grads, &s->am, &s->av, &s->pfrag, &s->pbias, &s->X, &s->T, &s->xb, &s->tb, &s->y,
+                 &s->loss, &s->tfrag, &s->tops, &s->tcols, &s->tloss, &s->stage, &s->fbl, &s->fbc,
                  &s->sx, &s->st, &s->sflag, &s->spos})
     sg_release(*b);
   fvm::scan_release(s->scan);
@@ -839,19 +691,25 @@ int fvm_sg_train(fvm_sg *s, int steps, int batch, double lr, double lam, unsigne
   if (s->nsamp < 1) return sg_fail(s, FVM_ESTATE, "train: no samples");
   (void)hipSetDevice(s->device);
   int rc;
-  if ((rc = ensure_batch(s, batch)) || (rc = sg_ensure(s, s->loss, 4 * (size_t)std::max(steps, 1)))) return rc;
-  SGCHK(s, hipMemsetAsync(s->loss.p, 0, 4 * (size_t)std::max(steps, 1), s->stream));
-  const float b1 = 0.9f, b2 = 0.999f;
+  TrainArgs A;
+  GradArgs D;
+  if ((rc = train_args(s, batch, (float)lam, A, D)) || (rc = sg_ensure(s, s->loss, 4 * (size_t)std::max(steps, 1)))) return rc;
+  A.X = (const float *)s->X.p;
+  A.T = (const float *)s->T.p;
+  A.nsamp = s->nsamp;
+  A.seed = seed;
+  D.lr = (float)lr;
+  D.b1 = 0.9f;
+  D.b2 = 0.999f;
+  D.eps = 1e-8f;
   for (int k = 0; k < steps; k++) {
-    hipLaunchKernelGGL(k_gather, dim3(nblk(batch)), dim3(256), 0, s->stream, (const float *)s->X.p,
-                       (const float *)s->T.p, s->nsamp, batch, seed, (unsigned long long)s->adam_t,
-                       (float *)s->xb.p, (float *)s->tb.p);
-    if ((rc = fwd_bwd(s, batch, (float)lam, k))) return rc;
+    A.step = (unsigned long long)s->adam_t;
+    hipLaunchKernelGGL(k_train_tile<true>, dim3(D.ntile), dim3(TB), 0, s->stream, A);
     s->adam_t++;
-    const float c1 = 1.0f - powf(b1, (float)s->adam_t), c2 = 1.0f - powf(b2, (float)s->adam_t);
-    hipLaunchKernelGGL(k_adam, dim3(nblk(NPARAM)), dim3(256), 0, s->stream, (float *)s->params.p,
-                       (const float *)s->grads.p, (float *)s->am.p, (float *)s->av.p, NPARAM, (float)lr, b1, b2, 1e-8f,
-                       c1, c2);
+    D.c1 = 1.0f - powf(D.b1, (float)s->adam_t);
+    D.c2 = 1.0f - powf(D.b2, (float)s->adam_t);
+    D.loss = (float *)s->loss.p + k;
+    hipLaunchKernelGGL(k_train_grad<true>, dim3(GRAD_BLOCKS), dim3(64), 0, s->stream, D);
     SGCHK(s, hipGetLastError());
   }
   s->packed = false;
@@ -866,11 +724,21 @@ int fvm_sg_gradients(fvm_sg *s, int n, const float *x, const float *t, double la
   if (!s || n < 1 || !x || !t) return sg_fail(s, FVM_EARG, "gradients: bad arguments");
   (void)hipSetDevice(s->device);
   int rc;
-  if ((rc = ensure_batch(s, n))) return rc;
+  TrainArgs A;
+  GradArgs D;
+  if ((rc = train_args(s, n, (float)lam, A, D)) || (rc = sg_ensure(s, s->xb, 4 * (size_t)n * NIN)) ||
+      (rc = sg_ensure(s, s->tb, 4 * (size_t)n * NOUT)) || (rc = sg_ensure(s, s->y, 4 * (size_t)n * NOUT)) ||
+      (rc = sg_ensure(s, s->loss, 4)))
+    return rc;
   SGCHK(s, hipMemcpyAsync(s->xb.p, x, 4 * (size_t)n * NIN, hipMemcpyHostToDevice, s->stream));
   SGCHK(s, hipMemcpyAsync(s->tb.p, t, 4 * (size_t)n * NOUT, hipMemcpyHostToDevice, s->stream));
-  SGCHK(s, hipMemsetAsync(s->loss.p, 0, 4, s->stream));
-  if ((rc = fwd_bwd(s, n, (float)lam, 0))) return rc;
+  A.X = (const float *)s->xb.p;
+  A.T = (const float *)s->tb.p;
+  A.Y = (float *)s->y.p;
+  D.loss = (float *)s->loss.p;
+  hipLaunchKernelGGL(k_train_tile<false>, dim3(D.ntile), dim3(TB), 0, s->stream, A);
+  hipLaunchKernelGGL(k_train_grad<false>, dim3(GRAD_BLOCKS), dim3(64), 0, s->stream, D);
+  SGCHK(s, hipGetLastError());
   float l = 0.0f;
   if (y) SGCHK(s, hipMemcpyAsync(y, s->y.p, 4 * (size_t)n * NOUT, hipMemcpyDeviceToHost, s->stream));
   if (grads) SGCHK(s, hipMemcpyAsync(grads, s->grads.p, 4 * (size_t)NPARAM, hipMemcpyDeviceToHost, s->stream));

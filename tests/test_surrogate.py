@@ -221,6 +221,35 @@ def test_gpu_gradients_match_oracle():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 31, 33, 8191, 8192 + 33])
+def test_gpu_gradients_at_tile_edges(n):
+    """Batches around the 32-sample tiles of the training kernel and past one tile
+    per block (256 blocks); operands are rounded to bf16 as the oracle rounds
+    them, so what differs is a value within FP32 rounding of a bf16 tie (2^-8 of
+    that value, one of 128 terms) and the order of the FP32 sums."""
+    from fvmhd3d_amd.surrogate import Surrogate
+    rng = np.random.default_rng(n)
+    P = R.init_params(11)
+    for k in P:
+        if k.startswith("b"):
+            P[k] = rng.normal(0, 0.1, P[k].shape)
+    sg = Surrogate(params=P)
+    P = {k: v.astype(np.float32).astype(np.float64) for k, v in sg.params().items()}
+    x = rng.normal(0, 1, (n, R.N_IN)).astype(np.float32)
+    t = np.zeros((n, 8), np.float32)
+    t[:, :7] = rng.normal(0, 1, (n, 7))
+    y, G, loss = sg.gradients(x, t, lam=0.05)
+    yo, cache = R.forward(P, x.astype(np.float64))
+    lo, dy = R.loss_and_dy(yo, t[:, :7].astype(np.float64), 0.05)
+    Go = R.backward(P, cache, dy)
+    assert _rel_fro(y, yo) < 2e-3
+    assert abs(loss - lo) < 2e-3 * lo
+    for k in Go:
+        assert _rel_fro(G[k], Go[k]) < 1e-2, k
+    sg.close()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("n", [1, 63, 65, 1000, 5000])
 def test_gpu_inference_kernel_matches_oracle(n):
     from fvmhd3d_amd.surrogate import Surrogate

@@ -70,7 +70,7 @@ struct SubstepState {
   bool ready = false;
   bool complete = false;  // the global cell lists list every face under each of its cells
   int n = 0, nface = 0, nref = 0;
-  DBuf gs1, gs2, gc, gn, goff, gface, gvol;  // global mesh (SoA)
+  DBuf gs1, gs2, gc, gn, goff, gface, gnbr, gvol;  // global mesh (SoA; gnbr: the other cell of every gface entry)
   DBuf g[FVM_NFIELDS];                        // global fields, SoA [k*n + i]
   DBuf rung;                                  // int per cell
   DBuf act, apos, fmark, fpos, fl, cmark, iflag, ipos, g2l, perm, len, hist, err;
@@ -115,6 +115,7 @@ struct fvm_ctx {
   // (fvm_set_face_precision)
   bool face32 = false;
   DBuf field[FVM_NFIELDS];
+  DBuf m_cnbr;  // the other cell of every m_cface entry
   DBuf m_s1, m_s2, m_c, m_n, m_coff, m_cface, m_cvol, m_fact, m_soff, m_sent;
   DBuf m_cn;  // per-face geometry record (centroid, n) of the same faces as m_c / m_n
   DBuf rec, swp, tmp0, tmp1, tmp2, stage;

@@ -162,21 +162,24 @@ __global__ void k_sub_face_counts(const int *__restrict__ A, int nA, const int *
   len[j] = goff[A[j] + 1] - goff[A[j]];
 }
 
-// local cell lists (local face ids, in the order of the global list) and volumes
+// local cell lists (local face ids and neighbours, in the order of the global
+// list) and volumes; 16 lanes per cell, a list entry each
+constexpr int kLanes = 16;
 __global__ void k_sub_local_cells(const int *__restrict__ A, int nA, const int *__restrict__ goff,
-                              const int *__restrict__ gface, const int *__restrict__ fpos,
-                              const double *__restrict__ gvol, const int *__restrict__ coff, int *__restrict__ cface,
-                              double *__restrict__ cvol) {
-  const int j = gidx();
+                              const int *__restrict__ gface, const int *__restrict__ gnbr, const int *__restrict__ fpos,
+                              const int *__restrict__ g2l, const double *__restrict__ gvol, const int *__restrict__ coff,
+                              int *__restrict__ cface, int *__restrict__ cnbr, double *__restrict__ cvol) {
+  const int t = gidx();
+  const int j = t / kLanes, l = t & (kLanes - 1);
   if (j >= nA) return;
   const int g = A[j];
   const int e0 = goff[g], ne = goff[g + 1] - e0, o = coff[j];
-  for (int e = 0; e < ne; e++) cface[o + e] = fpos[gface[e0 + e]];
-  cvol[j] = gvol[g];
+  for (int e = l; e < ne; e += kLanes) {
+    cface[o + e] = fpos[gface[e0 + e]];
+    cnbr[o + e] = g2l[gnbr[e0 + e]];
+  }
+  if (l == 0) cvol[j] = gvol[g];
 }
-
-
-
 
 // new rungs of the active cells from dt_new (Scheduler.h get_rung with the
 // driver's clamp, Iterate.cpp:146-168): exponent difference to dtmax, at
@@ -525,7 +528,7 @@ void sparse_sweep(const int *off, const int *nbr, const int *rank, const int *or
 
 void fvm_substep_release(fvm_ctx *c) {
   SubstepState &s = c->sub;
-  for (DBuf *b : {&s.gs1, &s.gs2, &s.gc, &s.gn, &s.goff, &s.gface, &s.gvol, &s.rung, &s.act, &s.apos, &s.fmark,
+  for (DBuf *b : {&s.gs1, &s.gs2, &s.gc, &s.gn, &s.goff, &s.gface, &s.gnbr, &s.gvol, &s.rung, &s.act, &s.apos, &s.fmark,
                   &s.fpos, &s.fl, &s.cmark, &s.iflag, &s.ipos, &s.g2l, &s.perm, &s.len, &s.hist, &s.err, &s.sdti,
                   &s.hot, &s.hpos, &s.hlist, &s.chg, &s.dtig, &s.rankg, &s.seq, &s.okey,
                   &s.okey2, &s.oval2, &s.otmp})
@@ -618,8 +621,9 @@ int build_layout(fvm_ctx *c, unsigned mask, double t_global, int check, int *cou
   } else {
     SLAUNCH(c, 1, k_sub_fill_i, P<int>(c->m_coff), 1, 0);
   }
-  SLAUNCH(c, nA, k_sub_local_cells, P<int>(s.perm), nA, P<int>(s.goff), P<int>(s.gface), P<int>(s.fpos), P<double>(s.gvol),
-          P<int>(c->m_coff), P<int>(c->m_cface), P<double>(c->m_cvol));
+  SLAUNCH(c, (long long)nA * kLanes, k_sub_local_cells, P<int>(s.perm), nA, P<int>(s.goff), P<int>(s.gface), P<int>(s.gnbr),
+          P<int>(s.fpos), P<int>(s.g2l), P<double>(s.gvol), P<int>(c->m_coff), P<int>(c->m_cface), P<int>(c->m_cnbr),
+          P<double>(c->m_cvol));
   SCHK(c, hipStreamSynchronize(st));
   if (npl <= 0 || nref < 0 || nref > s.nref || nfl > nface)
     return fvm_fail(c, FVM_ESTATE, "substep: empty or inconsistent layout");
@@ -813,7 +817,7 @@ int fvm_substep_setup(fvm_ctx *c, int ncell, int nface, const fvm_face *faces, c
   const size_t N = (size_t)ncell, F = (size_t)nface;
   int rc;
   if ((rc = ensure_all(c, {{&s.gs1, 4 * F}, {&s.gs2, 4 * F}, {&s.gc, 24 * F}, {&s.gn, 24 * F}, {&s.goff, 4 * (N + 1)},
-                           {&s.gface, 4 * (size_t)nref}, {&s.gvol, 8 * N}, {&s.rung, 4 * N}, {&s.act, 4 * N},
+                           {&s.gface, 4 * (size_t)nref}, {&s.gnbr, 4 * (size_t)nref}, {&s.gvol, 8 * N}, {&s.rung, 4 * N}, {&s.act, 4 * N},
                            {&s.apos, 4 * N}, {&s.fmark, 4 * F}, {&s.fpos, 4 * F}, {&s.fl, 4 * F}, {&s.cmark, 4 * N},
                            {&s.iflag, 4 * N}, {&s.ipos, 4 * N}, {&s.g2l, 4 * N}, {&s.perm, 4 * N}, {&s.len, 4 * N},
                            {&s.hist, 4 * kRungMax}, {&s.err, 4}, {&s.sdti, 8 * N}, {&s.hot, 4 * N},
@@ -858,7 +862,7 @@ int fvm_substep_setup(fvm_ctx *c, int ncell, int nface, const fvm_face *faces, c
   // cell local), so that no substep grows a buffer
   const size_t R = (size_t)nref;
   if ((rc = ensure_all(c, {{&c->m_s1, 4 * F}, {&c->m_s2, 4 * F}, {&c->m_c, 24 * F}, {&c->m_n, 24 * F}, {&c->m_cn, 48 * F},
-                           {&c->m_coff, 4 * (N + 1)}, {&c->m_cface, 4 * R}, {&c->m_cvol, 8 * N},
+                           {&c->m_coff, 4 * (N + 1)}, {&c->m_cface, 4 * R}, {&c->m_cnbr, 4 * R}, {&c->m_cvol, 8 * N},
                            {&c->m_soff, 4 * (N + 1)}, {&c->m_sent, 8 * F + 4}, {&c->m_fact, 4 * (F + 1)},
                            {&c->tmp0, 4 * (std::max(N, R) + 1)}, {&c->tmp1, 4 * (std::max(F, R) + 1)},
                            {&c->tmp2, 4 * (R + 1)}, {&c->rec, 8 * 15 * F} /* 15-double face records */,
@@ -892,7 +896,10 @@ int fvm_substep_setup(fvm_ctx *c, int ncell, int nface, const fvm_face *faces, c
     SCHK(c, hipMemcpy(s.gn.p, nn.data(), 24 * F, hipMemcpyHostToDevice));
   }
   SCHK(c, hipMemcpy(s.goff.p, cell_face_off, 4 * (N + 1), hipMemcpyHostToDevice));
-  if (nref > 0) SCHK(c, hipMemcpy(s.gface.p, cell_face, 4 * (size_t)nref, hipMemcpyHostToDevice));
+  if (nref > 0) {
+    SCHK(c, hipMemcpy(s.gface.p, cell_face, 4 * (size_t)nref, hipMemcpyHostToDevice));
+    SCHK(c, hipMemcpy(s.gnbr.p, s.hnbr.data(), 4 * (size_t)nref, hipMemcpyHostToDevice));
+  }
   SCHK(c, hipMemcpy(s.gvol.p, cell_volume, 8 * N, hipMemcpyHostToDevice));
   SCHK(c, hipStreamSynchronize(c->stream));
   // first use of the host handover buffers and of the copy paths happens

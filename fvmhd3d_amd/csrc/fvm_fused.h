@@ -215,10 +215,6 @@ __device__ __forceinline__ void decode_fe(const FaceEndRec<T> &r, FE<T> &g) {
   }
 }
 
-template <typename T>
-__device__ __forceinline__ void load_fe(const FusedArgs<T> &A, int e, FE<T> &g) {
-  decode_fe(A.fe[e], g);
-}
 __device__ __forceinline__ int fe_nbr(int nbr) { return nbr >= 0 ? nbr : ~nbr; }
 
 // face velocity with Springel's correction (computeFluidUpdate.cpp:194-207), canonical orientation
@@ -664,16 +660,20 @@ k_cfl_predict_recon(FusedArgs<T> A) {
           gz[k] = gg[2 * NF + k];
         }
       } else if constexpr (LIMIT) {
-        T lm[NF];
-        for (int k = 0; k < NF; k++) lm[k] = T(1.0);
+        // extremes of the limiter's argument over the faces, divided once a
+        // variable (64^3 cells: this kernel 487 -> 376 us)
+        T lm[NF], lo[NF], hi[NF];
+        for (int k = 0; k < NF; k++) lo[k] = hi[k] = T(0.0);
         for (int q = 0, e = e0; q < deg; q++, e += 64) {
-          FE<T> fe;
-          load_fe(A, e, fe);
+          const T *cen = A.fe[e].cen;
+          const T c0 = cen[0], c1 = cen[1], c2 = cen[2];
           for (int k = 0; k < NF; k++) {
-            const T dWx = gx[k] * fe.cen[0] + gy[k] * fe.cen[1] + gz[k] * fe.cen[2];
-            lm[k] = smin(lm[k], limiter_rec_c<LIM, T>(dWx, dmn[k], dmx[k]));
+            const T d = gx[k] * c0 + gy[k] * c1 + gz[k] * c2;
+            lo[k] = __builtin_fmin(lo[k], d);
+            hi[k] = __builtin_fmax(hi[k], d);
           }
         }
+        for (int k = 0; k < NF; k++) lm[k] = limiter_of_extremes<false>(LIM, lo[k], hi[k], dmn[k], dmx[k]);
         for (int k = 0; k < NF; k++) {
           SF(A.mm, k, c, n) = dmn[k] + Wc[k];
           SF(A.mm, NF + k, c, n) = dmx[k] + Wc[k];
@@ -721,7 +721,8 @@ k_cfl_predict_recon(FusedArgs<T> A) {
 // ---------------------------------------------------------------------------
 // K1b (opt-in limiters, FP64 path): slopeLimiter compute part +
 // computeFluidUpdateI for the global step, per cell over its own face-ends
-// (own data only)
+// (own data only).  The extremes of the limiter's argument are tracked and
+// divided once a variable (64^3 cells: 184 -> 144 us a launch).
 // ---------------------------------------------------------------------------
 template <typename T, int LIM>
 __global__ void __launch_bounds__(FB) k_limit(FusedArgs<T> A) {
@@ -746,8 +747,8 @@ __global__ void __launch_bounds__(FB) k_limit(FusedArgs<T> A) {
     lo[k] = smin(lo[k], T(0.0));
     hi[k] = smax(hi[k], T(0.0));
   }
-  T lm[NF];
-  for (int k = 0; k < NF; k++) lm[k] = T(1.0);
+  T lm[NF], dmin[NF], dmax[NF];  // extremes of the limiter's argument over the faces
+  for (int k = 0; k < NF; k++) dmin[k] = dmax[k] = T(0.0);
   const T dtt = (T)(dtI - dth);
   const int deg = A.deg[c];
   const int e0 = A.gbase[c >> 6] + (c & 63);
@@ -761,10 +762,12 @@ __global__ void __launch_bounds__(FB) k_limit(FusedArgs<T> A) {
     const T *dr = fe.isL ? fe.drL : fe.drR;
     for (int k = 0; k < NF; k++) {
       const T dW = gg[k] * dr[0] + gg[NF + k] * dr[1] + gg[2 * NF + k] * dr[2] + tv[k] * dtt;
-      lm[k] = smin(lm[k], limiter_sl_c<LIM, T>(dW, lo[k], hi[k]));
+      dmin[k] = __builtin_fmin(dmin[k], dW);
+      dmax[k] = __builtin_fmax(dmax[k], dW);
     }
   }
   for (int k = 0; k < NF; k++) {
+    lm[k] = limiter_of_extremes<true>(LIM, dmin[k], dmax[k], lo[k], hi[k]);
     tv[k] *= lm[k];
     gg[k] *= lm[k];
     gg[NF + k] *= lm[k];

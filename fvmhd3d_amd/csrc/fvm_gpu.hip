@@ -190,22 +190,6 @@ __device__ __forceinline__ int wave_cells_max(int v) {
   return __builtin_amdgcn_readfirstlane(max(v, __shfl_xor(v, 32)));
 }
 
-// min(1, min over faces of the limiter) from the extremes dmin, dmax of its
-// argument d_f.  Phi rises up to Phi = 1 and stays >= 1 beyond, and bound / d is
-// monotone in d under rounding, so the smallest Phi is that of the largest |d|
-// on each side; a side within the flat threshold has no face that counts.  Two
-// division chains a variable instead of one a variable and face (equal unless
-// two faces' d agree to the last bits, where Phi's own rounding may differ by
-// an ulp).  The extremes skip NaN, as the reference's min does.
-template <bool SL>
-__device__ __forceinline__ double limiter_of_extremes(int mode, double dmin, double dmax, double mn, double mx) {
-  const double tau = 1.0e-16 * smax(dabs(mx), dabs(mn));
-  double lim = 1.0;
-  if (dmax > tau) lim = smin(lim, phi(mode, SL ? mx / dmax : mx * (1.0 / dmax)));
-  if (dmin < -tau) lim = smin(lim, phi(mode, SL ? mn / dmin : mn * (1.0 / dmin)));
-  return lim;
-}
-
 // System::computeReconstruction (computeReconstruction.cpp:42-264).
 // Bound by the latency of its gathers (cell list -> face -> neighbour -> W) and
 // of the FP64 geometry: with a face a lane each is paid once a cell instead of

@@ -86,22 +86,25 @@ __device__ __forceinline__ double phi(int mode, double x) {
   const double fac = 0.2, eps1 = 1.0e-16;
   return (x * x + 2.0 * x + fac * eps1) / (x * x + x + 2.0 + fac * eps1);
 }
-// computeReconstruction.cpp:19-40
-__device__ __forceinline__ double limiter_rec(int mode, double dWi, double mn, double mx) {
-  if (dabs(dWi) <= 1.0e-16 * smax(dabs(mx), dabs(mn))) return 1.0;
-  const double invWi = 1.0 / dWi;
-  if (dWi < 0.0) return phi(mode, mn * invWi);
-  return phi(mode, mx * invWi);
-}
-// slopeLimiter.cpp:20-25
-__device__ __forceinline__ double limiter_sl(int mode, double dWi, double mn, double mx) {
-  if (dabs(dWi) <= 1.0e-16 * smax(dabs(mx), dabs(mn))) return 1.0;
-  if (dWi < 0.0) return phi(mode, mn / dWi);
-  return phi(mode, mx / dWi);
+// limiter_rec (computeReconstruction.cpp:19-40) and limiter_sl (SL,
+// slopeLimiter.cpp:20-25) over all faces of a cell and variable:
+// min(1, min over faces of the limiter) from the extremes dmin, dmax of its
+// argument d_f.  Phi rises up to Phi = 1 and stays >= 1 beyond, and bound / d is
+// monotone in d under rounding, so the smallest Phi is that of the largest |d|
+// on each side; a side within the flat threshold has no face that counts.  Two
+// division chains a variable instead of one a variable and face (equal unless
+// two faces' d agree to the last bits, where Phi's own rounding may differ by
+// an ulp).  The extremes skip NaN, as the reference's min does.
+template <bool SL>
+__device__ __forceinline__ double limiter_of_extremes(int mode, double dmin, double dmax, double mn, double mx) {
+  const double tau = 1.0e-16 * smax(dabs(mx), dabs(mn));
+  double lim = 1.0;
+  if (dmax > tau) lim = smin(lim, phi(mode, SL ? mx / dmax : mx * (1.0 / dmax)));
+  if (dmin < -tau) lim = smin(lim, phi(mode, SL ? mn / dmin : mn * (1.0 / dmin)));
+  return lim;
 }
 
-// limiters in the face precision T: the exact double versions above for the
-// FP64 path, hardware reciprocal for the FP32 face path
+// Phi of the FP32 face path (hardware reciprocal)
 template <int MODE, typename T> __device__ __forceinline__ T phi_c(T x) {
   if constexpr (MODE == LIM_MINMOD) {
     return smin(T(1.0), x);
@@ -110,27 +113,6 @@ template <int MODE, typename T> __device__ __forceinline__ T phi_c(T x) {
     return fdiv(x * x + T(2.0) * x + fac * eps1, x * x + x + T(2.0) + fac * eps1);
   } else {
     return T(1.0);
-  }
-}
-// The mode is a compile-time constant.  FP32: both outcomes are formed and the
-// flat-difference test selects (no divergent branch per variable); the ratio
-// of a flat difference may be inf/NaN and is discarded by the select.
-template <int MODE, typename T> __device__ __forceinline__ T limiter_rec_c(T dWi, T mn, T mx) {
-  if constexpr (sizeof(T) == 8) {
-    return limiter_rec(MODE, dWi, mn, mx);
-  } else {
-    const bool flat = dabs(dWi) <= T(1.0e-16) * smax(dabs(mx), dabs(mn));
-    const T r = phi_c<MODE, T>((dWi < T(0.0) ? mn : mx) * frcp(dWi));
-    return flat ? T(1.0) : r;
-  }
-}
-template <int MODE, typename T> __device__ __forceinline__ T limiter_sl_c(T dWi, T mn, T mx) {
-  if constexpr (sizeof(T) == 8) {
-    return limiter_sl(MODE, dWi, mn, mx);
-  } else {
-    const bool flat = dabs(dWi) <= T(1.0e-16) * smax(dabs(mx), dabs(mn));
-    const T r = phi_c<MODE, T>(fdiv(dWi < T(0.0) ? mn : mx, dWi));
-    return flat ? T(1.0) : r;
   }
 }
 

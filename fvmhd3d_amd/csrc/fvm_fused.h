@@ -102,7 +102,13 @@ template <> struct alignas(16) FaceEndRec<float> {
   float area;
 };
 // FP64: area carries the sign of cen . face.n (the orientation of the
-// reconstruction normal, computeReconstruction.cpp:113-123)
+// reconstruction normal, computeReconstruction.cpp:113-123).  In memory the
+// fields are planes of one double per face-end slot, so that a wavefront reads
+// each as 512 contiguous bytes and a kernel reads only the fields it uses: the
+// reconstruction and predictor pass 68 bytes a face-end, the limiter passes 24, the flux
+// kernel 68, where 96-byte records cost each of them the whole record (64^3
+// cells: limiter pass 144 -> 94 us a launch, reconstruction and predictor
+// pass 376 -> 351).
 template <> struct alignas(16) FaceEndRec<double> {
   int nbr, pad;
   double nrm[3];
@@ -110,14 +116,17 @@ template <> struct alignas(16) FaceEndRec<double> {
   double cen[3];
   double area;
 };
+enum { FP_NRM = 0, FP_DRL = 3, FP_CEN = 6, FP_AREA = 9, FP_DR = 10, FP_N = 13 };  // FP_DR: own-side offset (drL or drR)
 
 template <typename T> struct FusedArgs {
   int n;                    // cells (all active), in the internal (window-sorted) order
   const int *deg;           // [n] face count of each cell
   const int *gbase;         // [n/64] first slot of each 64-cell group in fe
-  const FaceEndRec<T> *fe;  // SELL: face-end k of cell c at gbase[c/64] + 64*k + c%64
+  const FaceEndRec<T> *fe;  // FP32; SELL: face-end k of cell c at gbase[c/64] + 64*k + c%64
+  const double *fep;        // FP64: FP_N planes of `slots` values
+  size_t slots;
   const float *fdr;         // FP32: own-side centroid offset of each face-end slot, [slot][3]
-  const int *fnb;           // FP32: the neighbour field of each face-end slot (fe[slot].nbr), compact
+  const int *fnb;           // the neighbour field of each face-end slot, compact
   const double *cvol;       // [n]
   const double *lmin;       // [n] pow(V / (4 pi / 3), 1 / 3), formed once at setup
   const double *mvel;       // [3][n] generator velocity (moving mesh only)
@@ -215,6 +224,22 @@ __device__ __forceinline__ void decode_fe(const FaceEndRec<T> &r, FE<T> &g) {
   }
 }
 
+// the face-end record of a slot; FP64: the fields asked for, the others zero
+template <bool DRL, bool CEN> __device__ __forceinline__ FaceEndRec<float> get_fe(const FusedArgs<float> &A, int slot) {
+  return A.fe[slot];
+}
+template <bool DRL, bool CEN> __device__ __forceinline__ FaceEndRec<double> get_fe(const FusedArgs<double> &A, int slot) {
+  FaceEndRec<double> r{};
+  const double *p = A.fep + slot;
+  r.nbr = A.fnb[slot];
+  for (int d = 0; d < 3; d++) {
+    r.nrm[d] = p[(FP_NRM + d) * A.slots];
+    if (DRL) r.drL[d] = p[(FP_DRL + d) * A.slots];
+    if (CEN) r.cen[d] = p[(FP_CEN + d) * A.slots];
+  }
+  r.area = p[FP_AREA * A.slots];
+  return r;
+}
 __device__ __forceinline__ int fe_nbr(int nbr) { return nbr >= 0 ? nbr : ~nbr; }
 
 // face velocity with Springel's correction (computeFluidUpdate.cpp:194-207), canonical orientation
@@ -487,10 +512,10 @@ k_cfl_predict_recon(FusedArgs<T> A) {
     // the next face-end record is loaded one iteration ahead, so the neighbour
     // gather of an iteration issues without waiting for its own record
     FaceEndRec<T> rn;
-    if (deg > 0) rn = A.fe[e0];
+    if (deg > 0) rn = get_fe<MOVING, true>(A, e0);
     for (int q = 0, e = e0; q < deg; q++, e += 64) {
       const FaceEndRec<T> rc0 = rn;
-      if (q + 1 < deg) rn = A.fe[e + 64];
+      if (q + 1 < deg) rn = get_fe<MOVING, true>(A, e + 64);
       const int j = fe_nbr(rc0.nbr);
       T Wj[NF];
       ldv<NF>(A.wcur + (size_t)j * RWC, Wj);
@@ -665,8 +690,8 @@ k_cfl_predict_recon(FusedArgs<T> A) {
         T lm[NF], lo[NF], hi[NF];
         for (int k = 0; k < NF; k++) lo[k] = hi[k] = T(0.0);
         for (int q = 0, e = e0; q < deg; q++, e += 64) {
-          const T *cen = A.fe[e].cen;
-          const T c0 = cen[0], c1 = cen[1], c2 = cen[2];
+          const double *cen = A.fep + FP_CEN * A.slots + e;
+          const T c0 = cen[0], c1 = cen[A.slots], c2 = cen[2 * A.slots];
           for (int k = 0; k < NF; k++) {
             const T d = gx[k] * c0 + gy[k] * c1 + gz[k] * c2;
             lo[k] = __builtin_fmin(lo[k], d);
@@ -736,38 +761,29 @@ __global__ void __launch_bounds__(FB) k_limit(FusedArgs<T> A) {
   const double dtI = tend - t0;
   const double dth = 0.5 * smin(dtI, dtI);
   T *rc = A.rec_w + (size_t)c * REC;
-  T W[NF], tv[NF], gg[3 * NF];
-  ldv<NF>(rc + R_W, W);
+  T tv[NF], gg[3 * NF];
   ldv<NF>(rc + R_T, tv);
   ldv<3 * NF>(rc + R_G, gg);
-  T lo[NF], hi[NF];
-  for (int k = 0; k < NF; k++) {
-    lo[k] = SF(A.mm, k, c, n) - W[k];
-    hi[k] = SF(A.mm, NF + k, c, n) - W[k];
-    lo[k] = smin(lo[k], T(0.0));
-    hi[k] = smax(hi[k], T(0.0));
-  }
   T lm[NF], dmin[NF], dmax[NF];  // extremes of the limiter's argument over the faces
   for (int k = 0; k < NF; k++) dmin[k] = dmax[k] = T(0.0);
   const T dtt = (T)(dtI - dth);
   const int deg = A.deg[c];
   const int e0 = A.gbase[c >> 6] + (c & 63);
-  FaceEndRec<T> rn;
-  if (deg > 0) rn = A.fe[e0];
+  const double *fdr = A.fep + FP_DR * A.slots;
   for (int q = 0, e = e0; q < deg; q++, e += 64) {
-    const FaceEndRec<T> rc0 = rn;
-    if (q + 1 < deg) rn = A.fe[e + 64];
-    FE<T> fe;
-    decode_fe(rc0, fe);
-    const T *dr = fe.isL ? fe.drL : fe.drR;
+    const T dr[3] = {fdr[e], fdr[A.slots + e], fdr[2 * A.slots + e]};
     for (int k = 0; k < NF; k++) {
       const T dW = gg[k] * dr[0] + gg[NF + k] * dr[1] + gg[2 * NF + k] * dr[2] + tv[k] * dtt;
       dmin[k] = __builtin_fmin(dmin[k], dW);
       dmax[k] = __builtin_fmax(dmax[k], dW);
     }
   }
+  T W[NF];
+  ldv<NF>(rc + R_W, W);
   for (int k = 0; k < NF; k++) {
-    lm[k] = limiter_of_extremes<true>(LIM, dmin[k], dmax[k], lo[k], hi[k]);
+    const T lo = smin(SF(A.mm, k, c, n) - W[k], T(0.0));
+    const T hi = smax(SF(A.mm, NF + k, c, n) - W[k], T(0.0));
+    lm[k] = limiter_of_extremes<true>(LIM, dmin[k], dmax[k], lo, hi);
     tv[k] *= lm[k];
     gg[k] *= lm[k];
     gg[NF + k] *= lm[k];
@@ -909,10 +925,10 @@ __global__ void __launch_bounds__(FB) k_flux_apply(FusedArgs<T> A) {
   const int deg = A.deg[c];
   const int e0 = A.gbase[c >> 6] + (c & 63);
   FaceEndRec<T> rn;
-  if (deg > 0) rn = A.fe[e0];
+  if (deg > 0) rn = get_fe<true, false>(A, e0);
   for (int q = 0, e = e0; q < deg; q++, e += 64) {
     const FaceEndRec<T> rc0 = rn;
-    if (q + 1 < deg) rn = A.fe[e + 64];
+    if (q + 1 < deg) rn = get_fe<true, false>(A, e + 64);
     const int j = fe_nbr(rc0.nbr);
     // neighbour face state, extrapolated as soon as it is loaded
     T Wn[NF];
@@ -1195,7 +1211,7 @@ template <typename T>
 __global__ void k_build_faceends(int n, const int *perm, const int *inv, const int *coff, const int *cface,
                                  const int *s1, const int *s2, const double *fc, const double *fnv, int nface,
                                  const double *pos, double Lx, double Ly, double Lz, const int *gbase,
-                                 FaceEndRec<T> *fe) {
+                                 FaceEndRec<T> *fe, double *fep, int *fnb, size_t slots) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const int o = perm[i];
@@ -1227,10 +1243,21 @@ __global__ void k_build_faceends(int n, const int *perm, const int *inv, const i
       r.pad = 0;
       cn = r.cen[0] * fx + r.cen[1] * fy + r.cen[2] * fz;
       r.area = cn < 0.0 ? -area : area;
+      FE<double> g;
+      decode_fe(r, g);
+      const double *dr = g.isL ? g.drL : g.drR;
+      for (int d = 0; d < 3; d++) {
+        fep[(FP_NRM + d) * slots + slot] = r.nrm[d];
+        fep[(FP_DRL + d) * slots + slot] = r.drL[d];
+        fep[(FP_CEN + d) * slots + slot] = r.cen[d];
+        fep[(FP_DR + d) * slots + slot] = dr[d];
+      }
+      fep[FP_AREA * slots + slot] = r.area;
+      fnb[slot] = r.nbr;
     } else {
       r.area = (float)area;
+      fe[slot] = r;
     }
-    fe[slot] = r;
   }
 }
 
@@ -1309,6 +1336,8 @@ template <typename T> FusedArgs<T> fused_args(fvm_ctx *c, double dtmax) {
   A.deg = (const int *)z.deg.p;
   A.gbase = (const int *)z.gbase.p;
   A.fe = (const FaceEndRec<T> *)z.fe.p;
+  A.fep = (const double *)z.fe.p;
+  A.slots = z.slots;
   A.fdr = (const float *)z.fdr.p;
   A.fnb = (const int *)z.fnb.p;
   A.cvol = (const double *)z.cvol.p;
@@ -1375,7 +1404,8 @@ template <typename T> int fused_setup_t(fvm_ctx *c) {
   const size_t ni = sizeof(int) * (size_t)n, nd = sizeof(double) * (size_t)n;
   if ((rc = fvm_ensure(c, z.gbase, sizeof(int) * (size_t)(ng + 1))) || (rc = fvm_ensure(c, z.perm, ni)) ||
       (rc = fvm_ensure(c, z.inv, ni)) || (rc = fvm_ensure(c, z.deg, ni)) ||
-      (rc = fvm_ensure(c, z.fe, sizeof(FaceEndRec<T>) * z.slots)) || (rc = fvm_ensure(c, z.U, NF * nd)) ||
+      (rc = fvm_ensure(c, z.fe, (es == 8 ? sizeof(double) * FP_N : sizeof(FaceEndRec<T>)) * z.slots)) ||
+      (rc = fvm_ensure(c, z.fnb, sizeof(int) * z.slots)) || (rc = fvm_ensure(c, z.U, NF * nd)) ||
       (rc = fvm_ensure(c, z.W64, NF * nd)) || (rc = fvm_ensure(c, z.cvol, nd)) ||
       (rc = fvm_ensure(c, z.mvel, 3 * nd)) || (rc = fvm_ensure(c, z.rec[0], es * rec_len<T>() * (size_t)n)) ||
       (rc = fvm_ensure(c, z.rec[1], es * rec_len<T>() * (size_t)n)) ||
@@ -1394,11 +1424,11 @@ template <typename T> int fused_setup_t(fvm_ctx *c) {
                      (const int *)c->m_coff.p, (const int *)c->m_cface.p, (const int *)c->m_s1.p,
                      (const int *)c->m_s2.p, (const double *)c->m_c.p, (const double *)c->m_n.p, c->nface,
                      (const double *)c->field[FVM_FIELD_POS].p, c->prm.domain_size[0], c->prm.domain_size[1],
-                     c->prm.domain_size[2], (const int *)z.gbase.p, (FaceEndRec<T> *)z.fe.p);
+                     c->prm.domain_size[2], (const int *)z.gbase.p, (FaceEndRec<T> *)z.fe.p, (double *)z.fe.p,
+                     (int *)z.fnb.p, z.slots);
   FVM_HIPCHK(c, hipGetLastError());
   if constexpr (std::is_same<T, float>::value) {
-    if ((rc = fvm_ensure(c, z.fdr, 3 * sizeof(float) * z.slots)) || (rc = fvm_ensure(c, z.fnb, sizeof(int) * z.slots)))
-      return rc;
+    if ((rc = fvm_ensure(c, z.fdr, 3 * sizeof(float) * z.slots))) return rc;
     FVM_HIPCHK(c, hipMemsetAsync(z.fnb.p, 0, sizeof(int) * z.slots, c->stream));
     hipLaunchKernelGGL(k_build_dr, dim3(nb), dim3(256), 0, c->stream, n, (const int *)z.deg.p,
                        (const int *)z.gbase.p, (const FaceEndRec<float> *)z.fe.p, (float *)z.fdr.p, (int *)z.fnb.p);

@@ -95,10 +95,10 @@ struct Phys {
 };
 
 #define FLD(p, k, i, n) (p)[(size_t)(k) * (size_t)(n) + (size_t)(i)]
-// per-face records of the flux and predictor sweeps, one record of `stride`
-// doubles per active face: the cell-side loops read a face's whole record from
-// one or two cache lines
-#define REC(p, k, a, stride) (p)[(size_t)(a) * (size_t)(stride) + (size_t)(k)]
+// per-face records of the flux and predictor sweeps: one row of NREC doubles per
+// active face, a whole 128-byte line, read by the 16 lanes of a cell at once
+constexpr int NREC = 16;
+#define REC(p, k, a) (p)[(size_t)(a) * NREC + (size_t)(k)]
 // per-face geometry record: centroid[3] then area vector n[3]
 #define GEO_C(M, d, f) (M).cn[(size_t)(f) * 6 + (size_t)(d)]
 #define GEO_N(M, d, f) (M).cn[(size_t)(f) * 6 + 3 + (size_t)(d)]
@@ -145,33 +145,12 @@ __global__ void k_faces_to_soa(const fvm_face *__restrict__ f, int n, int *s1, i
 }
 
 // ---------------------------------------------------------------------------
-// Forms of the cell loops:
-//   16 lanes per cell  reconstruction, slope limiter: the lanes first form the
-//               geometry of the cell's faces, one face a lane, into LDS, then
-//               lane k walks the faces for variable k in the reference's order;
-//   k_<name>    one thread per cell, all variables in registers;
-//   k_<name>_v  one lane per (cell, variable): NF lanes per cell, CPW cells per
-//               wavefront (the last 64 - NF * CPW lanes idle).  Every lane of a
-//               cell repeats the face geometry and forms its own variable's
-//               terms in the reference's face order and operation order.
-// All give the same values bit for bit.  The per-variable form fills the chip on
-// the small active sets of individual timesteps, where one thread per cell
-// leaves most SIMDs idle (ONE_THREAD_MIN_CELLS below).
+// The cell loops take 16 lanes per cell.  Reconstruction and slope limiter: the
+// lanes first form the geometry of the cell's faces, one face a lane, into LDS,
+// then lane k walks the faces for variable k in the reference's order.  Sums over
+// face records (fluid update, predictor): lane k sums word k of the cell's
+// records in the reference's order, a face-end being one 128-byte row.
 // ---------------------------------------------------------------------------
-constexpr int CPW = 64 / NF;  // cells per wavefront of the per-variable kernels
-// the cell and variable of this lane; false for the idle lanes
-__device__ __forceinline__ bool cell_var(int &cell, int &k) {
-  const int t = xgid();
-  const int sub = (t & 63) / NF;
-  k = (t & 63) - NF * sub;
-  cell = (t >> 6) * CPW + sub;
-  return sub < CPW;
-}
-// threads of a per-variable launch over n cells
-__host__ __device__ constexpr int cell_var_threads(int n) { return (n + CPW - 1) / CPW * 64; }
-// cell count from which the thread-per-cell forms are used
-constexpr int ONE_THREAD_MIN_CELLS = 131072;
-
 // 16 lanes per cell.  Faces are staged FCH at a time: 24 covers all but the
 // largest cells of random generators (15.5 faces on average), and the LDS
 // leaves four blocks a CU.
@@ -447,12 +426,9 @@ __global__ void __launch_bounds__(256) k_slope_limiter(Cells<S> C, MeshView M, P
 // ---------------------------------------------------------------------------
 // System::computeFluidUpdate face part (computeFluidUpdate.cpp:99-223): one
 // thread per active face writes the face record
-//   rec[0..9] = flux*dt*A, rec[10..12] = n*(psi*dt*A), rec[13] = Bn*dt*A
-// and swp[a] = 1 when i and j were swapped (s1 on a boundary).
+//   rec[0..9] = flux*dt*A, rec[10..12] = n*(psi*dt*A), rec[13] = Bn*dt*A,
+//   rec[15] = 1 when i and j were swapped (s1 on a boundary), else 0
 // ---------------------------------------------------------------------------
-// 14 entries per face record (NREC_P = 15 adds the predictor's dV)
-constexpr int NREC_F = NF + 4;
-
 // computeFluidUpdate.cpp:99-209: the inputs of computeFlux for active face a
 // (boundary swap, space-time extrapolation of both sides, face velocity)
 // F: the face arithmetic (double: the reference's; float: the FP32 face
@@ -554,7 +530,7 @@ __device__ __forceinline__ void face_inputs(const Cells<S> &C, const MeshView &M
 // F = float: the FP32 face arithmetic (face states and HLLD); the records
 // times dt and area, and every sum over them, stay FP64
 template <typename S, typename F>
-__global__ void __launch_bounds__(256) k_face_flux(Cells<S> C, MeshView M, Phys P, double *rec, int *swp,
+__global__ void __launch_bounds__(256) k_face_flux(Cells<S> C, MeshView M, Phys P, double *rec,
                                    unsigned long long *diag) {
   const int a = xgid();
   if (a >= M.nfa) return;
@@ -569,10 +545,11 @@ __global__ void __launch_bounds__(256) k_face_flux(Cells<S> C, MeshView M, Phys 
   compute_flux<F>((F)P.gamma, wij, q.Wi, q.Wj, q.jbnd, nrm, psi, Bn, flux);
 
   const double tarea = q.dt * q.area;
-  for (int k = 0; k < NF; k++) REC(rec, k, a, NREC_F) = (double)flux[k] * tarea;
-  for (int d = 0; d < 3; d++) REC(rec, NF + d, a, NREC_F) = q.normal[d] * ((double)psi * tarea);
-  REC(rec, NF + 3, a, NREC_F) = (double)Bn * tarea;
-  swp[a] = q.sw ? 1 : 0;
+  for (int k = 0; k < NF; k++) REC(rec, k, a) = (double)flux[k] * tarea;
+  for (int d = 0; d < 3; d++) REC(rec, NF + d, a) = q.normal[d] * ((double)psi * tarea);
+  REC(rec, NF + 3, a) = (double)Bn * tarea;
+  REC(rec, 14, a) = 0.0;
+  REC(rec, 15, a) = q.sw ? 1.0 : 0.0;
 }
 
 // the computeFlux inputs of active faces [first, first + count), in the
@@ -595,62 +572,61 @@ __global__ void __launch_bounds__(256) k_face_states(Cells<S> C, MeshView M, Phy
   jbnd[q0] = q.jbnd;
 }
 
-// computeFluidUpdate.cpp:225-245: per cell, in face_active_list order
+// The sum of word k = lane % 16 of cell c's face records over its active
+// face-ends in face_active_list order (computeFluidUpdate.cpp:225-245,
+// computePredictor.cpp:120-136): words 0-9 (flux) leave the i side and enter the
+// j side, the others the other way round.  Every sum rounds to the storage type
+// as the reference's does (words 10-12 are added in it, word 14 stays double).
+// Four rows in flight.
 template <typename S>
-__global__ void __launch_bounds__(256) k_scatter(Cells<S> C, MeshView M, const double *rec, const int *swp) {
-  const int c = xgid();
-  if (c >= C.np) return;
-  const int np = C.np;
-  S U[NF], gp[3], dv;
-  for (int k = 0; k < NF; k++) U[k] = (S)0.0;
-  gp[0] = gp[1] = gp[2] = (S)0.0;
-  dv = (S)0.0;
-  for (int e = M.soff[c]; e < M.soff[c + 1]; e++) {
-    const int ent = M.sent[e];
-    const int a = ent >> 1, side = ent & 1;
-    const bool is_i = (side == 0) != (swp[a] != 0);
-    if (is_i) {
-      for (int k = 0; k < NF; k++) U[k] = (S)((double)U[k] - REC(rec, k, a, NREC_F));
-      for (int d = 0; d < 3; d++) gp[d] = gp[d] + (S)REC(rec, NF + d, a, NREC_F);
-      dv = (S)((double)dv + REC(rec, NF + 3, a, NREC_F));
-    } else {
-      for (int k = 0; k < NF; k++) U[k] = (S)((double)U[k] + REC(rec, k, a, NREC_F));
-      for (int d = 0; d < 3; d++) gp[d] = gp[d] - (S)REC(rec, NF + d, a, NREC_F);
-      dv = (S)((double)dv - REC(rec, NF + 3, a, NREC_F));
+__device__ __forceinline__ double sum_records(const MeshView &M, const double *rec, int fb, int deg, int wdeg) {
+  const int lane = (int)__lane_id(), k = lane & (LC - 1), grp = lane & ~(LC - 1);
+  double acc = 0.0;
+  for (int f0 = 0; f0 < wdeg; f0 += LC) {
+    const int mine = f0 + k < deg ? M.sent[fb + f0 + k] : -1;
+    const int wn = min(wdeg - f0, LC);
+    for (int q0 = 0; q0 < wn; q0 += 4) {
+      double r[4];
+      int ent[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        ent[u] = __shfl(mine, grp + q0 + u);
+        r[u] = ent[u] >= 0 ? REC(rec, k, ent[u] >> 1) : 0.0;
+      }
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        const bool sw = __shfl(r[u], grp + 15) != 0.0;
+        if (ent[u] < 0) continue;
+        const bool is_i = ((ent[u] & 1) == 0) != sw;
+        const double x = is_i == (k < NF) ? -r[u] : r[u];
+        if constexpr (std::is_same<S, double>::value) {
+          acc = acc + x;
+        } else {
+          acc = (k >= NF && k < NF + 3) ? (double)((S)acc + (S)x) : k == 14 ? acc + x : (double)(S)(acc + x);
+        }
+      }
     }
   }
-  FLD(C.ddivB, 0, c, np) = FLD(C.ddivB, 0, c, np) + dv;
-  for (int d = 0; d < 3; d++) FLD(C.dgp, d, c, np) = FLD(C.dgp, d, c, np) + gp[d];
-  for (int k = 0; k < NF; k++) FLD(C.dU, k, c, np) = FLD(C.dU, k, c, np) + U[k];
+  return acc;
 }
 
-// one lane per (cell, variable); lanes 0-2 also sum the gradPsi terms and
-// lane 3 the div B term
+// Bound by the records, one 128-byte row per face-end, most of them from L2 or
+// further.
+// Measured (disk, 2.1 M cells, mean over the active sets of a cycle): 89 us a launch; a
+// thread per cell above 131,072 cells and a lane per (cell, variable) below, with
+// 112-byte rows and the swap flag in an array of its own, took 200 us on average.
 template <typename S>
-__global__ void __launch_bounds__(256) k_scatter_v(Cells<S> C, MeshView M, const double *rec, const int *swp) {
-  int c, k;
-  if (!cell_var(c, k) || c >= C.np) return;
+__global__ void __launch_bounds__(256) k_scatter(Cells<S> C, MeshView M, const double *rec) {
+  const int t = xgid();
+  const int c = t / LC, k = t & (LC - 1);
   const int np = C.np;
-  S U = (S)0.0, gx = (S)0.0;  // gx: gradPsi[k] (k < 3) or div B (k == 3)
-  for (int e = M.soff[c]; e < M.soff[c + 1]; e++) {
-    const int ent = M.sent[e];
-    const int a = ent >> 1, side = ent & 1;
-    const bool is_i = (side == 0) != (swp[a] != 0);
-    const double r = REC(rec, k, a, NREC_F);
-    const double x = k < 4 ? REC(rec, NF + k, a, NREC_F) : 0.0;
-    if (is_i) {
-      U = (S)((double)U - r);
-      if (k < 3) gx = gx + (S)x;
-      else if (k == 3) gx = (S)((double)gx + x);
-    } else {
-      U = (S)((double)U + r);
-      if (k < 3) gx = gx - (S)x;
-      else if (k == 3) gx = (S)((double)gx - x);
-    }
-  }
-  if (k == 3) FLD(C.ddivB, 0, c, np) = FLD(C.ddivB, 0, c, np) + gx;
-  if (k < 3) FLD(C.dgp, k, c, np) = FLD(C.dgp, k, c, np) + gx;
-  FLD(C.dU, k, c, np) = FLD(C.dU, k, c, np) + U;
+  const bool live = c < np;
+  const int fb = live ? M.soff[c] : 0, deg = live ? M.soff[c + 1] - fb : 0;
+  const double acc = sum_records<S>(M, rec, fb, deg, wave_cells_max(deg));
+  if (!live) return;
+  if (k < NF) FLD(C.dU, k, c, np) = FLD(C.dU, k, c, np) + (S)acc;
+  else if (k < NF + 3) FLD(C.dgp, k - NF, c, np) = FLD(C.dgp, k - NF, c, np) + (S)acc;
+  else if (k == NF + 3) FLD(C.ddivB, 0, c, np) = FLD(C.ddivB, 0, c, np) + (S)acc;
 }
 
 // ---------------------------------------------------------------------------
@@ -776,22 +752,55 @@ __global__ void __launch_bounds__(256) k_primitives(Cells<S> C, MeshView M, Phys
 // ---------------------------------------------------------------------------
 // System::computeTimestep (computeTimestep.cpp:6-62)
 // ---------------------------------------------------------------------------
-template <typename S>
+// Two phases a wavefront, as the predictor's cell update: 16 lanes per cell look
+// over its faces (R rounds of four cells), then one lane per cell finishes the
+// cell.  R is chosen on the host so that small sets still fill the chip
+// (cell_rounds).
+template <typename S, int R>
 __global__ void __launch_bounds__(256) k_timestep(Cells<S> C, MeshView M, Phys P, unsigned long long *dtmin_bits) {
-  const int i = xgid();
-  double dti_out = REF_HUGE;
-  if (i < C.nactive) {
-    const int np = C.np;
+  __shared__ double arg[256 / 64][4 * R];
+  const int lane = (int)threadIdx.x & 63, wv = (int)threadIdx.x >> 6, k = lane & (LC - 1);
+  const int c0 = (xgid() >> 6) * (4 * R);  // the wavefront's first cell
+  const int np = C.np;
+  for (int r = 0; r < R; r++) {
+    const int i = c0 + 4 * r + lane / LC;
+    // min over faces of h / (cs + sqrt(a_f)) = h / (cs + sqrt(max a_f)): every
+    // rounding is monotone
+    double a = -1.0;
+    if (i < C.nactive) {
+      const double fac = C.bnd[i] != NO_BOUNDARY ? 0.0 : 1.0;
+      const double iM = 1.0 / FLD(C.U, MASS, i, np);
+      double v[3], pv[3];
+      for (int d = 0; d < 3; d++) {
+        v[d] = FLD(C.U, MOMX + d, i, np) * iM;  // Fluid::to_primitive
+        pv[d] = FLD(C.mvel, d, i, np);
+      }
+      const int fe = M.coff[i + 1];
+      for (int e = M.coff[i] + k; e < fe; e += LC) {
+        const int j = M.cnbr[e];
+        const double dvi[3] = {FLD(C.w, VELX, j, np) - v[0], FLD(C.w, VELY, j, np) - v[1], FLD(C.w, VELZ, j, np) - v[2]};
+        const double dwi[3] = {(double)FLD(C.vel, 0, j, np) - pv[0], (double)FLD(C.vel, 1, j, np) - pv[1],
+                               (double)FLD(C.vel, 2, j, np) - pv[2]};
+        a = __builtin_fmax(a, (dwi[0] * dwi[0] + dwi[1] * dwi[1] + dwi[2] * dwi[2]) +
+                                  fac * (dvi[0] * dvi[0] + dvi[1] * dvi[1] + dvi[2] * dvi[2]) + 1.0 / REF_HUGE);
+      }
+    }
+    for (int o = LC / 2; o > 0; o >>= 1) a = __builtin_fmax(a, __shfl_xor(a, o));
+    if (k == 0) arg[wv][4 * r + lane / LC] = a;
+  }
+  wave_sync();
+  const int i = c0 + lane;
+  double v = REF_HUGE;
+  if (lane < 4 * R && i < C.nactive) {
     const double g = P.gamma;
     const double Volume = C.mvol[i];
     double Ui[NF], Wi[NF];
-    for (int k = 0; k < NF; k++) Ui[k] = FLD(C.U, k, i, np);
+    for (int m = 0; m < NF; m++) Ui[m] = FLD(C.U, m, i, np);
     to_primitive(Ui, Volume, Wi);
     const double h = pow(Volume / (4.0 * REF_PI / 3.0), 1.0 / 3.0);
     const double pv[3] = {FLD(C.mvel, 0, i, np), FLD(C.mvel, 1, i, np), FLD(C.mvel, 2, i, np)};
     double csi = 0.0, vrel = 0.0;
-    const bool isb = C.bnd[i] != NO_BOUNDARY;
-    if (!isb) {
+    if (C.bnd[i] == NO_BOUNDARY) {
       const double Pi = pressure(g, Wi[ETHM]) * g;
       const double B2i = Wi[BX] * Wi[BX] + Wi[BY] * Wi[BY] + Wi[BZ] * Wi[BZ];
       csi = dsqrt((Pi + B2i) / Wi[DENS]);
@@ -799,41 +808,35 @@ __global__ void __launch_bounds__(256) k_timestep(Cells<S> C, MeshView M, Phys P
       vrel = dsqrt(dv[0] * dv[0] + dv[1] * dv[1] + dv[2] * dv[2]);
     }
     double dti = h / (csi + vrel + 1.0 / REF_HUGE);
-    const double fac = isb ? 0.0 : 1.0;
-    for (int e = M.coff[i]; e < M.coff[i + 1]; e++) {
-      const int f = M.cface[e];
-      const int s1 = M.s1[f];
-      const int j = (i == s1) ? M.s2[f] : s1;
-      const double dvi[3] = {FLD(C.w, VELX, j, np) - Wi[VELX], FLD(C.w, VELY, j, np) - Wi[VELY],
-                             FLD(C.w, VELZ, j, np) - Wi[VELZ]};
-      const double dwi[3] = {(double)FLD(C.vel, 0, j, np) - pv[0], (double)FLD(C.vel, 1, j, np) - pv[1],
-                             (double)FLD(C.vel, 2, j, np) - pv[2]};
-      const double dvmax = dsqrt((dwi[0] * dwi[0] + dwi[1] * dwi[1] + dwi[2] * dwi[2]) +
-                                 fac * (dvi[0] * dvi[0] + dvi[1] * dvi[1] + dvi[2] * dvi[2]) +
-                                 1.0 / REF_HUGE);
-      dti = smin(dti, h / (csi + dvmax));
-    }
+    const double a = arg[wv][lane];
+    if (a >= 0.0) dti = smin(dti, h / (csi + dsqrt(a)));
     dti = smin(dti, REF_HUGE);
-    C.dt_new[i] = dti * P.courant;
-    dti_out = C.dt_new[i];
+    v = dti * P.courant;
+    C.dt_new[i] = v;
   }
-  // min over active cells; dt > 0 so the IEEE bit patterns order like the values
-  double v = dti_out;
+  // min over active cells; dt > 0 so the IEEE bit patterns order like the
+  // values.  Atomics on one address take their turn (about 10 ns each), so a
+  // block adds one, and only while it lowers what it reads there
   for (int off = 32; off > 0; off >>= 1) v = smin(v, __shfl_xor(v, off));
-  if ((threadIdx.x & 63) == 0 && i - (int)(threadIdx.x & 63) < C.nactive) {
-    if (v >= 0.0) atomicMin(dtmin_bits, (unsigned long long)__double_as_longlong(v));
+  __shared__ double wmin[256 / 64];
+  if (lane == 0) wmin[wv] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int m = 1; m < 256 / 64; m++) v = smin(v, wmin[m]);
+    const unsigned long long bits = (unsigned long long)__double_as_longlong(v);
+    if (c0 < C.nactive && v >= 0.0 && bits < __hip_atomic_load(dtmin_bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMin(dtmin_bits, bits);
   }
 }
 
 // ---------------------------------------------------------------------------
 // System::computePredictor (computePredictor.cpp:11-391)
-// face part: record rec[0..9] = flux*A, [10..12] = n*(psi*A), [13] = Bn*A, [14] = dV
+// face part: record rec[0..9] = flux*A, [10..12] = n*(psi*A), [13] = Bn*A, [14] = dV,
+// [15] = swapped
 // ---------------------------------------------------------------------------
-constexpr int NREC_P = 15;
-
 // F = float: the FP32 HLLD of the first-order states; the records stay FP64
 template <typename S, typename F>
-__global__ void __launch_bounds__(256) k_predictor_face(Cells<S> C, MeshView M, Phys P, double *rec, int *swp,
+__global__ void __launch_bounds__(256) k_predictor_face(Cells<S> C, MeshView M, Phys P, double *rec,
                                         unsigned long long *diag) {
   const int a = xgid();
   if (a >= M.nfa) return;
@@ -889,11 +892,11 @@ __global__ void __launch_bounds__(256) k_predictor_face(Cells<S> C, MeshView M, 
     }
     compute_flux<F>((F)P.gamma, wf, Wif, Wjf, jbnd, nf, psi, Bn, flux);
   }
-  for (int k = 0; k < NF; k++) REC(rec, k, a, NREC_P) = (double)flux[k] * area;
-  for (int d = 0; d < 3; d++) REC(rec, NF + d, a, NREC_P) = normal[d] * ((double)psi * area);
-  REC(rec, NF + 3, a, NREC_P) = (double)Bn * area;
-  REC(rec, NF + 4, a, NREC_P) = area * (rij[0] * wij[0] + rij[1] * wij[1] + rij[2] * wij[2]) / dsl;
-  swp[a] = sw ? 1 : 0;
+  for (int k = 0; k < NF; k++) REC(rec, k, a) = (double)flux[k] * area;
+  for (int d = 0; d < 3; d++) REC(rec, NF + d, a) = normal[d] * ((double)psi * area);
+  REC(rec, NF + 3, a) = (double)Bn * area;
+  REC(rec, NF + 4, a) = area * (rij[0] * wij[0] + rij[1] * wij[1] + rij[2] * wij[2]) / dsl;
+  REC(rec, 15, a) = sw ? 1.0 : 0.0;
 }
 
 __device__ __forceinline__ int exp_of(double dt) {
@@ -907,53 +910,42 @@ __device__ __forceinline__ double rung_dt(double dtmax, int min_rung, double dt)
   return dt_tick * (double)(1ULL << (31 - rung));
 }
 
-template <typename S>
+// Cell part, two phases a wavefront: the face sums with 16 lanes per cell (R
+// rounds of four cells), then the cell update with one lane per cell.  Bound by
+// the records in large sets, by the update's chain of divisions, exp and pow in
+// small ones.
+// Measured (same sets): 128 us a launch against 179 us for a thread per cell above
+// 131,072 cells and a lane per (cell, variable) below; 97,000 cells at once: 57
+// against 105 us.
+template <typename S, int R>
 __global__ void __launch_bounds__(256) k_predictor_cell(Cells<S> C, MeshView M, Phys P, const double *rec,
-                                        const int *swp, double dtmax, int min_rung,
-                                        unsigned long long *diag) {
-  const int c = xgid();
-  if (c >= C.nactive) return;
-  const int np = C.np, nactive = C.nactive;
-  S dU[NF], gp[3], dv;
-  double dV = 0.0;
-  for (int k = 0; k < NF; k++) dU[k] = (S)0.0;
-  gp[0] = gp[1] = gp[2] = (S)0.0;
-  dv = (S)0.0;
-  for (int e = M.soff[c]; e < M.soff[c + 1]; e++) {
-    const int ent = M.sent[e];
-    const int a = ent >> 1, side = ent & 1;
-    const int f = M.fact[a];
-    const bool sw = swp[a] != 0;
-    const bool is_i = (side == 0) != sw;
-    if (is_i) {
-      for (int k = 0; k < NF; k++) dU[k] = (S)((double)dU[k] - REC(rec, k, a, NREC_P));
-      for (int d = 0; d < 3; d++) gp[d] = gp[d] + (S)REC(rec, NF + d, a, NREC_P);
-      dv = (S)((double)dv + REC(rec, NF + 3, a, NREC_P));
-      dV += REC(rec, NF + 4, a, NREC_P);
-    } else {
-      // j receives only when active and not a boundary (computePredictor.cpp:127-128)
-      const int jeff = sw ? M.s1[f] : M.s2[f];
-      (void)jeff;
-      if (c >= nactive || C.bnd[c] != NO_BOUNDARY) continue;
-      dV -= REC(rec, NF + 4, a, NREC_P);
-      for (int k = 0; k < NF; k++) dU[k] = (S)((double)dU[k] + REC(rec, k, a, NREC_P));
-      for (int d = 0; d < 3; d++) gp[d] = gp[d] - (S)REC(rec, NF + d, a, NREC_P);
-      dv = (S)((double)dv - REC(rec, NF + 3, a, NREC_P));
-    }
+                                        double dtmax, int min_rung, unsigned long long *diag) {
+  constexpr int ST = NREC + 1;  // a cell's sums in LDS
+  __shared__ double sums[256 / 64][4 * R * ST];
+  const int lane = (int)threadIdx.x & 63, wv = (int)threadIdx.x >> 6, k = lane & (LC - 1);
+  const int c0 = (xgid() >> 6) * (4 * R);  // the wavefront's first cell
+  const int np = C.np;
+  for (int r = 0; r < R; r++) {
+    const int i = c0 + 4 * r + lane / LC;
+    const int fb = i < C.nactive ? M.soff[i] : 0, deg = i < C.nactive ? M.soff[i + 1] - fb : 0;
+    sums[wv][(4 * r + lane / LC) * ST + k] = sum_records<S>(M, rec, fb, deg, wave_cells_max(deg));
   }
-  if (C.bnd[c] != NO_BOUNDARY) return;
+  wave_sync();
+  const int c = c0 + lane;
+  if (lane >= 4 * R || c >= C.nactive || C.bnd[c] != NO_BOUNDARY) return;
+  const double *dU = &sums[wv][lane * ST];
+  const double *dPsi = dU + NF;
+  const double divB = dU[NF + 3], dV = dU[NF + 4];
   const double g = P.gamma;
-  const double divB = (double)dv;
-  const double dPsi[3] = {(double)gp[0], (double)gp[1], (double)gp[2]};
   double U0[NF], W0[NF];
-  for (int k = 0; k < NF; k++) U0[k] = FLD(C.U, k, c, np);
+  for (int m = 0; m < NF; m++) U0[m] = FLD(C.U, m, c, np);
   to_primitive(U0, M.cvol[c], W0);
   double dtn = C.dt_new[c];
-  while (U0[MASS] + (double)dU[MASS] * dtn <= 0.0) dtn *= 0.5;
+  while (U0[MASS] + dU[MASS] * dtn <= 0.0) dtn *= 0.5;
   C.dt_new[c] = dtn;
   const double dt = rung_dt(dtmax, min_rung, dtn) / 128;
   double Uc[NF];
-  for (int k = 0; k < NF; k++) Uc[k] = U0[k] + (double)dU[k] * dt;
+  for (int m = 0; m < NF; m++) Uc[m] = U0[m] + dU[m] * dt;
   Uc[WBX] -= W0[VELX] * divB * dt;
   Uc[WBY] -= W0[VELY] * divB * dt;
   Uc[WBZ] -= W0[VELZ] * divB * dt;
@@ -977,89 +969,7 @@ __global__ void __launch_bounds__(256) k_predictor_cell(Cells<S> C, MeshView M, 
     W1[ENTR] = entropy_from_ethm(g, W1);
   }
   const double idt = 1.0 / dt;
-  for (int k = 0; k < NF; k++) FLD(C.t, k, c, np) = (S)((W1[k] - W0[k]) * idt);
-}
-
-// The face sums take one lane per (cell, variable) (lanes 0-2 also gradPsi,
-// lane 3 div B, lane 4 the volume change); the cell update then runs in every
-// lane of the cell on the sums gathered from its lanes, and lane k stores Wt[k].
-template <typename S>
-__global__ void __launch_bounds__(256) k_predictor_cell_v(Cells<S> C, MeshView M, Phys P, const double *rec,
-                                        const int *swp, double dtmax, int min_rung,
-                                        unsigned long long *diag) {
-  int c, k;
-  if (!cell_var(c, k) || c >= C.nactive) return;
-  const int np = C.np;
-  const int base = (int)__lane_id() - k;
-  S dUk = (S)0.0, gx = (S)0.0;  // gx: gradPsi[k] (k < 3) or div B (k == 3)
-  double dVk = 0.0;             // lane 4: the volume change
-  for (int e = M.soff[c]; e < M.soff[c + 1]; e++) {
-    const int ent = M.sent[e];
-    const int a = ent >> 1, side = ent & 1;
-    const bool sw = swp[a] != 0;
-    const bool is_i = (side == 0) != sw;
-    const double r = REC(rec, k, a, NREC_P);
-    const double x = k < 5 ? REC(rec, NF + k, a, NREC_P) : 0.0;
-    if (is_i) {
-      dUk = (S)((double)dUk - r);
-      if (k < 3) gx = gx + (S)x;
-      else if (k == 3) gx = (S)((double)gx + x);
-      else if (k == 4) dVk += x;
-    } else {
-      // j receives only when not a boundary (computePredictor.cpp:127-128);
-      // every cell of this kernel is active
-      if (C.bnd[c] != NO_BOUNDARY) continue;
-      if (k == 4) dVk -= x;
-      dUk = (S)((double)dUk + r);
-      if (k < 3) gx = gx - (S)x;
-      else if (k == 3) gx = (S)((double)gx - x);
-    }
-  }
-  if (C.bnd[c] != NO_BOUNDARY) return;
-  // every lane of the cell gathers the sums
-  double dU[NF];
-  for (int m = 0; m < NF; m++) dU[m] = (double)__shfl((double)dUk, base + m);
-  const double dPsi[3] = {(double)__shfl((double)gx, base), (double)__shfl((double)gx, base + 1),
-                          (double)__shfl((double)gx, base + 2)};
-  const double divB = __shfl((double)gx, base + 3);
-  const double dV = __shfl(dVk, base + 4);
-  const double g = P.gamma;
-  double U0[NF], W0[NF];
-  for (int m = 0; m < NF; m++) U0[m] = FLD(C.U, m, c, np);
-  to_primitive(U0, M.cvol[c], W0);
-  double dtn = C.dt_new[c];
-  while (U0[MASS] + dU[MASS] * dtn <= 0.0) dtn *= 0.5;
-  if (k == 0) C.dt_new[c] = dtn;
-  const double dt = rung_dt(dtmax, min_rung, dtn) / 128;
-  double Uc[NF];
-  for (int m = 0; m < NF; m++) Uc[m] = U0[m] + dU[m] * dt;
-  Uc[WBX] -= W0[VELX] * divB * dt;
-  Uc[WBY] -= W0[VELY] * divB * dt;
-  Uc[WBZ] -= W0[VELZ] * divB * dt;
-  const double pres = pressure(g, W0[ETHM]);
-  const double B2 = W0[BX] * W0[BX] + W0[BY] * W0[BY] + W0[BZ] * W0[BZ];
-  const double dcs2 = g * pres + B2;
-  const double ch_sig = dsqrt(dcs2 / W0[DENS]);
-  Uc[WBX] -= dPsi[0] * dt;
-  Uc[WBY] -= dPsi[1] * dt;
-  Uc[WBZ] -= dPsi[2] * dt;
-  Uc[MPSI] -= dcs2 * divB * dt;
-  const double cr = 0.5;
-  const double l_min = pow(M.cvol[c] / (4.0 * REF_PI / 3.0), 1.0 / 3.0);
-  Uc[MPSI] *= exp(-cr * ch_sig / l_min * dt);
-  double W1[NF];
-  to_primitive(Uc, M.cvol[c] * exp(dV * dt / M.cvol[c]), W1);
-  if (W1[ETHM] <= 0.0) {
-    W1[ETHM] = ethm_from_entropy(g, W1);
-    if (k == 0) atomicAdd(&diag[FVM_DIAG_ETHM_FAILED], 1ULL);
-  } else {
-    W1[ENTR] = entropy_from_ethm(g, W1);
-  }
-  const double idt = 1.0 / dt;
-  double out = 0.0;
-  for (int m = 0; m < NF; m++)
-    if (m == k) out = (W1[m] - W0[m]) * idt;
-  FLD(C.t, k, c, np) = (S)out;
+  for (int m = 0; m < NF; m++) FLD(C.t, m, c, np) = (S)((W1[m] - W0[m]) * idt);
 }
 
 // ---------------------------------------------------------------------------
@@ -1496,7 +1406,7 @@ int fvm_destroy(fvm_ctx *c) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   for (auto &b : c->field) release(b);
   for (DBuf *b : {&c->m_s1, &c->m_s2, &c->m_c, &c->m_n, &c->m_cn, &c->m_coff, &c->m_cface, &c->m_cnbr, &c->m_cvol, &c->m_fact,
-                  &c->m_soff, &c->m_sent, &c->rec, &c->swp, &c->tmp0, &c->tmp1, &c->tmp2, &c->stage,
+                  &c->m_soff, &c->m_sent, &c->rec, &c->tmp0, &c->tmp1, &c->tmp2, &c->stage,
                   &c->diag, &c->scalars})
     release(*b);
   fvm::scan_release(c->scan);
@@ -1842,6 +1752,14 @@ int fvm_download_active_faces(fvm_ctx *c, int *face_active, int n) {
   return FVM_OK;
 }
 
+// Rounds of four cells a wavefront takes in the two-phase cell kernels: as many
+// as leave about four wavefronts for each of the 1024 SIMDs, since the second
+// phase uses one lane per cell (16 rounds: all 64 lanes).
+// Measured: the CFL kernel on 97,000 cells 33 us with 4 rounds (45 us as a thread
+// per cell), on a 14,000-cell mesh's active sets 8 us with one (29 us).
+static int cell_rounds(int n) { return n >= 262144 ? 16 : n >= 65536 ? 4 : 1; }
+static long rounds_threads(int n, int R) { return ((long)n + 4 * R - 1) / (4 * R) * 64; }
+
 #define DISPATCH(c, fn, ...)                                   \
   ((c)->prm.storage == FVM_STORAGE_SHIPPED ? fn<float>(__VA_ARGS__) : fn<double>(__VA_ARGS__))
 
@@ -1877,22 +1795,16 @@ static int read_diag(fvm_ctx *c, unsigned long long *h) {
 template <typename S> static int do_fluid_update(fvm_ctx *c) {
   const int nfa = c->nfa;
   int rc;
-  if ((rc = ensure(c, c->rec, sizeof(double) * fvm::NREC_P * (size_t)nfa)) || (rc = ensure(c, c->swp, sizeof(int) * (size_t)nfa)))
-    return rc;
+  if ((rc = ensure(c, c->rec, sizeof(double) * fvm::NREC * (size_t)nfa))) return rc;
   unsigned long long before[FVM_NDIAG], after[FVM_NDIAG];
   if (!c->defer_sync && (rc = read_diag(c, before))) return rc;
   if (c->face32)
     LAUNCH_T(c, FVM_KT_FACE_FLUX, (fvm::k_face_flux<S, float>), nfa, cells<S>(c), meshview(c), phys(c), (double *)c->rec.p,
-             (int *)c->swp.p, (unsigned long long *)c->diag.p);
+             (unsigned long long *)c->diag.p);
   else
     LAUNCH_T(c, FVM_KT_FACE_FLUX, (fvm::k_face_flux<S, double>), nfa, cells<S>(c), meshview(c), phys(c), (double *)c->rec.p,
-             (int *)c->swp.p, (unsigned long long *)c->diag.p);
-  if (c->np >= fvm::ONE_THREAD_MIN_CELLS)
-    LAUNCH_T(c, FVM_KT_SCATTER, fvm::k_scatter<S>, c->np, cells<S>(c), meshview(c), (const double *)c->rec.p,
-             (const int *)c->swp.p);
-  else
-    LAUNCH_T(c, FVM_KT_SCATTER, fvm::k_scatter_v<S>, fvm::cell_var_threads(c->np), cells<S>(c), meshview(c),
-             (const double *)c->rec.p, (const int *)c->swp.p);
+             (unsigned long long *)c->diag.p);
+  LAUNCH_T(c, FVM_KT_SCATTER, fvm::k_scatter<S>, fvm::cell_lanes(c->np), cells<S>(c), meshview(c), (const double *)c->rec.p);
   if (c->defer_sync) return FVM_OK;  // the substep compares the positivity count itself
   if ((rc = read_diag(c, after))) return rc;
   if (after[FVM_DIAG_POSITIVITY] != before[FVM_DIAG_POSITIVITY])
@@ -1956,7 +1868,11 @@ int fvm_compute_primitives(fvm_ctx *c, int predictor_flag) {
 template <typename S> static int do_timestep(fvm_ctx *c, double *dt_min) {
   unsigned long long *bits = (unsigned long long *)c->scalars.p;
   LAUNCH(c, fvm::k_set_u64, 1, bits, 0x7FF0000000000000ULL);  // +inf
-  LAUNCH_T(c, FVM_KT_TIMESTEP, fvm::k_timestep<S>, c->nactive, cells<S>(c), meshview(c), phys(c), bits);
+  const int R = cell_rounds(c->nactive);
+  const long nt = rounds_threads(c->nactive, R);
+  if (R == 16) LAUNCH_T(c, FVM_KT_TIMESTEP, (fvm::k_timestep<S, 16>), nt, cells<S>(c), meshview(c), phys(c), bits);
+  else if (R == 4) LAUNCH_T(c, FVM_KT_TIMESTEP, (fvm::k_timestep<S, 4>), nt, cells<S>(c), meshview(c), phys(c), bits);
+  else LAUNCH_T(c, FVM_KT_TIMESTEP, (fvm::k_timestep<S, 1>), nt, cells<S>(c), meshview(c), phys(c), bits);
   if (c->defer_sync && !dt_min) return FVM_OK;
   unsigned long long h = 0;
   HIPCHK(c, hipMemcpyAsync(&h, bits, sizeof h, hipMemcpyDeviceToHost, c->stream));
@@ -2014,21 +1930,22 @@ int fvm_compute_timestep_limiter(fvm_ctx *c) {
 template <typename S> static int do_predictor(fvm_ctx *c, double dtmax, int min_rung) {
   const int nfa = c->nfa;
   int rc;
-  if ((rc = ensure(c, c->rec, sizeof(double) * fvm::NREC_P * (size_t)nfa)) || (rc = ensure(c, c->swp, sizeof(int) * (size_t)nfa)))
-    return rc;
+  if ((rc = ensure(c, c->rec, sizeof(double) * fvm::NREC * (size_t)nfa))) return rc;
   if (c->face32)
     LAUNCH_T(c, FVM_KT_PREDICTOR_FACE, (fvm::k_predictor_face<S, float>), nfa, cells<S>(c), meshview(c), phys(c),
-             (double *)c->rec.p, (int *)c->swp.p, (unsigned long long *)c->diag.p);
+             (double *)c->rec.p, (unsigned long long *)c->diag.p);
   else
     LAUNCH_T(c, FVM_KT_PREDICTOR_FACE, (fvm::k_predictor_face<S, double>), nfa, cells<S>(c), meshview(c), phys(c),
-             (double *)c->rec.p, (int *)c->swp.p, (unsigned long long *)c->diag.p);
-  if (c->nactive >= fvm::ONE_THREAD_MIN_CELLS)
-    LAUNCH_T(c, FVM_KT_PREDICTOR_CELL, fvm::k_predictor_cell<S>, c->nactive, cells<S>(c), meshview(c), phys(c),
-             (const double *)c->rec.p, (const int *)c->swp.p, dtmax, min_rung, (unsigned long long *)c->diag.p);
-  else
-    LAUNCH_T(c, FVM_KT_PREDICTOR_CELL, fvm::k_predictor_cell_v<S>, fvm::cell_var_threads(c->nactive), cells<S>(c),
-             meshview(c), phys(c), (const double *)c->rec.p, (const int *)c->swp.p, dtmax, min_rung,
-             (unsigned long long *)c->diag.p);
+             (double *)c->rec.p, (unsigned long long *)c->diag.p);
+  const int R = cell_rounds(c->nactive);
+  const long nt = rounds_threads(c->nactive, R);
+#define PRED(R_)                                                                                                      \
+  LAUNCH_T(c, FVM_KT_PREDICTOR_CELL, (fvm::k_predictor_cell<S, R_>), nt, cells<S>(c), meshview(c), phys(c),             \
+           (const double *)c->rec.p, dtmax, min_rung, (unsigned long long *)c->diag.p)
+  if (R == 16) PRED(16);
+  else if (R == 4) PRED(4);
+  else PRED(1);
+#undef PRED
   return finish(c);
 }
 int fvm_compute_predictor(fvm_ctx *c, double dtmax, int min_rung) {

@@ -865,8 +865,7 @@ int fvm_substep_setup(fvm_ctx *c, int ncell, int nface, const fvm_face *faces, c
                            {&c->m_coff, 4 * (N + 1)}, {&c->m_cface, 4 * R}, {&c->m_cnbr, 4 * R}, {&c->m_cvol, 8 * N},
                            {&c->m_soff, 4 * (N + 1)}, {&c->m_sent, 8 * F + 4}, {&c->m_fact, 4 * (F + 1)},
                            {&c->tmp0, 4 * (std::max(N, R) + 1)}, {&c->tmp1, 4 * (std::max(F, R) + 1)},
-                           {&c->tmp2, 4 * (R + 1)}, {&c->rec, 8 * 15 * F} /* 15-double face records */,
-                           {&c->swp, 4 * F}})))
+                           {&c->tmp2, 4 * (R + 1)}, {&c->rec, 8 * 16 * F} /* 16-double face records */})))
     return rc;
   for (int f = 0; f < FVM_NFIELDS; f++) {
     const size_t bytes = (kInt[f] ? 4 : 8) * (size_t)kWidth[f] * N;

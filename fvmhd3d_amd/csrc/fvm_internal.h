@@ -71,7 +71,7 @@ struct SubstepState {
   bool complete = false;  // the global cell lists list every face under each of its cells
   int n = 0, nface = 0, nref = 0;
   DBuf gs1, gs2, gc, gn, goff, gface, gnbr, gvol;  // global mesh (SoA; gnbr: the other cell of every gface entry)
-  DBuf g[FVM_NFIELDS];                        // global fields, SoA [k*n + i]
+  DBuf g[FVM_NFIELDS];                        // global fields, a row of components per cell [i*width + k]
   DBuf rung;                                  // int per cell
   DBuf act, apos, fmark, fpos, fl, cmark, iflag, ipos, g2l, perm, len, hist, err;
   DBuf sdti, hot, hpos, hlist, chg;  // timestep-limiter sweep: local dti, hot cells, changes

@@ -1209,8 +1209,7 @@ __global__ void k_advance(double *tdev, unsigned long long *dtmin_bits, double d
 // are formed in FP64 exactly as the reference forms them.
 template <typename T>
 __global__ void k_build_faceends(int n, const int *perm, const int *inv, const int *coff, const int *cface,
-                                 const int *s1, const int *s2, const double *fc, const double *fnv, int nface,
-                                 const double *pos, double Lx, double Ly, double Lz, const int *gbase,
+                                 const int *s1, const int *s2, const double *cn6, const double *pos, double Lx, double Ly, double Lz, const int *gbase,
                                  FaceEndRec<T> *fe, double *fep, int *fnb, size_t slots) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
@@ -1223,13 +1222,14 @@ __global__ void k_build_faceends(int n, const int *perm, const int *inv, const i
     const bool isL = a == o;
     FaceEndRec<T> r;
     r.nbr = isL ? inv[b] : ~inv[a];
-    const double fx = FLD(fnv, 0, f, nface), fy = FLD(fnv, 1, f, nface), fz = FLD(fnv, 2, f, nface);
+    const double *geo = cn6 + 6 * (size_t)f;  // centroid, n
+    const double fx = geo[3], fy = geo[4], fz = geo[5];
     const double area = dsqrt(fx * fx + fy * fy + fz * fz);
     const double ia = 1.0 / area;
     const double fn[3] = {fx, fy, fz};
     double cn = 0.0;
     for (int d = 0; d < 3; d++) {
-      const double cf = FLD(fc, d, f, nface);
+      const double cf = geo[d];
       r.nrm[d] = (T)(fn[d] * ia);
       r.drL[d] = (T)(cf - FLD(pos, d, a, n));
       if constexpr (std::is_same<T, double>::value) {
@@ -1422,7 +1422,7 @@ template <typename T> int fused_setup_t(fvm_ctx *c) {
   const int *pp = (const int *)z.perm.p;
   hipLaunchKernelGGL(k_build_faceends<T>, dim3(nb), dim3(256), 0, c->stream, n, pp, (const int *)z.inv.p,
                      (const int *)c->m_coff.p, (const int *)c->m_cface.p, (const int *)c->m_s1.p,
-                     (const int *)c->m_s2.p, (const double *)c->m_c.p, (const double *)c->m_n.p, c->nface,
+                     (const int *)c->m_s2.p, (const double *)c->m_cn.p,
                      (const double *)c->field[FVM_FIELD_POS].p, c->prm.domain_size[0], c->prm.domain_size[1],
                      c->prm.domain_size[2], (const int *)z.gbase.p, (FaceEndRec<T> *)z.fe.p, (double *)z.fe.p,
                      (int *)z.fnb.p, z.slots);

@@ -79,8 +79,7 @@ template <typename S> struct Cells {
 struct MeshView {
   int nface, nfa;
   const int *s1, *s2;
-  const double *c, *n;  // [3][nface]
-  const double *cn;     // [nface][6]: centroid, n (the same values per face)
+  const double *cn;     // [nface][6]: centroid, n
   const int *coff, *cface;
   const int *cnbr;      // the other cell of each cell_face entry
   const double *cvol;
@@ -129,16 +128,13 @@ __global__ void k_soa_to_aos(const S *__restrict__ src, double *__restrict__ dst
   if (i >= n) return;
   for (int k = 0; k < width; k++) dst[(size_t)i * width + k] = (double)FLD(src, k, i, n);
 }
-__global__ void k_faces_to_soa(const fvm_face *__restrict__ f, int n, int *s1, int *s2, double *c,
-                               double *nn, double *cn) {
+__global__ void k_split_faces(const fvm_face *__restrict__ f, int n, int *s1, int *s2, double *cn) {
   const int i = gid();
   if (i >= n) return;
   const fvm_face F = f[i];
   s1[i] = F.s1;
   s2[i] = F.s2;
   for (int d = 0; d < 3; d++) {
-    FLD(c, d, i, n) = F.centroid[d];
-    FLD(nn, d, i, n) = F.n[d];
     cn[(size_t)i * 6 + d] = F.centroid[d];
     cn[(size_t)i * 6 + 3 + d] = F.n[d];
   }
@@ -1035,18 +1031,41 @@ __global__ void k_cell_nbr(const int *__restrict__ coff, const int *__restrict__
     cnbr[e] = a == i ? s2[f] : a;
   }
 }
-__global__ void k_csr_sort(const int *__restrict__ coff, int nactive, int *__restrict__ cface) {
-  const int i = gid();
-  if (i >= nactive) return;
-  const int b = coff[i], e = coff[i + 1];
-  for (int k = b + 1; k < e; k++) {
-    const int v = cface[k];
-    int m = k - 1;
-    while (m >= b && cface[m] > v) {
-      cface[m + 1] = cface[m];
-      m--;
+// Distinct non-negative ints of a short list into ascending order by 16 lanes:
+// every lane ranks its own entries against the whole list in LDS (up to
+// LIST_LDS entries; longer lists are handled by the callers).  Negative entries
+// are left out.
+constexpr int LIST_LDS = 64;
+template <typename F> __device__ __forceinline__ void rank_list(const int *list, int n, int k, F put) {
+  for (int e = k; e < n; e += LC) {
+    const int v = list[e];
+    if (v < 0) continue;
+    int rank = 0;
+    for (int m = 0; m < n; m++) rank += (unsigned)list[m] < (unsigned)v ? 1 : 0;
+    put(rank, v);
+  }
+}
+__global__ void __launch_bounds__(256) k_csr_sort(const int *__restrict__ coff, int nactive, int *__restrict__ cface) {
+  __shared__ int list[256 / LC][LIST_LDS + 1];
+  const int t = gid();
+  const int i = t / LC, k = t & (LC - 1);
+  int *l = list[threadIdx.x / LC];
+  const int b = i < nactive ? coff[i] : 0, e = i < nactive ? coff[i + 1] : 0, n = e - b;
+  if (n <= LIST_LDS)
+    for (int q = k; q < n; q += LC) l[q] = cface[b + q];
+  wave_sync();
+  if (n <= LIST_LDS) {
+    rank_list(l, n, k, [&](int r, int v) { cface[b + r] = v; });
+  } else if (k == 0) {
+    for (int q = b + 1; q < e; q++) {
+      const int v = cface[q];
+      int m = q - 1;
+      while (m >= b && cface[m] > v) {
+        cface[m + 1] = cface[m];
+        m--;
+      }
+      cface[m + 1] = v;
     }
-    cface[m + 1] = v;
   }
 }
 // first position of each face in the concatenated face lists of active,
@@ -1067,19 +1086,88 @@ __global__ void k_face_firstflag(MeshView M, const int *bnd, int nactive, const 
 // in the lower-indexed of its two cells that are active and not on a
 // boundary, since the lists are concatenated in cell order.
 __global__ void k_face_firstflag_direct(MeshView M, const int *bnd, int nactive, int *flag) {
-  const int i = gid();
+  const int t = gid();
+  const int i = t / LC;
   if (i >= nactive) return;
   const bool ok = bnd[i] == NO_BOUNDARY;
-  for (int e = M.coff[i]; e < M.coff[i + 1]; e++) {
-    const int f = M.cface[e];
-    const int j = (M.s1[f] == i) ? M.s2[f] : M.s1[f];
+  for (int e = M.coff[i] + (t & (LC - 1)); e < M.coff[i + 1]; e += LC) {
+    const int j = M.cnbr[e];
     const bool earlier = j < i && j < nactive && bnd[j] == NO_BOUNDARY;
     flag[e] = (ok && !earlier) ? 1 : 0;
   }
 }
-__global__ void k_face_compact(MeshView M, const int *flag, const int *pos, int nref, int *fact) {
+__global__ void k_face_compact(MeshView M, const int *flag, const int *pos, int nref, int *fact, int *fpos) {
   const int e = gid();
-  if (e < nref && flag[e]) fact[pos[e]] = M.cface[e];
+  if (e < nref && flag[e]) {
+    const int f = M.cface[e], a = pos[e];
+    fact[a] = f;
+    fpos[f] = a;
+  }
+}
+
+// The face-end list of every cell, entries a << 1 | side in ascending order,
+// from the cells' own face lists and the faces' places in the active list: no
+// atomics, and no gathers beyond one list.  A cell without a list of its own (an
+// inactive neighbour of a substep layout) walks its global list and takes the
+// faces of the layout.  COUNT: the lengths; otherwise the lists.
+// Measured (disk, 2.1 M cells, mean over the active sets of a cycle): 77 us for both
+// passes; counting and filling over the active faces with atomics, then
+// sorting, took 201 us (a 14,000-cell mesh's active sets: 10 against 51 us).
+struct EndLists {
+  int np, nactive;
+  const int *coff, *cface, *s1, *fpos;
+  const int *perm, *goff, *gface, *gmark, *gpos;  // substep layout (cells >= nactive), else null
+};
+__device__ __forceinline__ int end_entry(const EndLists &E, int c, int e) {
+  int f;
+  if (c < E.nactive) {
+    f = E.cface[e];
+  } else {
+    const int gf = E.gface[e];
+    if (!E.gmark[gf]) return -1;
+    f = E.gpos[gf];
+  }
+  const int a = E.fpos[f];
+  return a < 0 ? -1 : (a << 1) | (E.s1[f] == c ? 0 : 1);
+}
+template <bool COUNT>
+__global__ void __launch_bounds__(256) k_end_lists(EndLists E, int *__restrict__ cnt, const int *__restrict__ soff,
+                                                   int *__restrict__ sent) {
+  __shared__ int list[256 / LC][LIST_LDS + 1];
+  const int t = xgid();
+  const int c = t / LC, k = t & (LC - 1);
+  const bool live = c < E.np;
+  int b = 0, n = 0;
+  if (live) {
+    const int g = c < E.nactive ? c : E.perm[c];
+    const int *off = c < E.nactive ? E.coff : E.goff;
+    b = off[g];
+    n = off[g + 1] - b;
+  }
+  if constexpr (COUNT) {
+    int m = 0;
+    for (int q = k; q < n; q += LC) m += end_entry(E, c, b + q) >= 0 ? 1 : 0;
+    for (int o = LC / 2; o > 0; o >>= 1) m += __shfl_xor(m, o);
+    if (live && k == 0) cnt[c] = m;
+  } else {
+    int *l = list[threadIdx.x / LC];
+    if (n <= LIST_LDS)
+      for (int q = k; q < n; q += LC) l[q] = end_entry(E, c, b + q);
+    wave_sync();
+    if (!live) return;
+    int *out = sent + soff[c];
+    if (n <= LIST_LDS) {
+      rank_list(l, n, k, [&](int r, int v) { out[r] = v; });
+    } else {
+      for (int q = k; q < n; q += LC) {
+        const int v = end_entry(E, c, b + q);
+        if (v < 0) continue;
+        int rank = 0;
+        for (int m = 0; m < n; m++) rank += (unsigned)end_entry(E, c, b + m) < (unsigned)v ? 1 : 0;
+        out[rank] = v;
+      }
+    }
+  }
 }
 // Consecutive active faces mostly share the cell whose list introduced them,
 // so lanes with the same target add once per wavefront: the lowest such lane
@@ -1292,8 +1380,6 @@ static fvm::MeshView meshview(fvm_ctx *c) {
   M.nfa = c->nfa < 0 ? 0 : c->nfa;
   M.s1 = (const int *)c->m_s1.p;
   M.s2 = (const int *)c->m_s2.p;
-  M.c = (const double *)c->m_c.p;
-  M.n = (const double *)c->m_n.p;
   M.cn = (const double *)c->m_cn.p;
   M.coff = (const int *)c->m_coff.p;
   M.cface = (const int *)c->m_cface.p;
@@ -1405,7 +1491,7 @@ int fvm_destroy(fvm_ctx *c) {
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   for (auto &b : c->field) release(b);
-  for (DBuf *b : {&c->m_s1, &c->m_s2, &c->m_c, &c->m_n, &c->m_cn, &c->m_coff, &c->m_cface, &c->m_cnbr, &c->m_cvol, &c->m_fact,
+  for (DBuf *b : {&c->m_s1, &c->m_s2, &c->m_fpos, &c->m_cn, &c->m_coff, &c->m_cface, &c->m_cnbr, &c->m_cvol, &c->m_fact,
                   &c->m_soff, &c->m_sent, &c->rec, &c->tmp0, &c->tmp1, &c->tmp2, &c->stage,
                   &c->diag, &c->scalars})
     release(*b);
@@ -1511,6 +1597,7 @@ int fvm_upload_mesh(fvm_ctx *c, int np, int nactive, int nimport_loc, int nface,
   (void)hipSetDevice(c->device);
   fvm_fast_release(c);   // the fused state belongs to the previous mesh
   c->have_mesh = false;  // until the new mesh is complete
+  c->sub_layout = false;
   c->lists_complete = complete;
   const bool resize = np != c->np;
   c->np = np;
@@ -1529,7 +1616,6 @@ int fvm_upload_mesh(fvm_ctx *c, int np, int nactive, int nimport_loc, int nface,
   }
   int rc;
   if ((rc = ensure(c, c->m_s1, sizeof(int) * (size_t)nface)) || (rc = ensure(c, c->m_s2, sizeof(int) * (size_t)nface)) ||
-      (rc = ensure(c, c->m_c, sizeof(double) * 3 * (size_t)nface)) || (rc = ensure(c, c->m_n, sizeof(double) * 3 * (size_t)nface)) ||
       (rc = ensure(c, c->m_cn, sizeof(double) * 6 * (size_t)nface + 8)) ||
       (rc = ensure(c, c->m_coff, sizeof(int) * (size_t)(nactive + 1))) || (rc = ensure(c, c->m_cface, sizeof(int) * (size_t)nref)) ||
       (rc = ensure(c, c->m_cnbr, sizeof(int) * (size_t)nref)) ||
@@ -1537,8 +1623,8 @@ int fvm_upload_mesh(fvm_ctx *c, int np, int nactive, int nimport_loc, int nface,
     return rc;
   if (nface > 0) {
     HIPCHK(c, hipMemcpyAsync(c->stage.p, faces, sizeof(fvm_face) * (size_t)nface, hipMemcpyHostToDevice, c->stream));
-    LAUNCH(c, fvm::k_faces_to_soa, nface, (const fvm_face *)c->stage.p, nface, (int *)c->m_s1.p, (int *)c->m_s2.p,
-           (double *)c->m_c.p, (double *)c->m_n.p, (double *)c->m_cn.p);
+    LAUNCH(c, fvm::k_split_faces, nface, (const fvm_face *)c->stage.p, nface, (int *)c->m_s1.p, (int *)c->m_s2.p,
+           (double *)c->m_cn.p);
   }
   HIPCHK(c, hipMemcpyAsync(c->m_coff.p, cell_face_off, sizeof(int) * (size_t)(nactive + 1), hipMemcpyHostToDevice, c->stream));
   if (nref > 0) HIPCHK(c, hipMemcpyAsync(c->m_cface.p, cell_face, sizeof(int) * (size_t)nref, hipMemcpyHostToDevice, c->stream));
@@ -1563,6 +1649,7 @@ int fvm_upload_faces(fvm_ctx *c, int np, int nactive, int nimport_loc, int nface
   (void)hipSetDevice(c->device);
   fvm_fast_release(c);   // the fused state belongs to the previous mesh
   c->have_mesh = false;  // until the new mesh is complete
+  c->sub_layout = false;
   c->lists_complete = true;  // built below, every face under each active cell
   const bool resize = np != c->np;
   for (int f = 0; f < FVM_NFIELDS; f++) {
@@ -1575,7 +1662,6 @@ int fvm_upload_faces(fvm_ctx *c, int np, int nactive, int nimport_loc, int nface
   }
   int rc;
   if ((rc = ensure(c, c->m_s1, sizeof(int) * (size_t)nface)) || (rc = ensure(c, c->m_s2, sizeof(int) * (size_t)nface)) ||
-      (rc = ensure(c, c->m_c, sizeof(double) * 3 * (size_t)nface)) || (rc = ensure(c, c->m_n, sizeof(double) * 3 * (size_t)nface)) ||
       (rc = ensure(c, c->m_cn, sizeof(double) * 6 * (size_t)nface + 8)) ||
       (rc = ensure(c, c->m_coff, sizeof(int) * (size_t)(nactive + 1))) || (rc = ensure(c, c->m_cface, sizeof(int) * 2 * (size_t)nface + 4)) ||
       (rc = ensure(c, c->m_cnbr, sizeof(int) * 2 * (size_t)nface + 4)) ||
@@ -1586,8 +1672,8 @@ int fvm_upload_faces(fvm_ctx *c, int np, int nactive, int nimport_loc, int nface
   LAUNCH(c, fvm::k_fill_int, nactive + 1, cnt, 0, nactive + 1);
   if (nface > 0) {
     HIPCHK(c, hipMemcpyAsync(c->stage.p, faces, sizeof(fvm_face) * (size_t)nface, hipMemcpyHostToDevice, c->stream));
-    LAUNCH(c, fvm::k_faces_to_soa, nface, (const fvm_face *)c->stage.p, nface, (int *)c->m_s1.p, (int *)c->m_s2.p,
-           (double *)c->m_c.p, (double *)c->m_n.p, (double *)c->m_cn.p);
+    LAUNCH(c, fvm::k_split_faces, nface, (const fvm_face *)c->stage.p, nface, (int *)c->m_s1.p, (int *)c->m_s2.p,
+           (double *)c->m_cn.p);
     LAUNCH(c, fvm::k_csr_count, nface, (const int *)c->m_s1.p, (const int *)c->m_s2.p, nface, nactive, cnt);
   }
   if (fvm::exclusive_scan(c->scan, cnt, (int *)c->m_coff.p, nactive + 1, c->stream))
@@ -1598,7 +1684,7 @@ int fvm_upload_faces(fvm_ctx *c, int np, int nactive, int nimport_loc, int nface
   if (nface > 0) {
     LAUNCH(c, fvm::k_csr_fill, nface, (const int *)c->m_s1.p, (const int *)c->m_s2.p, nface, nactive, cursor,
            (int *)c->m_cface.p);
-    LAUNCH(c, fvm::k_csr_sort, nactive, (const int *)c->m_coff.p, nactive, (int *)c->m_cface.p);
+    LAUNCH(c, fvm::k_csr_sort, fvm::cell_lanes(nactive), (const int *)c->m_coff.p, nactive, (int *)c->m_cface.p);
     LAUNCH(c, fvm::k_cell_nbr, fvm::cell_lanes(nactive), (const int *)c->m_coff.p, (const int *)c->m_cface.p,
            (const int *)c->m_s1.p, (const int *)c->m_s2.p, nactive, (int *)c->m_cnbr.p);
   }
@@ -1672,14 +1758,36 @@ int fvm_download_field(fvm_ctx *c, int field, void *host, int np) {
   return FVM_OK;
 }
 
-// face-end lists of every cell over the current face_active_list
-static int build_face_ends(fvm_ctx *c) {
+// Face-end lists of every cell over the current face_active_list: from the
+// cells' lists when every cell has a complete one (fpos: the faces' places in
+// the active list), otherwise by counting over the active faces
+static int build_face_ends(fvm_ctx *c, bool from_lists) {
   const int np = c->np, nfa = c->nfa;
   int rc;
   if ((rc = ensure(c, c->m_soff, sizeof(int) * (size_t)(np + 1))) || (rc = ensure(c, c->m_sent, sizeof(int) * 2 * (size_t)nfa + 4)) ||
       (rc = ensure(c, c->tmp0, sizeof(int) * (size_t)(np + 1))))
     return rc;
   int *cnt = (int *)c->tmp0.p;
+  if (from_lists) {
+    fvm::EndLists E{};
+    E.np = np;
+    E.nactive = c->nactive;
+    E.coff = (const int *)c->m_coff.p;
+    E.cface = (const int *)c->m_cface.p;
+    E.s1 = (const int *)c->m_s1.p;
+    E.fpos = (const int *)c->m_fpos.p;
+    if (c->sub_layout) {
+      E.perm = (const int *)c->sub.perm.p;
+      E.goff = (const int *)c->sub.goff.p;
+      E.gface = (const int *)c->sub.gface.p;
+      E.gmark = (const int *)c->sub.fmark.p;
+      E.gpos = (const int *)c->sub.fpos.p;
+    }
+    LAUNCH_X(c, fvm::k_end_lists<true>, fvm::cell_lanes(np), E, cnt, nullptr, nullptr);
+    if (fvm::exclusive_scan(c->scan, cnt, (int *)c->m_soff.p, np, c->stream, true)) return fail(c, FVM_EHIP, "scan failed");
+    LAUNCH_X(c, fvm::k_end_lists<false>, fvm::cell_lanes(np), E, nullptr, (const int *)c->m_soff.p, (int *)c->m_sent.p);
+    return FVM_OK;
+  }
   HIPCHK(c, hipMemsetAsync(cnt, 0, sizeof(int) * (size_t)(np + 1), c->stream));
   fvm::MeshView M = meshview(c);
   LAUNCH(c, fvm::k_end_count, nfa, M, cnt);
@@ -1700,25 +1808,29 @@ int fvm_get_active_faces(fvm_ctx *c, int *nface_active) {
   int rc;
   if ((rc = ensure(c, c->tmp1, sizeof(int) * ((size_t)std::max(c->nface, nref) + 1))) ||
       (rc = ensure(c, c->tmp2, sizeof(int) * ((size_t)nref + 1))) || (rc = ensure(c, c->tmp0, sizeof(int) * ((size_t)nref + 1))) ||
-      (rc = ensure(c, c->m_fact, sizeof(int) * ((size_t)c->nface + 1))))
+      (rc = ensure(c, c->m_fact, sizeof(int) * ((size_t)c->nface + 1))) ||
+      (rc = ensure(c, c->m_fpos, sizeof(int) * ((size_t)c->nface + 1))))
     return rc;
-  int *firstpos = (int *)c->tmp1.p, *flag = (int *)c->tmp2.p, *pos = (int *)c->tmp0.p;
+  int *firstpos = (int *)c->tmp1.p, *flag = (int *)c->tmp2.p, *pos = (int *)c->tmp0.p, *fpos = (int *)c->m_fpos.p;
   fvm::MeshView M = meshview(c);
   if (c->lists_complete) {
-    LAUNCH(c, fvm::k_face_firstflag_direct, c->nactive, M, (const int *)c->field[FVM_FIELD_BND].p, c->nactive, flag);
+    LAUNCH(c, fvm::k_face_firstflag_direct, fvm::cell_lanes(c->nactive), M, (const int *)c->field[FVM_FIELD_BND].p, c->nactive, flag);
   } else {
     LAUNCH(c, fvm::k_fill_int, c->nface, firstpos, INT_MAX, c->nface);
     LAUNCH(c, fvm::k_face_firstpos, c->nactive, M, (const int *)c->field[FVM_FIELD_BND].p, c->nactive, firstpos);
     LAUNCH(c, fvm::k_face_firstflag, c->nactive, M, (const int *)c->field[FVM_FIELD_BND].p, c->nactive, firstpos, flag);
   }
-  int total = 0;
+  // a substep without boundary cells: every face of its complete lists is active
+  const bool all = c->lists_complete && c->sub_layout && !c->sub.has_bnd;
+  int total = all ? c->nface : 0;
+  if (!all) LAUNCH(c, fvm::k_fill_int, c->nface, fpos, -1, c->nface);
   if (nref > 0) {
-    rc = fvm::exclusive_scan_flags(c->scan, flag, pos, nref, &total, c->stream);
+    rc = fvm::exclusive_scan_flags(c->scan, flag, pos, nref, all ? nullptr : &total, c->stream);
     if (rc) return fail(c, FVM_EHIP, "flag scan failed");
-    LAUNCH(c, fvm::k_face_compact, nref, M, flag, pos, nref, (int *)c->m_fact.p);
+    LAUNCH(c, fvm::k_face_compact, nref, M, flag, pos, nref, (int *)c->m_fact.p, fpos);
   }
   c->nfa = total;
-  rc = build_face_ends(c);
+  rc = build_face_ends(c, c->lists_complete && (c->nactive == c->np || c->sub_layout));
   if (rc) return rc;
   if ((rc = finish(c))) return rc;
   *nface_active = total;
@@ -1736,7 +1848,7 @@ int fvm_set_active_faces(fvm_ctx *c, int nfa, const int *face_active) {
   if (rc) return rc;
   if (nfa > 0) HIPCHK(c, hipMemcpyAsync(c->m_fact.p, face_active, sizeof(int) * (size_t)nfa, hipMemcpyHostToDevice, c->stream));
   c->nfa = nfa;
-  rc = build_face_ends(c);
+  rc = build_face_ends(c, false);  // the list may name a face more than once
   if (rc) return rc;
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return FVM_OK;

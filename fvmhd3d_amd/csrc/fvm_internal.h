@@ -14,16 +14,20 @@ __host__ __device__ inline double smin_h(double a, double b) { return (b < a) ? 
 
 // Scratch of the device prefix scans (grown on demand, owned by a context).
 struct ScanScratch {
+  static constexpr int kTotals = 2;
   int *block_sums = nullptr;
   int *block_offs = nullptr;
-  int *total = nullptr;
+  int *total_h = nullptr;  // pinned: totals, valid once the stream has been waited for
   size_t nblocks = 0;
 };
 
-// out[i] = sum_{k<i} in[k] over n ints.
-int exclusive_scan(ScanScratch &s, const int *in, int *out, int n, hipStream_t st);
-// same for 0/1 flags with wavefront ballots; *total receives the count (host).
-int exclusive_scan_flags(ScanScratch &s, const int *flags, int *out, int n, int *total, hipStream_t st);
+// out[i] = sum_{k<i} in[k] over n ints; the total at out[n] (end) and in
+// total_h[slot].
+int exclusive_scan(ScanScratch &s, const int *in, int *out, int n, hipStream_t st, bool end = false, int slot = 0);
+// same for 0/1 flags with wavefront ballots; *total receives the count (host,
+// waits for the stream; NULL: no wait); list[base ..] the flagged elements.
+int exclusive_scan_flags(ScanScratch &s, const int *flags, int *out, int n, int *total, hipStream_t st,
+                         int *list = nullptr, int base = 0);
 void scan_release(ScanScratch &s);
 
 // every face listed once under each of its active cells (fvm_gpu.hip)
@@ -70,7 +74,10 @@ struct SubstepState {
   bool ready = false;
   bool complete = false;  // the global cell lists list every face under each of its cells
   int n = 0, nface = 0, nref = 0;
-  DBuf gs1, gs2, gc, gn, goff, gface, gnbr, gvol;  // global mesh (SoA; gnbr: the other cell of every gface entry)
+  // global mesh: cells of every face, its record (centroid, n), the cells' lists,
+  // the other cell of every list entry, volumes
+  DBuf gs1, gs2, gcn, goff, gface, gnbr, gvol;
+  bool has_bnd = false;  // a boundary flag was uploaded
   DBuf g[FVM_NFIELDS];                        // global fields, a row of components per cell [i*width + k]
   DBuf rung;                                  // int per cell
   DBuf act, apos, fmark, fpos, fl, cmark, iflag, ipos, g2l, perm, len, hist, err;
@@ -115,9 +122,13 @@ struct fvm_ctx {
   // (fvm_set_face_precision)
   bool face32 = false;
   DBuf field[FVM_NFIELDS];
+  DBuf m_s1, m_s2, m_coff, m_cface, m_cvol, m_fact, m_soff, m_sent;
+  DBuf m_cn;    // per-face geometry record (centroid, n)
   DBuf m_cnbr;  // the other cell of every m_cface entry
-  DBuf m_s1, m_s2, m_c, m_n, m_coff, m_cface, m_cvol, m_fact, m_soff, m_sent;
-  DBuf m_cn;  // per-face geometry record (centroid, n) of the same faces as m_c / m_n
+  DBuf m_fpos;  // place of every face in the active list, -1 when it is not in it
+  // the mesh is a substep's layout: the inactive cells' faces are found through
+  // the global lists (sub.goff, gface, fpos, fmark)
+  bool sub_layout = false;
   DBuf rec, tmp0, tmp1, tmp2, stage;
   DBuf diag;     // unsigned long long[FVM_NDIAG]
   DBuf scalars;  // unsigned long long[8]

@@ -1478,7 +1478,8 @@ int fvm_create(fvm_ctx **out, int device, const fvm_params *params) {
     return FVM_EHIP;
   }
   (void)hipMemsetAsync(c->diag.p, 0, c->diag.bytes, c->stream);
-  if (noalloc_scratch_init(device) != FVM_OK) {
+  fvm_xfer_ref();
+  if (noalloc_scratch_init(device) != FVM_OK || hipHostMalloc((void **)&c->pin, (size_t)1 << 20, hipHostMallocDefault) != hipSuccess) {
     (void)fvm_destroy(c);
     return FVM_EHIP;
   }
@@ -1498,6 +1499,8 @@ int fvm_destroy(fvm_ctx *c) {
   fvm::scan_release(c->scan);
   fvm_fast_release(c);
   fvm_substep_release(c);
+  if (c->pin) (void)hipHostFree(c->pin);
+  fvm_xfer_unref(c);
   for (hipEvent_t &e : c->kt.ev)
     if (e) (void)hipEventDestroy(e);
   if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -1622,12 +1625,12 @@ int fvm_upload_mesh(fvm_ctx *c, int np, int nactive, int nimport_loc, int nface,
       (rc = ensure(c, c->m_cvol, sizeof(double) * (size_t)nactive)) || (rc = ensure(c, c->stage, sizeof(fvm_face) * (size_t)nface)))
     return rc;
   if (nface > 0) {
-    HIPCHK(c, hipMemcpyAsync(c->stage.p, faces, sizeof(fvm_face) * (size_t)nface, hipMemcpyHostToDevice, c->stream));
+    if ((rc = fvm_to_device(c, c->stage.p, faces, sizeof(fvm_face) * (size_t)nface))) return rc;
     LAUNCH(c, fvm::k_split_faces, nface, (const fvm_face *)c->stage.p, nface, (int *)c->m_s1.p, (int *)c->m_s2.p,
            (double *)c->m_cn.p);
   }
   HIPCHK(c, hipMemcpyAsync(c->m_coff.p, cell_face_off, sizeof(int) * (size_t)(nactive + 1), hipMemcpyHostToDevice, c->stream));
-  if (nref > 0) HIPCHK(c, hipMemcpyAsync(c->m_cface.p, cell_face, sizeof(int) * (size_t)nref, hipMemcpyHostToDevice, c->stream));
+  if (nref > 0 && (rc = fvm_to_device(c, c->m_cface.p, cell_face, sizeof(int) * (size_t)nref))) return rc;
   if (nactive > 0) HIPCHK(c, hipMemcpyAsync(c->m_cvol.p, cell_volume, sizeof(double) * (size_t)nactive, hipMemcpyHostToDevice, c->stream));
   LAUNCH(c, fvm::k_cell_nbr, fvm::cell_lanes(nactive), (const int *)c->m_coff.p, (const int *)c->m_cface.p,
          (const int *)c->m_s1.p, (const int *)c->m_s2.p, nactive, (int *)c->m_cnbr.p);
@@ -1671,7 +1674,7 @@ int fvm_upload_faces(fvm_ctx *c, int np, int nactive, int nimport_loc, int nface
   int *cnt = (int *)c->tmp0.p, *cursor = (int *)c->tmp1.p;
   LAUNCH(c, fvm::k_fill_int, nactive + 1, cnt, 0, nactive + 1);
   if (nface > 0) {
-    HIPCHK(c, hipMemcpyAsync(c->stage.p, faces, sizeof(fvm_face) * (size_t)nface, hipMemcpyHostToDevice, c->stream));
+    if ((rc = fvm_to_device(c, c->stage.p, faces, sizeof(fvm_face) * (size_t)nface))) return rc;
     LAUNCH(c, fvm::k_split_faces, nface, (const fvm_face *)c->stage.p, nface, (int *)c->m_s1.p, (int *)c->m_s2.p,
            (double *)c->m_cn.p);
     LAUNCH(c, fvm::k_csr_count, nface, (const int *)c->m_s1.p, (const int *)c->m_s2.p, nface, nactive, cnt);
@@ -1725,7 +1728,7 @@ int fvm_upload_field(fvm_ctx *c, int field, const void *host, int np) {
     const size_t bytes = sizeof(double) * (size_t)fi.width * (size_t)np;
     int rc = ensure(c, c->stage, bytes);
     if (rc) return rc;
-    HIPCHK(c, hipMemcpyAsync(c->stage.p, host, bytes, hipMemcpyHostToDevice, c->stream));
+    if ((rc = fvm_to_device(c, c->stage.p, host, bytes))) return rc;
     if (fi.kind == fvm::K_STORE && c->prm.storage == FVM_STORAGE_SHIPPED)
       LAUNCH(c, fvm::k_aos_to_soa<float>, np, (const double *)c->stage.p, (float *)c->field[field].p, np, fi.width);
     else
@@ -1752,7 +1755,7 @@ int fvm_download_field(fvm_ctx *c, int field, void *host, int np) {
       LAUNCH(c, fvm::k_soa_to_aos<float>, np, (const float *)c->field[field].p, (double *)c->stage.p, np, fi.width);
     else
       LAUNCH(c, fvm::k_soa_to_aos<double>, np, (const double *)c->field[field].p, (double *)c->stage.p, np, fi.width);
-    HIPCHK(c, hipMemcpyAsync(host, c->stage.p, bytes, hipMemcpyDeviceToHost, c->stream));
+    return fvm_to_host(c, host, c->stage.p, bytes);
   }
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return FVM_OK;
@@ -2068,11 +2071,73 @@ int fvm_compute_predictor(fvm_ctx *c, double dtmax, int min_rung) {
   return DISPATCH(c, do_predictor, c, dtmax, min_rung);
 }
 
+// faces [f0, f0 + n) of a batch through contiguous staging: in h (host, pinned)
+// and d (device) the inputs of the n faces, then their outputs, in the batch's
+// array order (FVM_FLUX_BYTES_PER_FACE a face)
+namespace {
+struct FluxBatch {
+  const double *wij, *Wi, *Wj;
+  const int *jbnd;
+  const double *normal;
+  double *psi, *Bn, *flux;
+};
+constexpr size_t FLUX_IN_D = 26, FLUX_OUT_D = 12;  // doubles in and out per face, and one int in
+static_assert(FVM_FLUX_BYTES_PER_FACE == 8 * (FLUX_IN_D + FLUX_OUT_D) + 4, "face bytes");
+
+hipError_t flux_chunk(double gamma, const FluxBatch &b, size_t f0, size_t n, char *h, char *d, hipStream_t st) {
+  double *hw = (double *)h, *hi = hw + 3 * n, *hj = hi + 10 * n, *hn = hj + 10 * n, *ho = hn + 3 * n;
+  int *hb = (int *)(ho + FLUX_OUT_D * n);
+  double *dw = (double *)d, *di = dw + 3 * n, *dj = di + 10 * n, *dn = dj + 10 * n, *dpsi = dn + 3 * n, *dBn = dpsi + n,
+         *dfl = dBn + n;
+  int *db = (int *)(dfl + 10 * n);
+  std::memcpy(hw, b.wij + 3 * f0, 24 * n);
+  std::memcpy(hi, b.Wi + 10 * f0, 80 * n);
+  std::memcpy(hj, b.Wj + 10 * f0, 80 * n);
+  std::memcpy(hn, b.normal + 3 * f0, 24 * n);
+  std::memcpy(hb, b.jbnd + f0, 4 * n);
+  hipError_t e = hipMemcpyAsync(d, h, 8 * FLUX_IN_D * n, hipMemcpyHostToDevice, st);
+  if (e == hipSuccess) e = hipMemcpyAsync(db, hb, 4 * n, hipMemcpyHostToDevice, st);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(fvm::k_flux_batch, dim3(nblk((long)n)), dim3(256), 0, st, (int)n, gamma, dw, di, dj, db, dn, dpsi, dBn, dfl);
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+  e = hipMemcpyAsync(ho, dpsi, 8 * FLUX_OUT_D * n, hipMemcpyDeviceToHost, st);
+  if (e == hipSuccess) e = hipStreamSynchronize(st);
+  if (e != hipSuccess) return e;
+  std::memcpy(b.psi + f0, ho, 8 * n);
+  std::memcpy(b.Bn + f0, ho + n, 8 * n);
+  std::memcpy(b.flux + 10 * f0, ho + 2 * n, 80 * n);
+  return hipSuccess;
+}
+}  // namespace
+// faces of a small batch (the context's pinned staging, 1 MiB) and of a chunk of
+// a large one (a transfer slot); batches from two chunks up go chunk by chunk
+// over the transfer threads, uploads, kernels and downloads overlapping
+constexpr int FLUX_PIN = (1 << 20) / FVM_FLUX_BYTES_PER_FACE;
+constexpr int FLUX_CHUNK = 16384;
+static_assert((size_t)FLUX_CHUNK * FVM_FLUX_BYTES_PER_FACE <= fvm::kXferSlot, "a chunk fits a slot");
+
 // the batched computeFlux through device staging at base (room for n faces:
-// FVM_FLUX_BYTES_PER_FACE each): inputs in, one launch, outputs out, synchronous
-static int flux_batch_staged(fvm_ctx *c, char *base, int n, const double *wij, const double *Wi, const double *Wj,
+// FVM_FLUX_BYTES_PER_FACE each), synchronous; threads: the transfer threads may
+// be used (their slots and streams are allocated on first use)
+static int flux_batch_staged(fvm_ctx *c, char *base, bool threads, int n, const double *wij, const double *Wi, const double *Wj,
                              const int *jbnd, const double *normal, double *psi, double *Bn, double *flux) {
   const size_t N = (size_t)n;
+  const FluxBatch b{wij, Wi, Wj, jbnd, normal, psi, Bn, flux};
+  if (n <= FLUX_PIN && c->pin) {
+    HIPCHK(c, flux_chunk(c->prm.gamma_gas, b, 0, N, c->pin, base, c->stream));
+    return FVM_OK;
+  }
+  if (threads && n >= 2 * FLUX_CHUNK) {
+    hipError_t err = hipSuccess;
+    HIPCHK(c, hipStreamSynchronize(c->stream));  // the staging may be in use by work before this call
+    if (fvm_xfer_chunks(c, (n + FLUX_CHUNK - 1) / FLUX_CHUNK, [&](int k, char *slot, hipStream_t st) {
+          const size_t f0 = (size_t)k * FLUX_CHUNK, m = std::min<size_t>(N - f0, FLUX_CHUNK);
+          return flux_chunk(c->prm.gamma_gas, b, f0, m, slot, base + f0 * FVM_FLUX_BYTES_PER_FACE, st);
+        }, &err)) {
+      HIPCHK(c, err);
+      return FVM_OK;
+    }
+  }
   double *d_wij = (double *)base, *d_Wi = d_wij + 3 * N, *d_Wj = d_Wi + 10 * N, *d_n = d_Wj + 10 * N, *d_psi = d_n + 3 * N,
          *d_Bn = d_psi + N, *d_flux = d_Bn + N;
   int *d_jb = (int *)(d_flux + 10 * N);
@@ -2098,7 +2163,7 @@ int fvm_compute_flux(fvm_ctx *c, int n, const double *wij, const double *Wi, con
   (void)hipSetDevice(c->device);
   int rc = ensure(c, c->stage, (size_t)FVM_FLUX_BYTES_PER_FACE * (size_t)n);
   if (rc) return rc;
-  return flux_batch_staged(c, (char *)c->stage.p, n, wij, Wi, Wj, jbnd, normal, psi, Bn, flux);
+  return flux_batch_staged(c, (char *)c->stage.p, true, n, wij, Wi, Wj, jbnd, normal, psi, Bn, flux);
 }
 
 int fvm_compute_flux_noalloc(fvm_ctx *c, int n, const double *wij, const double *Wi, const double *Wj,
@@ -2113,7 +2178,7 @@ int fvm_compute_flux_noalloc(fvm_ctx *c, int n, const double *wij, const double 
   (void)hipSetDevice(c->device);
   char *base = (char *)noalloc_scratch(c->device);
   if (!base) return fail(c, FVM_ESTATE, "fvm_compute_flux_noalloc: no staging address for this device");
-  return flux_batch_staged(c, base, n, wij, Wi, Wj, jbnd, normal, psi, Bn, flux);
+  return flux_batch_staged(c, base, false, n, wij, Wi, Wj, jbnd, normal, psi, Bn, flux);
 }
 
 int fvm_get_diagnostics(fvm_ctx *c, long long *out, int n) {

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <string>
 #include <vector>
 
@@ -29,6 +30,12 @@ int exclusive_scan(ScanScratch &s, const int *in, int *out, int n, hipStream_t s
 int exclusive_scan_flags(ScanScratch &s, const int *flags, int *out, int n, int *total, hipStream_t st,
                          int *list = nullptr, int base = 0);
 void scan_release(ScanScratch &s);
+
+// host transfers (fvm_xfer.hip): threads, pinned bytes per thread, and the size
+// from which a transfer uses them (below, starting the threads costs more than
+// they gain)
+constexpr int kXferThreads = 4;
+constexpr size_t kXferSlot = (size_t)5 << 20, kXferMin = (size_t)8 << 20;
 
 // every face listed once under each of its active cells (fvm_gpu.hip)
 bool lists_complete(int nactive, int nface, const fvm_face *faces, const int *cell_face_off, const int *cell_face);
@@ -135,6 +142,8 @@ struct fvm_ctx {
   fvm::ScanScratch scan;
   FusedState fz;
   SubstepState sub;
+  hipStream_t xstream[fvm::kXferThreads - 1] = {};  // of the transfer threads (created on first use)
+  char *pin = nullptr;  // pinned staging of small computeFlux batches
   // HIP-event timing of the reference-order kernels (fvm_kernel_timing): per
   // kernel FVM_KT_*, total milliseconds and launches since timing was enabled
   struct {
@@ -148,6 +157,16 @@ struct fvm_ctx {
 int fvm_fail(fvm_ctx *c, int code, const std::string &msg);
 int fvm_ensure(fvm_ctx *c, DBuf &b, size_t bytes);
 void fvm_release(DBuf &b);
+
+// host transfers (fvm_xfer.hip)
+void fvm_xfer_ref();
+void fvm_xfer_unref(fvm_ctx *c);
+bool fvm_xfer_run(fvm_ctx *c, int n, hipError_t (*chunk)(void *, int, char *, hipStream_t), void *arg, hipError_t *err);
+template <typename F> bool fvm_xfer_chunks(fvm_ctx *c, int n, F chunk, hipError_t *err) {
+  return fvm_xfer_run(c, n, [](void *f, int k, char *slot, hipStream_t st) { return (*(F *)f)(k, slot, st); }, &chunk, err);
+}
+int fvm_to_device(fvm_ctx *c, void *dst, const void *src, size_t bytes);
+int fvm_to_host(fvm_ctx *c, void *dst, const void *src, size_t bytes);
 
 // release of the fused-path buffers of a context (fvm_fast.hip)
 void fvm_fast_release(fvm_ctx *c);

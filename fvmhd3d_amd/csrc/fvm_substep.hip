@@ -954,8 +954,7 @@ int fvm_substep_upload(fvm_ctx *c, int field, const void *host, int ncell) {
     const int *b = (const int *)host;
     s.has_bnd = std::any_of(b, b + ncell, [](int v) { return v != FVM_NO_BOUNDARY; });
   }
-  SCHK(c, hipMemcpy(s.g[field].p, host, (kInt[field] ? 4 : 8) * (size_t)kWidth[field] * ncell, hipMemcpyHostToDevice));
-  return FVM_OK;
+  return fvm_to_device(c, s.g[field].p, host, (kInt[field] ? 4 : 8) * (size_t)kWidth[field] * ncell);
 }
 
 int fvm_substep_download(fvm_ctx *c, int field, void *host, int ncell) {
@@ -969,8 +968,7 @@ int fvm_substep_download(fvm_ctx *c, int field, void *host, int ncell) {
   }
   if (field < 0 || field >= FVM_NFIELDS || !kept(field))
     return fvm_fail(c, FVM_EARG, "fvm_substep_download: field is not kept between substeps");
-  SCHK(c, hipMemcpy(host, s.g[field].p, (kInt[field] ? 4 : 8) * (size_t)kWidth[field] * ncell, hipMemcpyDeviceToHost));
-  return FVM_OK;
+  return fvm_to_host(c, host, s.g[field].p, (kInt[field] ? 4 : 8) * (size_t)kWidth[field] * ncell);
 }
 
 int fvm_substep_init_rungs(fvm_ctx *c, double dtmax, int nrung, int *rung_hist) {

@@ -355,6 +355,34 @@ struct Dr3 {
   float x, y, z;
 };
 
+// Four lanes per cell (the quad kernels of small meshes): lane L's value in all
+// four, and a reduction over the four by an exact, order-free operation
+template <int L> __device__ __forceinline__ int quad_get(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, L * 0x55, 0xf, 0xf, true);
+}
+template <int L> __device__ __forceinline__ float quad_get(float v) { return __int_as_float(quad_get<L>(__float_as_int(v))); }
+template <int L> __device__ __forceinline__ double quad_get(double v) {
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = (unsigned)quad_get<L>((int)(unsigned)b), hi = (unsigned)quad_get<L>((int)(unsigned)(b >> 32));
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+template <int C> __device__ __forceinline__ float quad_swap(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), C, 0xf, 0xf, true));
+}
+template <int C> __device__ __forceinline__ double quad_swap(double v) {
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)b, C, 0xf, 0xf, true);
+  const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), C, 0xf, 0xf, true);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+// x is final here: none of the operations that form it moves past this point
+__device__ __forceinline__ void keep_here(float &x) { __asm__ volatile("" : "+v"(x)); }
+__device__ __forceinline__ void keep_here(double &x) { __asm__ volatile("" : "+v"(x)); }
+template <typename T, typename F> __device__ __forceinline__ T quad_reduce(T v, F f) {
+  v = f(v, quad_swap<0xB1>(v));     // lanes 1 0 3 2
+  return f(v, quad_swap<0x4E>(v));  // lanes 2 3 0 1
+}
+
 // the slope limiter's time offset for a step of length dt from t0: every cell
 // has tend = t0 + dt, so dtI = dt, dth = dt / 2 and dtt = dtI - dth
 __device__ __forceinline__ float limiter_dtt(double t0, double dt_glob) {
@@ -367,8 +395,9 @@ __device__ __forceinline__ float limiter_dtt(double t0, double dt_glob) {
 // both FP32 limiters of one cell from one pass over its own-side offsets: mn /
 // mx the raw neighbour differences, tv and gg (x, y, z blocks) Wt and the
 // gradients, limited in place
-template <int LIM>
-__device__ __forceinline__ void limit_cell32(const FusedArgs<float> &A, int e0, int deg, const float *mn,
+// (LPC > 1: the cell's LPC lanes take every LPC-th face, sub the lane's place)
+template <int LIM, int LPC>
+__device__ __forceinline__ void limit_cell32(const FusedArgs<float> &A, int e0, int deg, int sub, const float *mn,
                                              const float *mx, float dtt, float *tv, float *gg) {
   // extremes of d_f = grad . dr_f over the faces; the slope limiter's
   // y_f = d_f + t dtt differs by a face-independent term, and rounding is
@@ -381,10 +410,10 @@ __device__ __forceinline__ void limit_cell32(const FusedArgs<float> &A, int e0, 
   // the own-side offsets only (12 bytes per face-end, not the 32-byte record)
   const Dr3 *fdr = reinterpret_cast<const Dr3 *>(A.fdr);
   Dr3 rn;
-  if (deg > 0) rn = fdr[e0];
-  for (int q = 0, e = e0; q < deg; q++, e += 64) {
+  if (deg > sub) rn = fdr[e0 + 64 * sub];
+  for (int q = sub, e = e0 + 64 * sub; q < deg; q += LPC, e += 64 * LPC) {
     const Dr3 r = rn;
-    if (q + 1 < deg) rn = fdr[e + 64];
+    if (q + LPC < deg) rn = fdr[e + 64 * LPC];
     const float dr[3] = {r.x, r.y, r.z};
     for (int k = 0; k < NF; k++) {
       const float d = gg[k] * dr[0] + gg[NF + k] * dr[1] + gg[2 * NF + k] * dr[2];
@@ -392,6 +421,11 @@ __device__ __forceinline__ void limit_cell32(const FusedArgs<float> &A, int e0, 
       dmax[k] = smax(dmax[k], d);
     }
   }
+  if constexpr (LPC > 1)
+    for (int k = 0; k < NF; k++) {
+      dmin[k] = quad_reduce(dmin[k], [](float a, float b) { return smin(a, b); });
+      dmax[k] = quad_reduce(dmax[k], [](float a, float b) { return smax(a, b); });
+    }
   for (int k = 0; k < NF; k++) {
     // the extremes start at 0 (a cell without faces gives 0, 0)
     const float dlo = smin(0.0f, dmin[k]), dhi = smax(0.0f, dmax[k]);
@@ -431,33 +465,201 @@ template <typename T> struct K1Waves {
   static constexpr int value = std::is_same<T, float>::value ? 3 : 1;
 };
 
+// global minimum of dt_new (dt > 0: IEEE bit patterns order like the values),
+// one atomic per block
+__device__ __forceinline__ void k1_minimum(unsigned long long *dtmin_bits, double v) {
+  for (int o = 32; o > 0; o >>= 1) v = smin(v, __shfl_xor(v, o));
+  __shared__ double wmin[FB / 64];
+  if (__lane_id() == 0) wmin[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < FB / 64; w++) v = smin(v, wmin[w]);
+    if (v < REF_HUGE && v >= 0.0) atomicMin(dtmin_bits, (unsigned long long)__double_as_longlong(v));
+  }
+}
+
+// FP32 path: the opt-in limiters and the half-step states of the records are
+// formed in the predictor kernel with the step's dt taken to be the last step's
+// (dt is the global minimum that kernel is computing).  A second launch
+// (k1_pass 1) compares it with the true dt: it returns at once when they agree
+// (every step of a run but the first, while the rung holds) and otherwise
+// redoes every cell with the true dt, so the result never depends on the guess.
+// The dt to use, or false where there is nothing to redo.
+template <typename T> __device__ __forceinline__ bool k1_step_dt(const FusedArgs<T> &A, double &dt_step) {
+  if constexpr (std::is_same<T, float>::value) {
+    dt_step = A.tdev[1];
+    if (A.k1_pass) {
+      const double dt_true = rung_dt0(A.dtmax, __longlong_as_double((long long)*A.dtmin_bits));
+      if (dt_true == dt_step) return false;
+      dt_step = dt_true;
+    }
+  }
+  return true;
+}
+
+// What a cell's pass over its face-ends leaves: reconstruction sums, neighbour
+// extremes, predictor sums, the CFL term
+template <typename T> struct K1Sums {
+  T gx[NF], gy[NF], gz[NF], dmn[NF], dmx[NF], pU[NF], pgp[3], pdv, gw[3];
+  double pdV, arg_max;
+};
+
+// The cell's CFL step, predictor update, gradients, limiters and record from its
+// sums; returns dt_new.  LPC lanes work on the cell (1 or 4, sub the lane's
+// place): all form the same values, the limiter passes and the stores are shared.
+template <typename T, int LIM, int LPC>
+__device__ __forceinline__ double k1_finish(const FusedArgs<T> &A, int c, int sub, int e0, int deg, double V, const T *Wc,
+                                            const double *pv, double dt_step, K1Sums<T> &S) {
+  constexpr bool LIMIT = LIM != LIM_SHIPPED;
+  constexpr bool FP32 = std::is_same<T, float>::value;
+  constexpr bool LIMIT32 = LIMIT && FP32;
+  const int n = A.n;
+  const double g64 = A.gamma;
+  T *gx = S.gx, *gy = S.gy, *gz = S.gz, *dmn = S.dmn, *dmx = S.dmx, *pU = S.pU, *pgp = S.pgp;
+  double dtn;
+  // --- predictor cell update (computePredictor.cpp:141-379), FP64
+  T tv[NF];
+  {
+    double U0[NF], W0[NF];
+    for (int k = 0; k < NF; k++) U0[k] = ntl(&SF(A.U, k, c, n));
+    to_primitive(U0, V, W0);
+    // CFL (computeTimestep.cpp:13-31), own-cell terms from the FP64 primitives
+    const double h = A.lmin[c];  // pow(V / (4 pi / 3), 1 / 3)
+    const double Pi = pressure(g64, W0[ETHM]) * g64;
+    const double B2i = W0[BX] * W0[BX] + W0[BY] * W0[BY] + W0[BZ] * W0[BZ];
+    const double csi = dsqrt((Pi + B2i) / W0[DENS]);
+    const double dvr[3] = {W0[VELX] - pv[0], W0[VELY] - pv[1], W0[VELZ] - pv[2]};
+    const double vrel = dsqrt(dvr[0] * dvr[0] + dvr[1] * dvr[1] + dvr[2] * dvr[2]);
+    double dti = h / (csi + vrel + 1.0 / REF_HUGE);
+    if (S.arg_max >= 0.0) dti = smin(dti, h / (csi + dsqrt(S.arg_max)));
+    dti = smin(dti, REF_HUGE);
+    dtn = dti * A.courant;
+    while (U0[MASS] + (double)pU[MASS] * dtn <= 0.0) dtn *= 0.5;
+    const double dt = rung_dt0(A.dtmax, dtn) / 128;
+    const double divB = (double)S.pdv;
+    double Uc[NF];
+    for (int k = 0; k < NF; k++) Uc[k] = U0[k] + (double)pU[k] * dt;
+    Uc[WBX] -= W0[VELX] * divB * dt;
+    Uc[WBY] -= W0[VELY] * divB * dt;
+    Uc[WBZ] -= W0[VELZ] * divB * dt;
+    const double pres = pressure(g64, W0[ETHM]);
+    const double B2 = W0[BX] * W0[BX] + W0[BY] * W0[BY] + W0[BZ] * W0[BZ];
+    const double dcs2 = g64 * pres + B2;
+    const double ch_sig = dsqrt(dcs2 / W0[DENS]);
+    Uc[WBX] -= (double)pgp[0] * dt;
+    Uc[WBY] -= (double)pgp[1] * dt;
+    Uc[WBZ] -= (double)pgp[2] * dt;
+    Uc[MPSI] -= dcs2 * divB * dt;
+    const double cr = 0.5;
+    const double l_min = A.lmin[c];
+    Uc[MPSI] *= exp(-cr * ch_sig / l_min * dt);
+    double W1[NF];
+    // exp(0) = 1 exactly: a static mesh skips the exponential
+    to_primitive(Uc, S.pdV == 0.0 ? V : V * exp(S.pdV * dt / V), W1);
+    const bool ef = W1[ETHM] <= 0.0;
+    if (ef) W1[ETHM] = ethm_from_entropy_d(g64, W1);
+    else W1[ENTR] = entropy_from_ethm_d(g64, W1);
+    if (!A.k1_pass) wave_count(&A.diag[FVM_DIAG_ETHM_FAILED], ef && sub == 0);  // a redo counts nothing twice
+    const double idt = 1.0 / dt;
+    for (int k = 0; k < NF; k++) tv[k] = (T)((W1[k] - W0[k]) * idt);
+  }
+
+  // --- reconstruction finish (computeReconstruction.cpp:162-239)
+  {
+    const double invV = 1.0 / V;
+    if constexpr (std::is_same<T, float>::value)
+      for (int k = 0; k < NF; k++) {
+        gx[k] += S.gw[0] * Wc[k];
+        gy[k] += S.gw[1] * Wc[k];
+        gz[k] += S.gw[2] * Wc[k];
+      }
+    for (int k = 0; k < NF; k++) {
+      gx[k] = (T)((double)gx[k] * invV);
+      gy[k] = (T)((double)gy[k] * invV);
+      gz[k] = (T)((double)gz[k] * invV);
+    }
+    if constexpr (LIMIT32) {
+      // FP32: the reconstruction and slope limiters in one pass over the
+      // own-side offsets, from the raw differences and the unlimited gradients
+      T gg[3 * NF];
+      for (int k = 0; k < NF; k++) {
+        gg[k] = gx[k];
+        gg[NF + k] = gy[k];
+        gg[2 * NF + k] = gz[k];
+      }
+      limit_cell32<LIM, LPC>(A, e0, deg, sub, dmn, dmx, limiter_dtt(A.tdev[0], dt_step), tv, gg);
+      for (int k = 0; k < NF; k++) {
+        gx[k] = gg[k];
+        gy[k] = gg[NF + k];
+        gz[k] = gg[2 * NF + k];
+      }
+    } else if constexpr (LIMIT) {
+      // extremes of the limiter's argument over the faces, divided once a
+      // variable (64^3 cells: this kernel 487 -> 376 us)
+      T lm[NF], lo[NF], hi[NF];
+      for (int k = 0; k < NF; k++) lo[k] = hi[k] = T(0.0);
+      for (int q = sub, e = e0 + 64 * sub; q < deg; q += LPC, e += 64 * LPC) {
+        const double *cen = A.fep + FP_CEN * A.slots + e;
+        const T c0 = cen[0], c1 = cen[A.slots], c2 = cen[2 * A.slots];
+        for (int k = 0; k < NF; k++) {
+          const T d = gx[k] * c0 + gy[k] * c1 + gz[k] * c2;
+          lo[k] = __builtin_fmin(lo[k], d);
+          hi[k] = __builtin_fmax(hi[k], d);
+        }
+      }
+      if constexpr (LPC > 1)
+        for (int k = 0; k < NF; k++) {
+          lo[k] = quad_reduce(lo[k], [](double a, double b) { return __builtin_fmin(a, b); });
+          hi[k] = quad_reduce(hi[k], [](double a, double b) { return __builtin_fmax(a, b); });
+        }
+      for (int k = 0; k < NF; k++) lm[k] = limiter_of_extremes<false>(LIM, lo[k], hi[k], dmn[k], dmx[k]);
+      for (int k = 0; k < NF; k++) {
+        if (sub == 0) SF(A.mm, k, c, n) = dmn[k] + Wc[k];
+        if (sub == LPC - 1) SF(A.mm, NF + k, c, n) = dmx[k] + Wc[k];
+        tv[k] = tv[k] * lm[k];
+        gx[k] = gx[k] * lm[k];
+        gy[k] = gy[k] * lm[k];
+        gz[k] = gz[k] * lm[k];
+      }
+    }
+    if constexpr (FP32) {
+      // the record starts from the half-step state W + Wt dti of the step,
+      // formed as the flux kernel formed it; Wt goes to its own array
+      const float dti = (float)step_times_dt(A.tdev[0], dt_step).dti;
+      T wh[NF];
+      for (int k = 0; k < NF; k++) wh[k] = half_step32(Wc[k], tv[k], dti);
+      T *r = A.rec_w + (size_t)c * REC32;
+      if (LPC == 1 || sub == 0) {
+        stv<NF>(r, wh);
+        stv<NF>(A.tv + (size_t)c * NF, tv);
+      }
+      if (LPC == 1 || sub == 1) stv<NF>(r + R32_G, gx);
+      if (LPC == 1 || sub == 2) stv<NF>(r + R32_G + NF, gy);
+      if (LPC == 1 || sub == 3) stv<NF>(r + R32_G + 2 * NF, gz);
+    } else {
+      T *wc = A.rec_w + (size_t)c * REC;
+      if (LPC == 1 || sub == 0) stv<NF>(wc + R_T, tv);
+      if (LPC == 1 || sub == 1) stv<NF>(wc + R_G, gx);
+      if (LPC == 1 || sub == 2) stv<NF>(wc + R_G + NF, gy);
+      if (LPC == 1 || sub == 3) stv<NF>(wc + R_G + 2 * NF, gz);
+    }
+  }
+  if (sub == 0) A.dt_new[c] = dtn;
+  return dtn;
+}
+
 template <typename T, bool MOVING, int LIM>
 __global__ void __launch_bounds__(FB) __attribute__((amdgpu_waves_per_eu(K1Waves<T>::value)))
 k_cfl_predict_recon(FusedArgs<T> A) {
   constexpr bool LIMIT = LIM != LIM_SHIPPED;
   constexpr bool FP32 = std::is_same<T, float>::value;
-  constexpr bool LIMIT32 = LIMIT && FP32;
-  // FP32 path: the opt-in limiters and the half-step states of the records are
-  // formed here with the step's dt taken to be the last step's (dt is the
-  // global minimum this kernel is computing).  A second launch (k1_pass 1)
-  // compares it with the true dt: it returns at once when they agree (every
-  // step of a run but the first, while the rung holds) and otherwise redoes
-  // every cell with the true dt, so the result never depends on the guess
   double dt_step = 0.0;
-  if constexpr (FP32) {
-    dt_step = A.tdev[1];
-    if (A.k1_pass) {
-      const double dt_true = rung_dt0(A.dtmax, __longlong_as_double((long long)*A.dtmin_bits));
-      if (dt_true == dt_step) return;  // uniform over the grid
-      dt_step = dt_true;
-    }
-  }
+  if (!k1_step_dt(A, dt_step)) return;  // uniform over the grid
   const int c = xcd_cell(A.n);
   const bool live = c < A.n;
   double dtn = REF_HUGE;
   if (live) {
     const int n = A.n;
-    const double g64 = A.gamma;
     const T g = (T)A.gamma;
     const double V = ntl(A.cvol + c);
     T Wc[NF];
@@ -467,38 +669,26 @@ k_cfl_predict_recon(FusedArgs<T> A) {
     double pv[3] = {0.0, 0.0, 0.0};
     if constexpr (MOVING)
       for (int d = 0; d < 3; d++) pv[d] = SF(A.mvel, d, c, n);
-    double v0[3], csi = 0.0, h = 0.0, dti = 0.0;
-    // the own-cell terms, from the FP64 primitives
-    auto cfl_cell = [&](const double *W0) {
-      h = A.lmin[c];  // pow(V / (4 pi / 3), 1 / 3)
-      const double Pi = pressure(g64, W0[ETHM]) * g64;
-      const double B2i = W0[BX] * W0[BX] + W0[BY] * W0[BY] + W0[BZ] * W0[BZ];
-      csi = dsqrt((Pi + B2i) / W0[DENS]);
-      const double dvr[3] = {W0[VELX] - pv[0], W0[VELY] - pv[1], W0[VELZ] - pv[2]};
-      const double vrel = dsqrt(dvr[0] * dvr[0] + dvr[1] * dvr[1] + dvr[2] * dvr[2]);
-      dti = h / (csi + vrel + 1.0 / REF_HUGE);
-    };
-    if constexpr (std::is_same<T, float>::value) {
+    double v0[3];
+    if constexpr (FP32) {
       // FP32 face path: the neighbour speed differences take the own velocity
       // from the FP32 record, as the neighbours' come from theirs; U is read
       // once, after the face loop, for the own-cell terms and the predictor
       for (int d = 0; d < 3; d++) v0[d] = (double)Wc[VELX + d];
     } else {
-      double U0[NF], W0[NF];
-      for (int k = 0; k < NF; k++) U0[k] = ntl(&SF(A.U, k, c, n));
-      to_primitive(U0, V, W0);
-      cfl_cell(W0);
-      v0[0] = W0[VELX];
-      v0[1] = W0[VELY];
-      v0[2] = W0[VELZ];
+      // Fluid::to_primitive's velocity
+      const double iM = 1.0 / ntl(&SF(A.U, MASS, c, n));
+      for (int d = 0; d < 3; d++) v0[d] = ntl(&SF(A.U, MOMX + d, c, n)) * iM;
     }
-    double arg_max = -1.0;  // min_j h/(cs + sqrt(a_j)) = h/(cs + sqrt(max_j a_j)), monotone roundings
-
-    T gx[NF], gy[NF], gz[NF], dmn[NF], dmx[NF], pU[NF], pgp[3], pdv;
-    double pdV = 0.0;
+    K1Sums<T> S;
+    T *gx = S.gx, *gy = S.gy, *gz = S.gz, *dmn = S.dmn, *dmx = S.dmx, *pU = S.pU, *pgp = S.pgp, *gw = S.gw;
+    T &pdv = S.pdv;
+    double &pdV = S.pdV, &arg_max = S.arg_max;
+    arg_max = -1.0;  // min_j h/(cs + sqrt(a_j)) = h/(cs + sqrt(max_j a_j)), monotone roundings
+    pdV = 0.0;
     for (int k = 0; k < NF; k++) gx[k] = gy[k] = gz[k] = dmn[k] = dmx[k] = pU[k] = T(0.0);
     pgp[0] = pgp[1] = pgp[2] = pdv = T(0.0);
-    T gw[3] = {T(0.0), T(0.0), T(0.0)};  // FP32 reconstruction: geometric weight of the own state
+    gw[0] = gw[1] = gw[2] = T(0.0);  // FP32 reconstruction: geometric weight of the own state
     // FP32: accumulators x[0,30) gradient sums, x[30,50) min/max, in LDS
     constexpr int K1NQ = LIMIT ? K1ACC : 8;
     if constexpr (std::is_same<T, float>::value) {
@@ -601,14 +791,7 @@ k_cfl_predict_recon(FusedArgs<T> A) {
         pdV += fe.isL ? (double)dV : -(double)dV;
       }
     }
-    // --- predictor cell update (computePredictor.cpp:141-379), FP64
-    T tv[NF];
-    {
-      double U0[NF], W0[NF];
-      for (int k = 0; k < NF; k++) U0[k] = ntl(&SF(A.U, k, c, n));
-      to_primitive(U0, V, W0);
-      if constexpr (std::is_same<T, float>::value) cfl_cell(W0);
-      if constexpr (std::is_same<T, float>::value) {
+    if constexpr (FP32) {
       __asm__ __volatile__("" ::: "memory");
       float x[4 * K1ACC];
       acc_ld<K1NQ>(k1_acc_slice(), x);
@@ -622,125 +805,180 @@ k_cfl_predict_recon(FusedArgs<T> A) {
         }
       }
     }
-    if (arg_max >= 0.0) dti = smin(dti, h / (csi + dsqrt(arg_max)));
-      dti = smin(dti, REF_HUGE);
-      dtn = dti * A.courant;
-      while (U0[MASS] + (double)pU[MASS] * dtn <= 0.0) dtn *= 0.5;
-      const double dt = rung_dt0(A.dtmax, dtn) / 128;
-      const double divB = (double)pdv;
-      double Uc[NF];
-      for (int k = 0; k < NF; k++) Uc[k] = U0[k] + (double)pU[k] * dt;
-      Uc[WBX] -= W0[VELX] * divB * dt;
-      Uc[WBY] -= W0[VELY] * divB * dt;
-      Uc[WBZ] -= W0[VELZ] * divB * dt;
-      const double pres = pressure(g64, W0[ETHM]);
-      const double B2 = W0[BX] * W0[BX] + W0[BY] * W0[BY] + W0[BZ] * W0[BZ];
-      const double dcs2 = g64 * pres + B2;
-      const double ch_sig = dsqrt(dcs2 / W0[DENS]);
-      Uc[WBX] -= (double)pgp[0] * dt;
-      Uc[WBY] -= (double)pgp[1] * dt;
-      Uc[WBZ] -= (double)pgp[2] * dt;
-      Uc[MPSI] -= dcs2 * divB * dt;
-      const double cr = 0.5;
-      const double l_min = A.lmin[c];
-      Uc[MPSI] *= exp(-cr * ch_sig / l_min * dt);
-      double W1[NF];
-      // exp(0) = 1 exactly: a static mesh skips the exponential
-      to_primitive(Uc, pdV == 0.0 ? V : V * exp(pdV * dt / V), W1);
-      const bool ef = W1[ETHM] <= 0.0;
-      if (ef) W1[ETHM] = ethm_from_entropy_d(g64, W1);
-      else W1[ENTR] = entropy_from_ethm_d(g64, W1);
-      if (!A.k1_pass) wave_count(&A.diag[FVM_DIAG_ETHM_FAILED], ef);  // a redo counts nothing twice
-      const double idt = 1.0 / dt;
-      for (int k = 0; k < NF; k++) tv[k] = (T)((W1[k] - W0[k]) * idt);
-    }
+    dtn = k1_finish<T, LIM, 1>(A, c, 0, e0, deg, V, Wc, pv, dt_step, S);
+  }
+  k1_minimum(A.dtmin_bits, dtn);
+}
 
-    // --- reconstruction finish (computeReconstruction.cpp:162-239)
-    {
-      const double invV = 1.0 / V;
-      if constexpr (std::is_same<T, float>::value)
-        for (int k = 0; k < NF; k++) {
-          gx[k] += gw[0] * Wc[k];
-          gy[k] += gw[1] * Wc[k];
-          gz[k] += gw[2] * Wc[k];
+// acc + a b: one rounding in FP32, the reference's two in FP64
+__device__ __forceinline__ float mul_acc(float a, float b, float acc) { return __builtin_fmaf(a, b, acc); }
+__device__ __forceinline__ double mul_acc(double a, double b, double acc) { return acc + a * b; }
+
+// the cell of a lane when four lanes work on each: 64 cells per block
+constexpr int QCELLS = FB / 4;
+__device__ __forceinline__ int quad_cell() {
+  const int per = (int)gridDim.x >> 3;
+  const int tile = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
+  return tile * QCELLS + ((int)threadIdx.x >> 2);
+}
+
+// Quad form of the predictor kernel.  A small mesh leaves most of the chip
+// without work at one lane per cell, and the launch is as long as one lane's
+// chain of face-ends.  Four lanes take four consecutive face-ends of the cell
+// at a time; the sums still run over the faces in order: after each round the
+// quad hands its four faces' terms round in turn, lane 0 to 2 summing the
+// gradient's x, y, z and lane 3 the predictor fluxes, so every sum has the bits
+// of the one-lane kernel.  32^3 cells, FP32, shipped limiter: 42 -> 25 us a
+// launch; what bounds it there is issue (two wavefronts a SIMD), below about
+// 16^3 the chain of the cell's own update after the faces.
+template <typename T, bool MOVING, int LIM>
+__global__ void __launch_bounds__(FB) k_cfl_predict_recon_quad(FusedArgs<T> A) {
+  constexpr bool LIMIT = LIM != LIM_SHIPPED;
+  constexpr bool FP32 = std::is_same<T, float>::value;
+  double dt_step = 0.0;
+  if (!k1_step_dt(A, dt_step)) return;  // uniform over the grid
+  const int c = quad_cell();
+  const int sub = (int)threadIdx.x & 3;
+  double dtn = REF_HUGE;
+  if (c < A.n) {
+    const int n = A.n;
+    const T g = (T)A.gamma;
+    const double V = ntl(A.cvol + c);
+    T Wc[NF];
+    ldv<NF>(A.wcur + (size_t)c * RWC, Wc);
+    double pv[3] = {0.0, 0.0, 0.0};
+    if constexpr (MOVING)
+      for (int d = 0; d < 3; d++) pv[d] = SF(A.mvel, d, c, n);
+    double v0[3];
+    if constexpr (FP32) {
+      for (int d = 0; d < 3; d++) v0[d] = (double)Wc[VELX + d];
+    } else {
+      const double iM = 1.0 / ntl(&SF(A.U, MASS, c, n));
+      for (int d = 0; d < 3; d++) v0[d] = ntl(&SF(A.U, MOMX + d, c, n)) * iM;
+    }
+    // the lane's sums: acc the gradient's component (lanes 0-2) or the fluxes
+    // (lane 3), geo the FP32 own-state weight (lanes 0-2) or div B (lane 3)
+    T acc[NF], mn[NF], mx[NF], geo = T(0.0), pg = T(0.0);
+    double arg_max = -1.0, pdV = 0.0;
+    for (int k = 0; k < NF; k++) acc[k] = mn[k] = mx[k] = T(0.0);
+
+    const int deg = A.deg[c];
+    const int e0 = A.gbase[c >> 6] + (c & 63);
+    // a lane past the last face repeats it: its terms are handed to nobody
+    FaceEndRec<T> rn;
+    if (deg > 0) rn = get_fe<MOVING, true>(A, e0 + 64 * min(sub, deg - 1));
+    for (int q0 = 0; q0 < deg; q0 += 4) {
+      const FaceEndRec<T> rc0 = rn;
+      if (q0 + 4 < deg) rn = get_fe<MOVING, true>(A, e0 + 64 * min(q0 + 4 + sub, deg - 1));
+      const int j = fe_nbr(rc0.nbr);
+      T Wj[NF];
+      ldv<NF>(A.wcur + (size_t)j * RWC, Wj);
+      FE<T> fe;
+      decode_fe(rc0, fe);
+      // reconstruction terms
+      const T dsh = fe.cen[0] * fe.ncen[0] + fe.cen[1] * fe.ncen[1] + fe.cen[2] * fe.ncen[2];
+      const T ids = (dsh != T(0.0)) ? fdiv(T(0.5), dsh) : T(0.0);
+      const T idsA = fe.area * ids;
+      T ra[3], rb[3];  // FP32: a, own-state weight; FP64: drh, fij
+      for (int d = 0; d < 3; d++) {
+        if constexpr (FP32) {
+          ra[d] = idsA * fe.cen[d];
+          rb[d] = T(2.0) * fe.ncen[d] * dsh - fe.cen[d];
+        } else {
+          ra[d] = fe.ncen[d] * dsh;
+          rb[d] = fe.cen[d] - ra[d];
         }
-      for (int k = 0; k < NF; k++) {
-        gx[k] = (T)((double)gx[k] * invV);
-        gy[k] = (T)((double)gy[k] * invV);
-        gz[k] = (T)((double)gz[k] * invV);
       }
-      if constexpr (LIMIT32) {
-        // FP32: the reconstruction and slope limiters in one pass over the
-        // own-side offsets, from the raw differences and the unlimited gradients
-        T gg[3 * NF];
+      if constexpr (LIMIT)
         for (int k = 0; k < NF; k++) {
-          gg[k] = gx[k];
-          gg[NF + k] = gy[k];
-          gg[2 * NF + k] = gz[k];
+          const T diff = Wj[k] - Wc[k];
+          mn[k] = smin(mn[k], diff);
+          mx[k] = smax(mx[k], diff);
         }
-        limit_cell32<LIM>(A, e0, deg, dmn, dmx, limiter_dtt(A.tdev[0], dt_step), tv, gg);
+      // CFL neighbour term (computeTimestep.cpp:37-54)
+      {
+        double dwi[3] = {0.0, 0.0, 0.0};
+        if constexpr (MOVING)
+          for (int d = 0; d < 3; d++) dwi[d] = (double)(T)SF(A.mvel, d, j, n) - pv[d];
+        const double dvi[3] = {(double)Wj[VELX] - v0[0], (double)Wj[VELY] - v0[1], (double)Wj[VELZ] - v0[2]};
+        const double a = (dwi[0] * dwi[0] + dwi[1] * dwi[1] + dwi[2] * dwi[2]) +
+                         1.0 * (dvi[0] * dvi[0] + dvi[1] * dvi[1] + dvi[2] * dvi[2]) + 1.0 / REF_HUGE;
+        arg_max = (arg_max < a) ? a : arg_max;
+      }
+      // predictor face flux, first order (computePredictor.cpp:44-136)
+      T flux[NF], psi, Bn, wij[3], dV;
+      {
+        const int L = fe.isL ? c : j, R = fe.isL ? j : c;
+        T WL[NF], WR[NF];
         for (int k = 0; k < NF; k++) {
-          gx[k] = gg[k];
-          gy[k] = gg[NF + k];
-          gz[k] = gg[2 * NF + k];
+          WL[k] = fe.isL ? Wc[k] : Wj[k];
+          WR[k] = fe.isL ? Wj[k] : Wc[k];
         }
-      } else if constexpr (LIMIT) {
-        // extremes of the limiter's argument over the faces, divided once a
-        // variable (64^3 cells: this kernel 487 -> 376 us)
-        T lm[NF], lo[NF], hi[NF];
-        for (int k = 0; k < NF; k++) lo[k] = hi[k] = T(0.0);
-        for (int q = 0, e = e0; q < deg; q++, e += 64) {
-          const double *cen = A.fep + FP_CEN * A.slots + e;
-          const T c0 = cen[0], c1 = cen[A.slots], c2 = cen[2 * A.slots];
+        face_velocity<T, MOVING>(A, L, R, fe, wij, dV);
+        compute_flux<T>(g, wij, WL, WR, NO_BOUNDARY, fe.nrm, psi, Bn, flux);
+      }
+      const T sa = fe.isL ? -fe.area : fe.area;
+      const T psa = psi * sa;
+      if (!fe.isL) dV = -dV;
+      // the round's faces in order
+      const auto take = [&](auto LN) {
+        constexpr int L = decltype(LN)::value;
+        if (q0 + L >= deg) return;  // the same for the four lanes
+        const T a0 = quad_get<L>(ra[0]), a1 = quad_get<L>(ra[1]), a2 = quad_get<L>(ra[2]);
+        const T b0 = quad_get<L>(rb[0]), b1 = quad_get<L>(rb[1]), b2 = quad_get<L>(rb[2]);
+        const T n0 = quad_get<L>(fe.nrm[0]), n1 = quad_get<L>(fe.nrm[1]), n2 = quad_get<L>(fe.nrm[2]);
+        const T sL = quad_get<L>(sa), iL = quad_get<L>(idsA), bL = quad_get<L>(Bn), pL = quad_get<L>(psa);
+        const T as = sub == 0 ? a0 : sub == 1 ? a1 : a2;
+        const T bs = sub == 0 ? b0 : sub == 1 ? b1 : b2;
+        const T ns = sub == 0 ? n0 : sub == 1 ? n1 : n2;
+        if constexpr (FP32) {
+          const T m = sub == 3 ? sL : as;
           for (int k = 0; k < NF; k++) {
-            const T d = gx[k] * c0 + gy[k] * c1 + gz[k] * c2;
-            lo[k] = __builtin_fmin(lo[k], d);
-            hi[k] = __builtin_fmax(hi[k], d);
+            const T w = quad_get<L>(Wj[k]), f = quad_get<L>(flux[k]);
+            acc[k] = mul_acc(sub == 3 ? f : w, m, acc[k]);
           }
+          geo = mul_acc(sub == 3 ? -bL : iL, sub == 3 ? sL : bs, geo);
+        } else {
+          for (int k = 0; k < NF; k++) {
+            const T w = quad_get<L>(Wj[k]), f = quad_get<L>(flux[k]);
+            const T sum = w + Wc[k];
+            const T diff = w - Wc[k];
+            const T x = sub == 3 ? f : sum * as + diff * bs;
+            acc[k] = acc[k] + x * (sub == 3 ? sL : iL);
+          }
+          geo = geo - bL * sL;  // used from lane 3
         }
-        for (int k = 0; k < NF; k++) lm[k] = limiter_of_extremes<false>(LIM, lo[k], hi[k], dmn[k], dmx[k]);
-        for (int k = 0; k < NF; k++) {
-          SF(A.mm, k, c, n) = dmn[k] + Wc[k];
-          SF(A.mm, NF + k, c, n) = dmx[k] + Wc[k];
-          tv[k] = tv[k] * lm[k];
-          gx[k] = gx[k] * lm[k];
-          gy[k] = gy[k] * lm[k];
-          gz[k] = gz[k] * lm[k];
-        }
-      }
-      if constexpr (FP32) {
-        // the record starts from the half-step state W + Wt dti of the step,
-        // formed as the flux kernel formed it; Wt goes to its own array
-        const float dti = (float)step_times_dt(A.tdev[0], dt_step).dti;
-        T wh[NF];
-        for (int k = 0; k < NF; k++) wh[k] = half_step32(Wc[k], tv[k], dti);
-        T *r = A.rec_w + (size_t)c * REC32;
-        stv<NF>(r, wh);
-        stv<NF>(r + R32_G, gx);
-        stv<NF>(r + R32_G + NF, gy);
-        stv<NF>(r + R32_G + 2 * NF, gz);
-        stv<NF>(A.tv + (size_t)c * NF, tv);
-      } else {
-        T *wc = A.rec_w + (size_t)c * REC;
-        stv<NF>(wc + R_T, tv);
-        stv<NF>(wc + R_G, gx);
-        stv<NF>(wc + R_G + NF, gy);
-        stv<NF>(wc + R_G + 2 * NF, gz);
+        pg = mul_acc(-ns, pL, pg);
+        if constexpr (MOVING) pdV += (double)quad_get<L>(dV);
+      };
+      take(std::integral_constant<int, 0>{});
+      take(std::integral_constant<int, 1>{});
+      take(std::integral_constant<int, 2>{});
+      take(std::integral_constant<int, 3>{});
+    }
+    K1Sums<T> S;
+    for (int k = 0; k < NF; k++) {
+      S.gx[k] = quad_get<0>(acc[k]);
+      S.gy[k] = quad_get<1>(acc[k]);
+      S.gz[k] = quad_get<2>(acc[k]);
+      S.pU[k] = quad_get<3>(acc[k]);
+      if constexpr (LIMIT) {
+        S.dmn[k] = quad_reduce(mn[k], [](T a, T b) { return smin(a, b); });
+        S.dmx[k] = quad_reduce(mx[k], [](T a, T b) { return smax(a, b); });
       }
     }
-    A.dt_new[c] = dtn;
+    S.gw[0] = quad_get<0>(geo);
+    S.gw[1] = quad_get<1>(geo);
+    S.gw[2] = quad_get<2>(geo);
+    S.pdv = quad_get<3>(geo);
+    S.pgp[0] = quad_get<0>(pg);
+    S.pgp[1] = quad_get<1>(pg);
+    S.pgp[2] = quad_get<2>(pg);
+    S.pdV = pdV;
+    S.arg_max = quad_reduce(arg_max, [](double a, double b) { return a < b ? b : a; });
+    dtn = k1_finish<T, LIM, 4>(A, c, sub, e0, deg, V, Wc, pv, dt_step, S);
   }
-  // global minimum of dt_new (dt > 0: IEEE bit patterns order like the values),
-  // one atomic per block
-  double v = dtn;
-  for (int o = 32; o > 0; o >>= 1) v = smin(v, __shfl_xor(v, o));
-  __shared__ double wmin[FB / 64];
-  if (__lane_id() == 0) wmin[threadIdx.x >> 6] = v;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < FB / 64; w++) v = smin(v, wmin[w]);
-    if (v < REF_HUGE && v >= 0.0) atomicMin(A.dtmin_bits, (unsigned long long)__double_as_longlong(v));
-  }
+  k1_minimum(A.dtmin_bits, dtn);
 }
 
 // ---------------------------------------------------------------------------
@@ -798,11 +1036,10 @@ __global__ void __launch_bounds__(FB) k_limit(FusedArgs<T> A) {
 // computePrimitives (FP64) for the own cell
 // ---------------------------------------------------------------------------
 // one face-end, given both extrapolated face states (Wo own side, Wn
-// neighbour side): HLLD in canonical orientation, FP64 sums of flux * dt * A
-// into the own cell (computeFluidUpdate.cpp:209-307)
+// neighbour side): HLLD in canonical orientation; sa is the signed dt * A
 template <typename T, bool MOVING>
-__device__ __forceinline__ void face_update(const FusedArgs<T> &A, int c, const FE<T> &fe, const T *Wn, const T *Wo,
-                                            double dtf, double *dU, double *gp, double &dv, int &nbad) {
+__device__ __forceinline__ void face_terms(const FusedArgs<T> &A, int c, const FE<T> &fe, const T *Wn, const T *Wo,
+                                           double dtf, T *flux, T &psi, T &Bn, double &sa, int &nbad) {
   T WL[NF], WR[NF];
   for (int k = 0; k < NF; k++) {
     WL[k] = fe.isL ? Wo[k] : Wn[k];
@@ -814,23 +1051,33 @@ __device__ __forceinline__ void face_update(const FusedArgs<T> &A, int c, const 
               ? 1 : 0;
   T wij[3], dV;
   face_velocity<T, MOVING>(A, fe.isL ? c : fe.j, fe.isL ? fe.j : c, fe, wij, dV);
-  T psi, Bn, flux[NF];
   compute_flux<T>((T)A.gamma, wij, WL, WR, NO_BOUNDARY, fe.nrm, psi, Bn, flux);
   // the L cell loses what flows L -> R: one signed area instead of two
   // branches (negation is exact, so the sums are those of the reference's
   // dU - F dt A and dU + F dt A)
   const double tarea = dtf * (double)fe.area;
-  const double sa = fe.isL ? -tarea : tarea;
+  sa = fe.isL ? -tarea : tarea;
+}
+
+// the same with its FP64 sums of flux * dt * A into the own cell
+// (computeFluidUpdate.cpp:209-307)
+template <typename T, bool MOVING>
+__device__ __forceinline__ void face_update(const FusedArgs<T> &A, int c, const FE<T> &fe, const T *Wn, const T *Wo,
+                                            double dtf, double *dU, double *gp, double &dv, int &nbad) {
+  T psi, Bn, flux[NF];
+  double sa;
+  face_terms<T, MOVING>(A, c, fe, Wn, Wo, dtf, flux, psi, Bn, sa, nbad);
   for (int k = 0; k < NF; k++) dU[k] = dU[k] + (double)flux[k] * sa;
   for (int d = 0; d < 3; d++) gp[d] = gp[d] - (double)fe.nrm[d] * ((double)psi * sa);
   dv = dv - (double)Bn * sa;
 }
 
 // computePrimitives at t1 = t0 + dt (computeFluidUpdate.cpp:367-505) for the
-// own cell, from the summed face terms
+// own cell, from the summed face terms; of several lanes on a cell the first
+// counts and stores
 template <typename T>
 __device__ __forceinline__ void cell_update(const FusedArgs<T> &A, int c, double t0, double dt_glob, const double *dU,
-                                            const double *gp, double dv, const T *tc) {
+                                            const double *gp, double dv, const T *tc, bool first = true) {
   const int n = A.n;
   const double g64 = A.gamma;
   const double t1 = t0 + dt_glob;
@@ -878,7 +1125,7 @@ __device__ __forceinline__ void cell_update(const FusedArgs<T> &A, int c, double
     const double cr = 0.5;
     const double l_min = A.lmin[c];
     Uc[MPSI] *= exp(-cr * ch_sig / l_min * dt);
-    to_primitive(Uc, V, W1);
+    to_primitive<sizeof(T) == 4>(Uc, V, W1);
     ef = W1[ETHM] <= 0.0;
     if (ef) W1[ETHM] = ethm_from_entropy_d(g64, W1);
     else W1[ENTR] = entropy_from_ethm_d(g64, W1);
@@ -890,9 +1137,13 @@ __device__ __forceinline__ void cell_update(const FusedArgs<T> &A, int c, double
     if (W1[ETHM] <= 0.0) W1[ETHM] = ethm_from_entropy_d(g64, W1);
     else W1[ENTR] = entropy_from_ethm_d(g64, W1);
   }
-  wave_count(&A.diag[FVM_DIAG_ETHM_FAILED], ef);
-  wave_count(&A.diag[FVM_DIAG_MASS_FAILED], failed);
+  wave_count(&A.diag[FVM_DIAG_ETHM_FAILED], ef && first);
+  wave_count(&A.diag[FVM_DIAG_MASS_FAILED], failed && first);
   to_conservative(W1, V, Ui);
+  // formed before the branch: a multiplication left behind by the additions
+  // that move past it would no longer fuse with them
+  for (int k = 0; k < NF; k++) keep_here(Ui[k]), keep_here(W1[k]);
+  if (!first) return;
   T Wn[NF];
   for (int k = 0; k < NF; k++) {
     if (sizeof(T) == 8 || A.write_w64) nts(W1[k], &SF(A.W64, k, c, n));
@@ -1191,6 +1442,79 @@ __global__ void __launch_bounds__(FB) k_flux_apply_coop(FusedArgs<float> A) {
   }
 }
 
+// Quad form of K2: four lanes take four consecutive face-ends of a cell at a
+// time (see the quad predictor kernel) and each sums all four faces' terms in
+// order; a lane past the last face repeats it.  32^3 cells, FP32: 36 -> 23 us a
+// launch.
+template <typename T, bool MOVING>
+__global__ void __launch_bounds__(FB) k_flux_apply_quad(FusedArgs<T> A) {
+  constexpr bool FP32 = std::is_same<T, float>::value;
+  const int c = quad_cell();
+  if (c >= A.n) return;
+  const int sub = (int)threadIdx.x & 3;
+  const StepTimes st = step_times(A);
+  const T dti = (T)st.dti;
+  const T *rc = A.rec + (size_t)c * rec_len<T>();
+  constexpr int G = FP32 ? R32_G : R_G;
+  T Wc[NF], tc[NF], gc[3 * NF];
+  ldv<NF>(rc, Wc);
+  if constexpr (!FP32) ldv<NF>(rc + R_T, tc);
+  ldv<3 * NF>(rc + G, gc);
+
+  double dU[NF], gp[3] = {0.0, 0.0, 0.0}, dv = 0.0;
+  for (int k = 0; k < NF; k++) dU[k] = 0.0;
+  int nbad = 0;
+  const int deg = A.deg[c];
+  const int e0 = A.gbase[c >> 6] + (c & 63);
+  FaceEndRec<T> rn;
+  if (deg > 0) rn = get_fe<true, false>(A, e0 + 64 * min(sub, deg - 1));
+  for (int q0 = 0; q0 < deg; q0 += 4) {
+    const FaceEndRec<T> rc0 = rn;
+    if (q0 + 4 < deg) rn = get_fe<true, false>(A, e0 + 64 * min(q0 + 4 + sub, deg - 1));
+    T Wn[NF], Wo[NF];
+    FE<T> fe;
+    {
+      const T *rj = A.rec + (size_t)fe_nbr(rc0.nbr) * rec_len<T>();
+      T Wj[NF], tj[NF], gj[3 * NF];
+      ldv<NF>(rj, Wj);
+      if constexpr (!FP32) ldv<NF>(rj + R_T, tj);
+      ldv<3 * NF>(rj + G, gj);
+      decode_fe(rc0, fe);
+      const T *drn = fe.isL ? fe.drR : fe.drL, *dro = fe.isL ? fe.drL : fe.drR;
+      for (int k = 0; k < NF; k++) {
+        if constexpr (FP32) {
+          Wn[k] = face_state32(Wj[k], gj[k], gj[NF + k], gj[2 * NF + k], drn);
+          Wo[k] = face_state32(Wc[k], gc[k], gc[NF + k], gc[2 * NF + k], dro);
+        } else {
+          Wn[k] = Wj[k] + (gj[k] * drn[0] + gj[NF + k] * drn[1] + gj[2 * NF + k] * drn[2] + tj[k] * dti);
+          Wo[k] = Wc[k] + (gc[k] * dro[0] + gc[NF + k] * dro[1] + gc[2 * NF + k] * dro[2] + tc[k] * dti);
+        }
+      }
+    }
+    T flux[NF], psi, Bn;
+    double sa;
+    int bad = 0;
+    face_terms<T, MOVING>(A, c, fe, Wn, Wo, st.dtf, flux, psi, Bn, sa, bad);
+    if (q0 + sub < deg) nbad += bad;
+    const double psa = (double)psi * sa;
+    const auto take = [&](auto LN) {
+      constexpr int L = decltype(LN)::value;
+      if (q0 + L >= deg) return;  // the same for the four lanes
+      const double sL = quad_get<L>(sa), pL = quad_get<L>(psa);
+      for (int k = 0; k < NF; k++) dU[k] = dU[k] + (double)quad_get<L>(flux[k]) * sL;
+      for (int d = 0; d < 3; d++) gp[d] = gp[d] - (double)quad_get<L>(fe.nrm[d]) * pL;
+      dv = dv - (double)quad_get<L>(Bn) * sL;
+    };
+    take(std::integral_constant<int, 0>{});
+    take(std::integral_constant<int, 1>{});
+    take(std::integral_constant<int, 2>{});
+    take(std::integral_constant<int, 3>{});
+  }
+  wave_add(&A.diag[FVM_DIAG_POSITIVITY], nbad);
+  if constexpr (FP32) ldv<NF>(A.tv + (size_t)c * NF, tc);
+  cell_update<T>(A, c, st.t0, st.dt_glob, dU, gp, dv, tc, sub == 0);
+}
+
 __global__ void k_advance(double *tdev, unsigned long long *dtmin_bits, double dtmax, double *hist, int step) {
   if (threadIdx.x == 0 && blockIdx.x == 0) {
     const double dt = rung_dt0(dtmax, __longlong_as_double((long long)*dtmin_bits));
@@ -1328,6 +1652,15 @@ unsigned fused_grid(int n) {
   unsigned nb = (unsigned)((n + FB - 1) / FB);
   return (nb + 7u) & ~7u;  // multiple of 8 for the XCD mapping
 }
+
+// Meshes up to this many cells run the quad kernels: as many as give each of the
+// chip's 1024 SIMDs three wavefronts of 16 cells in FP32, two in FP64 (whose
+// kernels keep one in flight).  Beyond, the quads' extra work costs more than
+// the shorter chain gives.  Ten steps of the vortex with the smooth limiter
+// (us, one lane / quad): FP32 20^3 959 / 524, 32^3 1168 / 864, 36^3 1263 / 1144,
+// 38^3 1281 / 1357, 48^3 1622 / 2065; FP64 20^3 1913 / 1042, 32^3 2205 / 1921,
+// 34^3 2242 / 2510, 48^3 4313 / 5417.
+template <typename T> constexpr int quad_cells() { return 16 * 1024 * (sizeof(T) == 4 ? 3 : 2); }
 
 template <typename T> FusedArgs<T> fused_args(fvm_ctx *c, double dtmax) {
   FusedState &z = c->fz;
@@ -1468,14 +1801,19 @@ template <typename T> int fused_setup_t(fvm_ctx *c) {
 int sg_step_launch(fvm_ctx *c, const FusedArgs<float> &A);
 
 template <typename T, bool MOVING, int LIM> int launch_step(fvm_ctx *c, const FusedArgs<T> &A, hipEvent_t *ev) {
-  const unsigned grid = fused_grid(c->np);
+  const bool quads = c->np <= quad_cells<T>();
+  const unsigned grid = fused_grid(c->np), qgrid = quads ? fused_grid(4 * c->np) : 0;
+  const auto k1 = [&](const FusedArgs<T> &a) {
+    if (quads) hipLaunchKernelGGL((k_cfl_predict_recon_quad<T, MOVING, LIM>), dim3(qgrid), dim3(FB), 0, c->stream, a);
+    else hipLaunchKernelGGL((k_cfl_predict_recon<T, MOVING, LIM>), dim3(grid), dim3(FB), 0, c->stream, a);
+  };
   if (ev) (void)hipEventRecord(ev[0], c->stream);
-  hipLaunchKernelGGL((k_cfl_predict_recon<T, MOVING, LIM>), dim3(grid), dim3(FB), 0, c->stream, A);
+  k1(A);
   if (ev) (void)hipEventRecord(ev[1], c->stream);
   if constexpr (std::is_same<T, float>::value) {
     FusedArgs<T> A2 = A;  // the check-and-redo pass of the step's dt
     A2.k1_pass = 1;
-    hipLaunchKernelGGL((k_cfl_predict_recon<T, MOVING, LIM>), dim3(grid), dim3(FB), 0, c->stream, A2);
+    k1(A2);
   } else if constexpr (LIM != LIM_SHIPPED) {
     hipLaunchKernelGGL((k_limit<T, LIM>), dim3(grid), dim3(FB), 0, c->stream, A);
   }
@@ -1489,11 +1827,15 @@ template <typename T, bool MOVING, int LIM> int launch_step(fvm_ctx *c, const Fu
         const int rc = sg_step_launch(c, A);
         if (rc) return rc;
       }
-    } else if (!addr64 && c->np <= (1 << 24))  // 24-bit record indices, < 2.7 GB of records
+    } else if (quads && !addr64)
+      hipLaunchKernelGGL((k_flux_apply_quad<T, MOVING>), dim3(qgrid), dim3(FB), 0, c->stream, A);
+    else if (!addr64 && c->np <= (1 << 24))  // 24-bit record indices, < 2.7 GB of records
       hipLaunchKernelGGL((k_flux_apply_coop<MOVING, true>), dim3(grid), dim3(FB), 0, c->stream, A);
     else
       hipLaunchKernelGGL((k_flux_apply_coop<MOVING, false>), dim3(grid), dim3(FB), 0, c->stream, A);
   }
+  else if (quads)
+    hipLaunchKernelGGL((k_flux_apply_quad<T, MOVING>), dim3(qgrid), dim3(FB), 0, c->stream, A);
   else
     hipLaunchKernelGGL((k_flux_apply<T, MOVING>), dim3(grid), dim3(FB), 0, c->stream, A);
   if (ev) (void)hipEventRecord(ev[3], c->stream);

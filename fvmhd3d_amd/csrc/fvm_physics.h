@@ -44,7 +44,11 @@ template <typename T> __device__ __forceinline__ T pressure(T gamma, T ethm) {
   return gamma > T(1.0) ? (gamma - T(1.0)) * ethm : ethm;
 }
 
-// Fluid::to_primitive (Fluid.h:61-98), total-energy form
+// Fluid::to_primitive (Fluid.h:61-98), total-energy form.  FUSE: the sums of
+// squares with their fused operations spelled out, for kernels compiled with
+// contraction that have to agree bit for bit: which product of a b + c d the
+// compiler fuses depends on the code around it.
+template <bool FUSE = false>
 __device__ __forceinline__ void to_primitive(const double *U, double volume, double *W) {
   const double iM = 1.0 / U[MASS];
   const double iV = 1.0 / volume;
@@ -57,8 +61,12 @@ __device__ __forceinline__ void to_primitive(const double *U, double volume, dou
   W[BZ] = U[WBZ] * iV;
   W[PSI] = U[MPSI] * iM;
   W[ENTR] = U[MENTR] * iM;
-  W[ETHM] = U[ENER] * iV - 0.5 * (sqr(W[BX]) + sqr(W[BY]) + sqr(W[BZ])) -
-            0.5 * (sqr(W[VELX]) + sqr(W[VELY]) + sqr(W[VELZ])) * W[DENS];
+  double B2 = sqr(W[BX]) + sqr(W[BY]) + sqr(W[BZ]), v2 = sqr(W[VELX]) + sqr(W[VELY]) + sqr(W[VELZ]);
+  if constexpr (FUSE) {
+    B2 = __builtin_fma(W[BZ], W[BZ], __builtin_fma(W[BX], W[BX], W[BY] * W[BY]));
+    v2 = __builtin_fma(W[VELZ], W[VELZ], __builtin_fma(W[VELX], W[VELX], W[VELY] * W[VELY]));
+  }
+  W[ETHM] = U[ENER] * iV - 0.5 * B2 - 0.5 * v2 * W[DENS];
 }
 
 // Fluid::to_conservative (Fluid.h:100-135)

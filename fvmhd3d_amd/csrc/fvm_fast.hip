@@ -63,7 +63,7 @@ int fvm_fused_run(fvm_ctx *c, int nsteps, double dtmax, double *t_out) {
   rc = z.precision == FVM_FUSED_FP64 ? fvm_fused_run_f64(c, nsteps, dtmax) : fvm_fused_run_f32(c, nsteps, dtmax);
   if (rc) return rc;
   double t2[2];
-  FVM_HIPCHK(c, hipMemcpyAsync(t2, z.tdev.p, sizeof t2, hipMemcpyDeviceToHost, c->stream));
+  FVM_HIPCHK(c, hipMemcpyAsync(t2, (const double *)z.tdev.p + 2 * z.cur, sizeof t2, hipMemcpyDeviceToHost, c->stream));
   FVM_HIPCHK(c, hipStreamSynchronize(c->stream));
   c->t_global = t2[0];
   if (t_out) *t_out = t2[0];

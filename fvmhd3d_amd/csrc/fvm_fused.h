@@ -14,7 +14,7 @@
 //        extrapolation + HLLD (computeFluidUpdate), FP64 sums of flux*dt*A in
 //        the cell's face order, then computePrimitives (FP64 pressure recovery,
 //        Dedner/Powell terms, fallbacks)
-//   K3 k_advance            t += dt, reset the CFL minimum
+//        and, by one lane, the next step's clock: t += dt, a fresh CFL minimum
 //
 // Each face is evaluated by both of its cells in the same canonical
 // orientation (L = s1, R = s2, normal L->R), so both see bit-identical fluxes:
@@ -140,8 +140,12 @@ template <typename T> struct FusedArgs {
   double *U;                // [10][n] FP64 conserved state (own cell only)
   T *mm;                    // [20][n] min/max (opt-in limiters)
   double *dt_new;           // [n]
-  unsigned long long *dtmin_bits;
-  double *tdev;             // [0] t_global, [1] dt of the last step
+  // the step's clock and the next one's (two, taken in turn): t_global and dt of
+  // the step before; the bits of the smallest dt_new
+  const double *tdev;
+  double *tdev_next;
+  unsigned long long *dtmin_bits, *dtmin_next;
+  double *hist;             // dt of this step goes here
   unsigned long long *diag;
   double gamma, courant, dtmax;
   int write_w64;            // FP32 path: store FP64 W (last step of a run)
@@ -457,6 +461,18 @@ __device__ __forceinline__ StepTimes step_times_dt(double t0, double dt_glob) {
 }
 template <typename T> __device__ __forceinline__ StepTimes step_times(const FusedArgs<T> &A) {
   return step_times_dt(A.tdev[0], rung_dt0(A.dtmax, __longlong_as_double((long long)*A.dtmin_bits)));
+}
+// The clock of the next step, by one lane of the step's last kernel, which alone
+// reads this step's (as a launch of its own: ten steps of 32^3 cells 737 us, now
+// 720).
+template <typename T> __device__ __forceinline__ void advance_clock(const FusedArgs<T> &A) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    const double dt = rung_dt0(A.dtmax, __longlong_as_double((long long)*A.dtmin_bits));
+    A.tdev_next[0] = A.tdev[0] + dt;
+    A.tdev_next[1] = dt;
+    *A.hist = dt;
+    *A.dtmin_next = 0x7FF0000000000000ULL;
+  }
 }
 // the half-step state W + Wt dti of one variable (FP32 path)
 __device__ __forceinline__ float half_step32(float W, float t, float dti) { return __builtin_fmaf(t, dti, W); }
@@ -1157,6 +1173,7 @@ __device__ __forceinline__ void cell_update(const FusedArgs<T> &A, int c, double
 // generic K2: each lane gathers its own neighbour records
 template <typename T, bool MOVING>
 __global__ void __launch_bounds__(FB) k_flux_apply(FusedArgs<T> A) {
+  advance_clock(A);
   const int c = xcd_cell(A.n);
   if (c >= A.n) return;
   const StepTimes st = step_times(A);
@@ -1312,6 +1329,7 @@ __device__ __forceinline__ FaceEndRec<float> fe_rec(const FeRaw &r) {
 template <bool MOVING, bool OFF32>
 __global__ void __launch_bounds__(FB) k_flux_apply_coop(FusedArgs<float> A) {
   using T = float;
+  advance_clock(A);
   __shared__ __attribute__((aligned(256))) float4 sbuf[FB / 64][2][GBUF];
   const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   float4 *buf0 = sbuf[wv][0], *buf1 = sbuf[wv][1];
@@ -1448,6 +1466,7 @@ __global__ void __launch_bounds__(FB) k_flux_apply_coop(FusedArgs<float> A) {
 // launch.
 template <typename T, bool MOVING>
 __global__ void __launch_bounds__(FB) k_flux_apply_quad(FusedArgs<T> A) {
+  advance_clock(A);
   constexpr bool FP32 = std::is_same<T, float>::value;
   const int c = quad_cell();
   if (c >= A.n) return;
@@ -1513,17 +1532,6 @@ __global__ void __launch_bounds__(FB) k_flux_apply_quad(FusedArgs<T> A) {
   wave_add(&A.diag[FVM_DIAG_POSITIVITY], nbad);
   if constexpr (FP32) ldv<NF>(A.tv + (size_t)c * NF, tc);
   cell_update<T>(A, c, st.t0, st.dt_glob, dU, gp, dv, tc, sub == 0);
-}
-
-__global__ void k_advance(double *tdev, unsigned long long *dtmin_bits, double dtmax, double *hist, int step) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    const double dt = rung_dt0(dtmax, __longlong_as_double((long long)*dtmin_bits));
-    const double t0 = tdev[0];
-    tdev[0] = t0 + dt;
-    tdev[1] = dt;
-    if (hist) hist[step] = dt;
-    *dtmin_bits = 0x7FF0000000000000ULL;
-  }
 }
 
 // face-end records from the uploaded mesh, in the internal cell order: internal
@@ -1686,8 +1694,11 @@ template <typename T> FusedArgs<T> fused_args(fvm_ctx *c, double dtmax) {
   A.U = (double *)z.U.p;
   A.mm = (T *)z.mm.p;
   A.dt_new = (double *)z.dt_new.p;
-  A.dtmin_bits = (unsigned long long *)z.dtmin.p;
-  A.tdev = (double *)z.tdev.p;
+  A.dtmin_bits = (unsigned long long *)z.dtmin.p + z.cur;
+  A.dtmin_next = (unsigned long long *)z.dtmin.p + (z.cur ^ 1);
+  A.tdev = (const double *)z.tdev.p + 2 * z.cur;
+  A.tdev_next = (double *)z.tdev.p + 2 * (z.cur ^ 1);
+  A.hist = (double *)z.hist.p;
   A.diag = (unsigned long long *)c->diag.p;
   A.gamma = c->prm.gamma_gas;
   A.courant = c->prm.courant_no;
@@ -1744,8 +1755,8 @@ template <typename T> int fused_setup_t(fvm_ctx *c) {
       (rc = fvm_ensure(c, z.rec[1], es * rec_len<T>() * (size_t)n)) ||
       (rc = fvm_ensure(c, z.tv, es * NF * (size_t)(es == 4 ? n : 1)))  /* FP32 path only */ || (rc = fvm_ensure(c, z.mm, es * 20 * (size_t)(es == 8 ? n : 1)))  /* FP64 path only */ ||
       (rc = fvm_ensure(c, z.wc[0], es * RWC * (size_t)n)) || (rc = fvm_ensure(c, z.wc[1], es * RWC * (size_t)n)) ||
-      (rc = fvm_ensure(c, z.dt_new, nd)) || (rc = fvm_ensure(c, z.dtmin, sizeof(unsigned long long))) ||
-      (rc = fvm_ensure(c, z.tdev, sizeof(double) * 2)))
+      (rc = fvm_ensure(c, z.dt_new, nd)) || (rc = fvm_ensure(c, z.dtmin, 2 * sizeof(unsigned long long))) ||
+      (rc = fvm_ensure(c, z.tdev, sizeof(double) * 4)))
     return rc;
   FVM_HIPCHK(c, hipMemcpy(z.gbase.p, gb.data(), sizeof(int) * (size_t)(ng + 1), hipMemcpyHostToDevice));
   FVM_HIPCHK(c, hipMemcpy(z.perm.p, perm.data(), ni, hipMemcpyHostToDevice));
@@ -1854,15 +1865,13 @@ template <typename T, bool MOVING> int fused_run_t(fvm_ctx *c, int nsteps, doubl
   for (int s = 0; s < nsteps; s++) {
     FusedArgs<T> A = fused_args<T>(c, dtmax);
     A.write_w64 = (s == nsteps - 1) ? 1 : 0;
+    A.hist += s;
     hipEvent_t *ev = z.timing ? &z.ev[5 * s] : nullptr;
     int rc;
     if (lim == LIM_MINMOD) rc = launch_step<T, MOVING, LIM_MINMOD>(c, A, ev);
     else if (lim == LIM_SMOOTH) rc = launch_step<T, MOVING, LIM_SMOOTH>(c, A, ev);
     else rc = launch_step<T, MOVING, LIM_SHIPPED>(c, A, ev);
     if (rc) return rc;
-    FVM_HIPCHK(c, hipGetLastError());
-    hipLaunchKernelGGL(k_advance, dim3(1), dim3(64), 0, c->stream, (double *)z.tdev.p, (unsigned long long *)z.dtmin.p,
-                       dtmax, (double *)z.hist.p, s);
     FVM_HIPCHK(c, hipGetLastError());
     if (ev) FVM_HIPCHK(c, hipEventRecord(ev[4], c->stream));
     z.cur ^= 1;

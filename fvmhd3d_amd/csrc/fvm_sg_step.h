@@ -232,6 +232,7 @@ __global__ void __launch_bounds__(SGB) k_sg_faces(FusedArgs<float> A, SgStepArgs
 // per cell: the FP64 sums of the face records in the cell's face order
 // (computeFluidUpdate.cpp:209-307), then computePrimitives
 __global__ void __launch_bounds__(FB) k_sg_cells(FusedArgs<float> A, SgStepArgs S) {
+  advance_clock(A);
   const int c = xcd_cell(A.n);
   if (c >= A.n) return;
   const StepTimes st = step_times(A);

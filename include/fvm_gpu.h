@@ -231,7 +231,7 @@ int fvm_fused_sync(fvm_ctx *ctx);
  * ms[0] CFL+predictor+reconstruction (FP32 path: with the opt-in limiters),
  * ms[1] FP32 path: the second launch that checks the limiters' dt and redoes
  *       the step when it changed; FP64 path: the limiter launch,
- * ms[2] flux+apply, ms[3] advance */
+ * ms[2] flux+apply (it also advances the clock), ms[3] what follows it, no launch */
 int fvm_fused_timing(fvm_ctx *ctx, int enable);
 int fvm_fused_kernel_ms(fvm_ctx *ctx, double *ms, long long *launches, int n);
 /* per-kernel HIP-event timing of the reference-order entry points (and so of

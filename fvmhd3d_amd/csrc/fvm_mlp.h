@@ -150,9 +150,12 @@ constexpr int P_BIAS = 3 * NH + 16;           // floats
 constexpr int P_BYTES = P_BF * 2 + P_BIAS * 4;
 __device__ __forceinline__ int kfeat(int c, int g, int e) { return 32 * c + (e < 4 ? 4 * g + e : 16 + 4 * g + e - 4); }
 
+// max(x, 0) with NaN to 0, as fmaxf, in one instruction where fmaxf takes two (it
+// first quiets x): 384 fewer a wavefront's 64 faces, of 2200.  The upper bound
+// rounds to infinity in bf16.
+__device__ __forceinline__ float relu(float x) { return __builtin_amdgcn_fmed3f(x, 0.0f, 3.4028234663852886e38f); }
 __device__ __forceinline__ bf16x4 relu_pack(f32x4 v) {
-  return bf16x4{(__bf16)fmaxf(v[0], 0.0f), (__bf16)fmaxf(v[1], 0.0f), (__bf16)fmaxf(v[2], 0.0f),
-                (__bf16)fmaxf(v[3], 0.0f)};
+  return bf16x4{(__bf16)relu(v[0]), (__bf16)relu(v[1]), (__bf16)relu(v[2]), (__bf16)relu(v[3])};
 }
 __device__ __forceinline__ bf16x8 cat(bf16x4 a, bf16x4 b) {
   return bf16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};

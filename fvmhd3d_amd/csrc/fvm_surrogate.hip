@@ -182,7 +182,8 @@ struct FaceCtx {
 };
 constexpr int CTX_B = 64 * (int)sizeof(FaceCtx);
 constexpr int WAVE_B = (FEAT_B > OUT_B ? FEAT_B : OUT_B) + CTX_B;
-constexpr int LDS_B = P_BYTES + (IB / 64) * WAVE_B;
+constexpr int REJ_N = 128;                     // rejected faces a wavefront gathers
+constexpr int LDS_B = P_BYTES + (IB / 64) * (WAVE_B + REJ_N * 4 + 8);
 static_assert(sizeof(FaceCtx) == 104, "FaceCtx layout");
 static_assert(LDS_B <= 160 * 1024, "LDS budget");
 
@@ -216,6 +217,13 @@ __global__ void k_pack(const float *P, __bf16 *frag, float *bias) {
 
 // MODE 0: computeFlux batch (features from the faces, gate, FP64 assembly,
 // fallback list); MODE 1: raw features x[n][16] -> y[n][8]
+// The rejected faces: each wavefront gathers its own in LDS and takes their place
+// in the list with one atomic addition per 128, what is left with one per block.
+// An addition per batch of 64 faces was the bound of the launch: at about 10 ns
+// each on one address, 156 of 181 us for 10^6 faces.  Now (10^6 faces, with the
+// fallback launch: 214 -> 130 us a call) it waits on its inputs, two wavefronts a
+// SIMD: no faster with a third (the network in two passes of 32 faces), nor with
+// inputs loaded in whole lines, with or without a batch's lead.
 template <int MODE>
 __global__ void __launch_bounds__(IB) k_infer(int n, double gamma, const double *__restrict__ wij,
                                               const double *__restrict__ Wi, const double *__restrict__ Wj,
@@ -240,6 +248,9 @@ __global__ void __launch_bounds__(IB) k_infer(int n, double gamma, const double 
   __bf16 *feat = reinterpret_cast<__bf16 *>(wb);
   float *out = reinterpret_cast<float *>(wb);
   FaceCtx *ctx = reinterpret_cast<FaceCtx *>(wb + (FEAT_B > OUT_B ? FEAT_B : OUT_B));
+  int *rejs = reinterpret_cast<int *>(smem + P_BYTES + (IB / 64) * WAVE_B) + wv * REJ_N;
+  unsigned long long *wrej = reinterpret_cast<unsigned long long *>(smem + P_BYTES + (IB / 64) * (WAVE_B + REJ_N * 4));
+  int nrej = 0;
   const int nbatch = (n + 63) / 64;
   const int wstride = gridDim.x * (IB / 64);
   for (int bw = blockIdx.x * (IB / 64) + wv; bw < nbatch; bw += wstride) {
@@ -326,29 +337,64 @@ __global__ void __launch_bounds__(IB) k_infer(int n, double gamma, const double 
         psi_out[f] = cx.psi;
         Bn_out[f] = cx.Bn;
       }
+      // rejected faces gather in the wavefront's list
       const bool rej = live && !ok;
       const unsigned long long m = __ballot(rej);
-      unsigned long long b0 = 0;
-      if (lane == 0 && m) b0 = atomicAdd(fb_count, (unsigned long long)__popcll(m));
-      b0 = __shfl(b0, 0);
-      if (rej) fb_list[b0 + (unsigned long long)__popcll(m & ((1ULL << lane) - 1ULL))] = f;
+      const int nr = __popcll(m);
+      if (nrej + nr > REJ_N) {
+        unsigned long long b0 = 0;
+        if (lane == 0) b0 = atomicAdd(fb_count, (unsigned long long)nrej);
+        b0 = __shfl(b0, 0);
+        for (int i = lane; i < nrej; i += 64) fb_list[b0 + i] = rejs[i];
+        nrej = 0;
+        wave_sync();
+      }
+      if (rej) rejs[nrej + __popcll(m & ((1ULL << lane) - 1ULL))] = f;
+      nrej += nr;
+      wave_sync();
     }
+  }
+  if constexpr (MODE == 0) {
+    // what is left, with one addition to the count for the block
+    if (lane == 0) wrej[wv] = (unsigned long long)nrej;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      unsigned long long t = 0;
+      for (int w = 0; w < IB / 64; w++) t += wrej[w];
+      unsigned long long b0 = t ? atomicAdd(fb_count, t) : 0;
+      for (int w = 0; w < IB / 64; w++) {
+        const unsigned long long k = wrej[w];
+        wrej[w] = b0;
+        b0 += k;
+      }
+    }
+    __syncthreads();
+    for (int i = lane; i < nrej; i += 64) fb_list[wrej[wv] + i] = rejs[i];
   }
 }
 
-// FP64 computeFlux on the rejected faces
-__global__ void __launch_bounds__(256) k_fallback(const int *list, const unsigned long long *count, double gamma, const double *wij,
-                           const double *Wi, const double *Wj, const int *jbnd, const double *nrm, double *psi,
-                           double *Bn, double *flux) {
-  const int i = gid();
-  if ((unsigned long long)i >= *count) return;
-  const int f = list[i];
-  double w3[3], L[NF], R[NF], n3[3], F[NF], p, b;
-  load_face(f, wij, Wi, Wj, nrm, w3, L, R, n3);
-  compute_flux<double>(gamma, w3, L, R, jbnd[f], n3, p, b, F);
-  psi[f] = p;
-  Bn[f] = b;
-  for (int k = 0; k < NF; k++) flux[(size_t)NF * f + k] = F[k];
+// FP64 computeFlux on the rejected faces; passes their number on to the host and
+// clears the counter of the next call, so that a call makes two launches and no
+// copy (1000 faces: 44 -> 32 us a call)
+__global__ void __launch_bounds__(256) k_fallback(const int *list, const unsigned long long *count,
+                                                  unsigned long long *next, unsigned long long *host, double gamma,
+                                                  const double *wij, const double *Wi, const double *Wj,
+                                                  const int *jbnd, const double *nrm, double *psi, double *Bn,
+                                                  double *flux) {
+  const unsigned long long nf = *count;
+  if (gid() == 0) {
+    *next = 0;
+    *host = nf;
+  }
+  for (unsigned long long i = (unsigned long long)gid(); i < nf; i += (unsigned long long)gridDim.x * blockDim.x) {
+    const int f = list[i];
+    double w3[3], L[NF], R[NF], n3[3], F[NF], p, b;
+    load_face(f, wij, Wi, Wj, nrm, w3, L, R, n3);
+    compute_flux<double>(gamma, w3, L, R, jbnd[f], n3, p, b, F);
+    psi[f] = p;
+    Bn[f] = b;
+    for (int k = 0; k < NF; k++) flux[(size_t)NF * f + k] = F[k];
+  }
 }
 
 // computeFlux on every face in precision T (the comparison kernels)
@@ -400,6 +446,8 @@ struct fvm_sg {
   Buf xb, tb, y, loss;     // fvm_sg_gradients' batch and outputs; the steps' losses
   Buf tfrag, tops, tcols, tloss;  // training: packed weights; the tiles' operands, FP32 gradients and losses
   Buf stage, fbl, fbc;
+  unsigned long long *nfb = nullptr;  // pinned: rejected faces of the last batch
+  int fslot = -1;                     // the counter in turn (of the two of fbc); -1: neither is clear
   Buf sx, st, sflag, spos;  // sample staging of one add_faces call
   fvm::ScanScratch scan;
   int adam_t = 0;
@@ -488,9 +536,11 @@ static int pack(fvm_sg *s) {
   return FVM_OK;
 }
 
+// one block a CU, all resident: the weights are loaded once (over 1024 blocks:
+// 10^6 faces 15 us more)
 static unsigned infer_grid(int n) {
   const unsigned nb = (unsigned)(((long long)n + IB - 1) / IB);
-  return std::max(1u, std::min(nb, 256u * 4u));
+  return std::max(1u, std::min(nb, 256u));
 }
 
 template <int MODE>
@@ -506,6 +556,26 @@ static int launch_infer(fvm_sg *s, int n, const double *wij, const double *Wi, c
                      nrm, (const __bf16 *)s->pfrag.p, (const float *)s->pbias.p, s->gate, psi, Bn, flux, fbl, fbc,
                      xin, yout);
   SGCHK(s, hipGetLastError());
+  return FVM_OK;
+}
+
+// surrogate fluxes of a batch and the FP64 fluxes of the faces it rejects
+static int launch_flux(fvm_sg *s, int n, const double *wij, const double *Wi, const double *Wj, const int *jbnd,
+                       const double *nrm, double *psi, double *Bn, double *flux) {
+  int rc;
+  if ((rc = sg_ensure(s, s->fbl, sizeof(int) * (size_t)n)) ||
+      (rc = sg_ensure(s, s->fbc, 2 * sizeof(unsigned long long))))
+    return rc;
+  unsigned long long *cnt = (unsigned long long *)s->fbc.p;
+  if (s->fslot < 0) SGCHK(s, hipMemsetAsync(cnt, 0, 2 * sizeof(unsigned long long), s->stream));
+  const int slot = s->fslot < 0 ? 0 : s->fslot;
+  s->fslot = -1;  // until both launches are made
+  if ((rc = launch_infer<0>(s, n, wij, Wi, Wj, jbnd, nrm, psi, Bn, flux, (int *)s->fbl.p, cnt + slot, nullptr, nullptr)))
+    return rc;
+  hipLaunchKernelGGL(k_fallback, dim3(std::min(nblk(n), 1024u)), dim3(256), 0, s->stream, (const int *)s->fbl.p,
+                     cnt + slot, cnt + (slot ^ 1), s->nfb, s->gamma, wij, Wi, Wj, jbnd, nrm, psi, Bn, flux);
+  SGCHK(s, hipGetLastError());
+  s->fslot = slot ^ 1;
   return FVM_OK;
 }
 
@@ -543,7 +613,8 @@ int fvm_sg_create(fvm_sg **out, int device, double gamma_gas) {
     return FVM_EHIP;
   }
   if (sg_ensure(s, s->params, 4 * NPARAM) || sg_ensure(s, s->grads, 4 * NPARAM) || sg_ensure(s, s->am, 4 * NPARAM) ||
-      sg_ensure(s, s->av, 4 * NPARAM)) {
+      sg_ensure(s, s->av, 4 * NPARAM) ||
+      hipHostMalloc((void **)&s->nfb, sizeof(unsigned long long), hipHostMallocDefault) != hipSuccess) {
     fvm_sg_destroy(s);
     return FVM_EHIP;
   }
@@ -561,6 +632,7 @@ void fvm_sg_destroy(fvm_sg *s) {
                  &s->loss, &s->tfrag, &s->tops, &s->tcols, &s->tloss, &s->stage, &s->fbl, &s->fbc,
                  &s->sx, &s->st, &s->sflag, &s->spos})
     sg_release(*b);
+  if (s->nfb) (void)hipHostFree(s->nfb);
   fvm::scan_release(s->scan);
   if (s->stream) (void)hipStreamDestroy(s->stream);
   delete s;
@@ -776,20 +848,9 @@ int fvm_sg_compute_flux_device(fvm_sg *s, int n, const double *wij, const double
     return sg_fail(s, FVM_EARG, "compute_flux: NULL array");
   (void)hipSetDevice(s->device);
   int rc;
-  if ((rc = pack(s)) || (rc = sg_ensure(s, s->fbl, sizeof(int) * (size_t)n)) ||
-      (rc = sg_ensure(s, s->fbc, sizeof(unsigned long long))))
-    return rc;
-  unsigned long long *cnt = (unsigned long long *)s->fbc.p;
-  SGCHK(s, hipMemsetAsync(cnt, 0, sizeof(unsigned long long), s->stream));
-  if ((rc = launch_infer<0>(s, n, wij, Wi, Wj, jbnd, normal, psi, Bn, flux, (int *)s->fbl.p, cnt, nullptr, nullptr)))
-    return rc;
-  hipLaunchKernelGGL(k_fallback, dim3(nblk(n)), dim3(256), 0, s->stream, (const int *)s->fbl.p, cnt, s->gamma, wij, Wi,
-                     Wj, jbnd, normal, psi, Bn, flux);
-  SGCHK(s, hipGetLastError());
-  unsigned long long nf = 0;
-  SGCHK(s, hipMemcpyAsync(&nf, cnt, sizeof nf, hipMemcpyDeviceToHost, s->stream));
+  if ((rc = pack(s)) || (rc = launch_flux(s, n, wij, Wi, Wj, jbnd, normal, psi, Bn, flux))) return rc;
   SGCHK(s, hipStreamSynchronize(s->stream));
-  if (n_fallback) *n_fallback = (int)nf;
+  if (n_fallback) *n_fallback = (int)*s->nfb;
   return FVM_OK;
 }
 
@@ -827,16 +888,9 @@ int fvm_sg_time_flux(fvm_sg *s, int n, const double *wij, const double *Wi, cons
   if ((rc = fvm_sg_compute_flux_device(s, n, d[0], d[1], d[2], jb, d[3], d[4], d[5], d[6], n_fallback))) return rc;
   hipEvent_t e[4];
   for (auto &x : e) SGCHK(s, hipEventCreate(&x));
-  unsigned long long *cnt = (unsigned long long *)s->fbc.p;
   SGCHK(s, hipEventRecord(e[0], s->stream));
-  for (int k = 0; k < iters; k++) {
-    SGCHK(s, hipMemsetAsync(cnt, 0, sizeof(unsigned long long), s->stream));
-    if ((rc = launch_infer<0>(s, n, d[0], d[1], d[2], jb, d[3], d[4], d[5], d[6], (int *)s->fbl.p, cnt, nullptr,
-                              nullptr)))
-      return rc;
-    hipLaunchKernelGGL(k_fallback, dim3(nblk(n)), dim3(256), 0, s->stream, (const int *)s->fbl.p, cnt, s->gamma, d[0],
-                       d[1], d[2], jb, d[3], d[4], d[5], d[6]);
-  }
+  for (int k = 0; k < iters; k++)
+    if ((rc = launch_flux(s, n, d[0], d[1], d[2], jb, d[3], d[4], d[5], d[6]))) return rc;
   SGCHK(s, hipEventRecord(e[1], s->stream));
   for (int k = 0; k < iters; k++)
     hipLaunchKernelGGL(k_hlld<double>, dim3(nblk(n)), dim3(256), 0, s->stream, n, s->gamma, d[0], d[1], d[2], jb, d[3],

@@ -342,6 +342,28 @@ def test_gpu_fallback_is_fp64_compute_flux():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [9, 64, 513, 400_001])
+def test_gpu_rejected_faces_over_batches(n):
+    """No, some and every face rejected, call after call: each wavefront's list of rejected faces (128 long) stays
+    empty, is left over at its end, or overflows (over 2 x 131072 faces); the FP64 flux of each is exact."""
+    from fvmhd3d_amd import gpu as G
+    from fvmhd3d_amd.surrogate import Surrogate
+    wij, Wi, Wj, _, nrm = _random_faces(n)
+    every, some, none = np.full(n, G.REFLECTING, np.int32), np.zeros(n, np.int32), np.zeros(n, np.int32)
+    some[::3] = G.REFLECTING
+    ctx = G.Context()
+    sg = Surrogate(gate=(1e30, 1e30, 1e30, 1e30))  # boundary faces alone fall back
+    for jb in (none, every, some, every, none):
+        psi, Bn, F = ctx.compute_flux(wij, Wi, Wj, jb, nrm)
+        psi2, Bn2, F2, nfb = sg.compute_flux(wij, Wi, Wj, jb, nrm)
+        rej = jb != 0
+        assert nfb == rej.sum()
+        assert np.array_equal(psi[rej], psi2[rej]) and np.array_equal(Bn[rej], Bn2[rej]) and np.array_equal(F[rej], F2[rej])
+    sg.close()
+    ctx.close()
+
+
+@pytest.mark.gpu
 def test_gpu_training_lowers_loss_and_gates_accuracy():
     """Train on harvested blast faces, evaluate on a held-out harvest: the loss
     falls by 10x and the faces the gate accepts are within 2e-2 of the FP64 HLLD

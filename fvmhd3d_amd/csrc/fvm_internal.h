@@ -137,6 +137,7 @@ struct fvm_ctx {
   // the global lists (sub.goff, gface, fpos, fmark)
   bool sub_layout = false;
   DBuf rec, tmp0, tmp1, tmp2, stage;
+  DBuf crow;  // cell rows of the face kernels
   DBuf diag;     // unsigned long long[FVM_NDIAG]
   DBuf scalars;  // unsigned long long[8]
   fvm::ScanScratch scan;
@@ -156,6 +157,8 @@ struct fvm_ctx {
 
 int fvm_fail(fvm_ctx *c, int code, const std::string &msg);
 int fvm_ensure(fvm_ctx *c, DBuf &b, size_t bytes);
+// room for the cell rows of nfa active faces, or false: too few faces, or no memory
+bool fvm_cell_row_space(fvm_ctx *c, int np, int nfa);
 void fvm_release(DBuf &b);
 
 // host transfers (fvm_xfer.hip)

@@ -423,23 +423,28 @@ __global__ void k_sub_order_keys(const int *__restrict__ perm, int nA, const int
   key[k] = order_key(rung[g], seq[g], base);
 }
 
-// The same order for a short list, by ranks: 16 lanes count the keys below one
-// cell's (keys are distinct: the stamps are); the list in that order and each
-// cell's place in it.  4096 keys are 16.8 M comparisons over the whole chip:
-// 28 us on average on a 14,000-cell mesh, against 48 us for the 78 block-wide
-// steps of a sort in one workgroup.
+// The same order for a short list, by ranks: a wavefront counts the keys below
+// one cell's (keys are distinct: the stamps are), four loads in flight; the list
+// in that order and each cell's place in it.  Each trip round the loop costs a
+// load's latency: 2100 keys with 16 lanes a key and one load 32 us, now 5.5.
+// (Bounded to 4096 keys, 16.8 M comparisons; a sort in one workgroup took 48 us.)
 constexpr int kSmallSort = 4096;
 __global__ void k_sub_rank_sort(const int *__restrict__ perm, const unsigned long long *__restrict__ key, int nA,
                                 int *__restrict__ out, int *__restrict__ apos) {
   const int t = gidx();
-  const int i = t / kLanes;
+  const int i = t >> 6, l = t & 63;
+  if (i >= nA) return;  // whole wavefronts
+  const unsigned long long mine = key[i];
   int below = 0;
-  if (i < nA) {
-    const unsigned long long mine = key[i];
-    for (int m = t & (kLanes - 1); m < nA; m += kLanes) below += key[m] < mine ? 1 : 0;
+  for (int m0 = 0; m0 < nA; m0 += 256) {
+    unsigned long long k[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) k[u] = key[min(m0 + 64 * u + l, nA - 1)];
+#pragma unroll
+    for (int u = 0; u < 4; u++) below += m0 + 64 * u + l < nA && k[u] < mine ? 1 : 0;
   }
-  for (int o = kLanes / 2; o > 0; o >>= 1) below += __shfl_xor(below, o);
-  if (i < nA && (t & (kLanes - 1)) == 0) {
+  for (int o = 32; o > 0; o >>= 1) below += __shfl_xor(below, o);
+  if (l == 0) {
     const int g = perm[i];
     out[below] = g;
     apos[g] = below;
@@ -595,7 +600,7 @@ int build_layout(fvm_ctx *c, unsigned mask, double t_global, int check, int *cou
     SLAUNCH(c, nA, k_sub_order_keys, P<int>(s.perm), nA, P<int>(s.rung), P<unsigned long long>(s.seq), base,
             P<unsigned long long>(s.okey));
     if (nA <= kSmallSort) {
-      SLAUNCH(c, (long long)nA * kLanes, k_sub_rank_sort, P<int>(s.perm), P<unsigned long long>(s.okey), nA, P<int>(s.oval2),
+      SLAUNCH(c, 64LL * nA, k_sub_rank_sort, P<int>(s.perm), P<unsigned long long>(s.okey), nA, P<int>(s.oval2),
               P<int>(s.apos));
     } else {
       size_t tb = s.otmp_bytes;

@@ -3,7 +3,7 @@
 // buffers.
 //
 // Device layout: every per-cell field is structure-of-arrays, component k of
-// cell i at [k*np + i]; face records likewise [k*nface_act + a].  Fields the
+// cell i at [k*np + i]; per-face records and geometry are rows.  Fields the
 // reference stores as float (Fluid_flt, fvec3, FluidD) use the storage type S
 // (float as shipped, double for the all-FP64 build); everything else is double.
 //

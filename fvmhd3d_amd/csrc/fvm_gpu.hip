@@ -1065,6 +1065,53 @@ __global__ void __launch_bounds__(256) k_flux_batch(int n, double gamma, const d
   for (int k = 0; k < NF; k++) flux[(size_t)NF * f + k] = F[k];
 }
 
+// The same on a small batch in pinned host memory: in wij[n][3], Wi[n][10],
+// Wj[n][10], normal[n][3], jbnd; out psi[n], B_n[n], flux[n][10].  A wavefront reads
+// and writes its 64 faces' rows over the link in whole lines, all in flight,
+// through LDS; one launch in place of two copies in, a launch and a copy out, each
+// a few microseconds after the other (2048 faces: 64 -> 43 us a call).
+__global__ void __launch_bounds__(64) k_flux_pinned(int n, double gamma, const double *in, const int *jbnd, double *out) {
+  constexpr int W = 26;
+  __shared__ double tile[64 * W];
+  const int l = (int)threadIdx.x, f0 = (int)blockIdx.x * 64, m = min(64, n - f0);
+  const int width[4] = {3, NF, NF, 3};
+  {
+    double v[W];
+    int off = 0;
+#pragma unroll
+    for (int a = 0; a < 4; a++) {
+      const double *p = in + (size_t)off * n + (size_t)width[a] * f0;
+#pragma unroll
+      for (int u = 0; u < width[a]; u++) v[off + u] = 64 * u + l < width[a] * m ? p[64 * u + l] : 0.0;
+      off += width[a];
+    }
+#pragma unroll
+    for (int u = 0; u < W; u++) tile[64 * u + l] = v[u];
+  }
+  const int jb = l < m ? jbnd[f0 + l] : NO_BOUNDARY;
+  __syncthreads();
+  double w3[3], n3[3], L[NF], R[NF], F[NF], p, b;
+  for (int d = 0; d < 3; d++) {
+    w3[d] = tile[3 * l + d];
+    n3[d] = tile[64 * 23 + 3 * l + d];
+  }
+  for (int k = 0; k < NF; k++) {
+    L[k] = tile[64 * 3 + NF * l + k];
+    R[k] = tile[64 * 13 + NF * l + k];
+  }
+  __syncthreads();
+  if (l < m) {
+    compute_flux<double>(gamma, w3, L, R, jb, n3, p, b, F);
+    out[f0 + l] = p;
+    out[n + f0 + l] = b;
+    for (int k = 0; k < NF; k++) tile[NF * l + k] = F[k];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < NF; u++)
+    if (64 * u + l < NF * m) out[2 * (size_t)n + (size_t)NF * f0 + 64 * u + l] = tile[64 * u + l];
+}
+
 // ---------------------------------------------------------------------------
 // get_active_faces (Iterate.cpp:298-324) and the per-cell face-end lists
 // ---------------------------------------------------------------------------
@@ -2179,32 +2226,57 @@ struct FluxBatch {
 constexpr size_t FLUX_IN_D = 26, FLUX_OUT_D = 12;  // doubles in and out per face, and one int in
 static_assert(FVM_FLUX_BYTES_PER_FACE == 8 * (FLUX_IN_D + FLUX_OUT_D) + 4, "face bytes");
 
+// in and out of the staging: [n] faces' inputs, outputs, boundary kinds
+struct FluxStage {
+  double *in, *out;
+  int *jb;
+};
+FluxStage flux_stage(char *h, size_t n) {
+  double *in = (double *)h, *out = in + FLUX_IN_D * n;
+  return {in, out, (int *)(out + FLUX_OUT_D * n)};
+}
+void flux_stage_in(const FluxBatch &b, size_t f0, size_t n, const FluxStage &s) {
+  std::memcpy(s.in, b.wij + 3 * f0, 24 * n);
+  std::memcpy(s.in + 3 * n, b.Wi + 10 * f0, 80 * n);
+  std::memcpy(s.in + 13 * n, b.Wj + 10 * f0, 80 * n);
+  std::memcpy(s.in + 23 * n, b.normal + 3 * f0, 24 * n);
+  std::memcpy(s.jb, b.jbnd + f0, 4 * n);
+}
+void flux_stage_out(const FluxBatch &b, size_t f0, size_t n, const FluxStage &s) {
+  std::memcpy(b.psi + f0, s.out, 8 * n);
+  std::memcpy(b.Bn + f0, s.out + n, 8 * n);
+  std::memcpy(b.flux + 10 * f0, s.out + 2 * n, 80 * n);
+}
+
 hipError_t flux_chunk(double gamma, const FluxBatch &b, size_t f0, size_t n, char *h, char *d, hipStream_t st) {
-  double *hw = (double *)h, *hi = hw + 3 * n, *hj = hi + 10 * n, *hn = hj + 10 * n, *ho = hn + 3 * n;
-  int *hb = (int *)(ho + FLUX_OUT_D * n);
-  double *dw = (double *)d, *di = dw + 3 * n, *dj = di + 10 * n, *dn = dj + 10 * n, *dpsi = dn + 3 * n, *dBn = dpsi + n,
-         *dfl = dBn + n;
-  int *db = (int *)(dfl + 10 * n);
-  std::memcpy(hw, b.wij + 3 * f0, 24 * n);
-  std::memcpy(hi, b.Wi + 10 * f0, 80 * n);
-  std::memcpy(hj, b.Wj + 10 * f0, 80 * n);
-  std::memcpy(hn, b.normal + 3 * f0, 24 * n);
-  std::memcpy(hb, b.jbnd + f0, 4 * n);
-  hipError_t e = hipMemcpyAsync(d, h, 8 * FLUX_IN_D * n, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(db, hb, 4 * n, hipMemcpyHostToDevice, st);
+  const FluxStage H = flux_stage(h, n), D = flux_stage(d, n);
+  flux_stage_in(b, f0, n, H);
+  hipError_t e = hipMemcpyAsync(D.in, H.in, 8 * FLUX_IN_D * n, hipMemcpyHostToDevice, st);
+  if (e == hipSuccess) e = hipMemcpyAsync(D.jb, H.jb, 4 * n, hipMemcpyHostToDevice, st);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(fvm::k_flux_batch, dim3(nblk((long)n)), dim3(256), 0, st, (int)n, gamma, dw, di, dj, db, dn, dpsi, dBn, dfl);
+  hipLaunchKernelGGL(fvm::k_flux_batch, dim3(nblk((long)n)), dim3(256), 0, st, (int)n, gamma, D.in, D.in + 3 * n, D.in + 13 * n,
+                     D.jb, D.in + 23 * n, D.out, D.out + n, D.out + 2 * n);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  e = hipMemcpyAsync(ho, dpsi, 8 * FLUX_OUT_D * n, hipMemcpyDeviceToHost, st);
+  e = hipMemcpyAsync(H.out, D.out, 8 * FLUX_OUT_D * n, hipMemcpyDeviceToHost, st);
   if (e == hipSuccess) e = hipStreamSynchronize(st);
   if (e != hipSuccess) return e;
-  std::memcpy(b.psi + f0, ho, 8 * n);
-  std::memcpy(b.Bn + f0, ho + n, 8 * n);
-  std::memcpy(b.flux + 10 * f0, ho + 2 * n, 80 * n);
+  flux_stage_out(b, f0, n, H);
+  return hipSuccess;
+}
+
+// a small batch computed where it lies in pinned memory (h)
+hipError_t flux_pinned(double gamma, const FluxBatch &b, size_t n, char *h, hipStream_t st) {
+  const FluxStage H = flux_stage(h, n);
+  flux_stage_in(b, 0, n, H);
+  hipLaunchKernelGGL(fvm::k_flux_pinned, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, st, (int)n, gamma, H.in, H.jb, H.out);
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess) e = hipStreamSynchronize(st);
+  if (e != hipSuccess) return e;
+  flux_stage_out(b, 0, n, H);
   return hipSuccess;
 }
 }  // namespace
-// faces of a small batch (the context's pinned staging, 1 MiB) and of a chunk of
+// faces of a small batch (the context's pinned staging, 1 MiB: 3400 faces) and of a chunk of
 // a large one (a transfer slot); batches from two chunks up go chunk by chunk
 // over the transfer threads, uploads, kernels and downloads overlapping
 constexpr int FLUX_PIN = (1 << 20) / FVM_FLUX_BYTES_PER_FACE;
@@ -2219,7 +2291,7 @@ static int flux_batch_staged(fvm_ctx *c, char *base, bool threads, int n, const 
   const size_t N = (size_t)n;
   const FluxBatch b{wij, Wi, Wj, jbnd, normal, psi, Bn, flux};
   if (n <= FLUX_PIN && c->pin) {
-    HIPCHK(c, flux_chunk(c->prm.gamma_gas, b, 0, N, c->pin, base, c->stream));
+    HIPCHK(c, flux_pinned(c->prm.gamma_gas, b, N, c->pin, c->stream));
     return FVM_OK;
   }
   if (threads && n >= 2 * FLUX_CHUNK) {

@@ -145,6 +145,7 @@ struct fvm_ctx {
   SubstepState sub;
   hipStream_t xstream[fvm::kXferThreads - 1] = {};  // of the transfer threads (created on first use)
   char *pin = nullptr;  // pinned staging of small computeFlux batches
+  hipEvent_t pin_ev[2] = {nullptr, nullptr};  // a piece of a batch in each half of pin is done
   // HIP-event timing of the reference-order kernels (fvm_kernel_timing): per
   // kernel FVM_KT_*, total milliseconds and launches since timing was enabled
   struct {

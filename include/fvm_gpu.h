@@ -173,7 +173,8 @@ int fvm_compute_flux(fvm_ctx *ctx, int n, const double *wij, const double *Wi, c
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
  * Same arguments and results as fvm_compute_flux; the device staging is a
  * fixed array of FVM_FLUX_NOALLOC_BYTES in the library, one per GPU, held
- * until the process ends.  n > FVM_FLUX_NOALLOC_MAX is refused with FVM_EARG.
+ * until the process ends (up to 3404 faces: the context's pinned host staging,
+ * made at fvm_create).  n > FVM_FLUX_NOALLOC_MAX is refused with FVM_EARG.
  * Calls that overlap on one GPU (from any context on that device) share that
  * array and race: serialise them. */
 #define FVM_FLUX_BYTES_PER_FACE 308 /* wij 3, Wi 10, Wj 10, normal 3, psi, Bn, flux 10 doubles + jbnd int */

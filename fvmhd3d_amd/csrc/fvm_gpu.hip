@@ -1948,8 +1948,10 @@ int fvm_get_active_faces(fvm_ctx *c, int *nface_active) {
     LAUNCH(c, fvm::k_face_firstpos, c->nactive, M, (const int *)c->field[FVM_FIELD_BND].p, c->nactive, firstpos);
     LAUNCH(c, fvm::k_face_firstflag, c->nactive, M, (const int *)c->field[FVM_FIELD_BND].p, c->nactive, firstpos, flag);
   }
-  // a substep without boundary cells: every face of its complete lists is active
-  const bool all = c->lists_complete && c->sub_layout && !c->sub.has_bnd;
+  // within a substep without boundary cells every face of its complete lists is
+  // active: has_bnd tells what the layout was gathered from, which a caller may
+  // have replaced since, on either side
+  const bool all = c->lists_complete && c->sub_layout && c->defer_sync && !c->sub.has_bnd;
   int total = all ? c->nface : 0;
   if (!all) LAUNCH(c, fvm::k_fill_int, c->nface, fpos, -1, c->nface);
   if (nref > 0) {

@@ -1,0 +1,76 @@
+"""What a substep leaves behind, and what it starts from: the layout in the
+context after fvm_substep_run stays usable through the other entry points."""
+import numpy as np
+import pytest
+
+from fvmhd3d_amd import gpu as G
+from fvmhd3d_amd import mesh as M
+from fvmhd3d_amd.substep import DeviceSubstepper, GpuBackend, Substepper, ic_disk
+from oracle.oracle import Oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def _mesh(n, seed):
+    pos = M.uniform_random(n, seed=seed)
+    return M.build_periodic(pos[M.morton_order(pos, (1, 1, 1))])
+
+
+def _partial_substep(m):
+    """A device substepper just after a substep with inactive neighbours, the host
+    driver of the same substeps, and that substep's layout (state, perm)."""
+    W = ic_disk(m.pos)
+    D = DeviceSubstepper(m, W, dtmax=0.25, limiter=G.LIMITER_SMOOTH)
+    H = Substepper(m, W, dtmax=0.25, limiter=G.LIMITER_SMOOTH)
+    B = GpuBackend(H.gamma, H.courant, tuple(float(b) for b in m.box), limiter=G.LIMITER_SMOOTH)
+    D.init_rungs()
+    H.init_rungs(B)
+    for k in range(16):
+        assert D.substep() == H.substep(B)
+        nact, _, nimp, _ = D.local_counts[-1]
+        if k > 2 and 0 < nact < m.ncell // 2 and nimp > 0:
+            break
+    else:
+        raise AssertionError("no partial substep")
+    active = np.zeros(m.ncell, dtype=bool)
+    active[H.last_active] = True
+    st, perm = H._state(active, H.last_active)
+    D.ctx.np = len(perm)
+    return D, H, st, perm
+
+
+def _lists_and_results(ctx, st):
+    for name in G.FIELDS:
+        ctx.upload(name, getattr(st, name))
+    ctx.set_time(st.t_global)
+    fa = ctx.get_active_faces()
+    ctx.compute_reconstruction()
+    ctx.slope_limiter()
+    ctx.compute_fluid_update(False)
+    return [fa] + [ctx.download(f) for f in ("x", "y", "z", "t", "lim", "dU", "dgp", "ddivB")]
+
+
+def test_layout_with_boundary_flags_lists_its_active_faces():
+    """Boundary flags uploaded to a substep's layout, then the active faces asked for
+    again: the list is that of the flags in the layout (the oracle's, on the same
+    layout), whatever flags the global state has had uploaded; the face-end lists
+    agree with those of a context that was given the layout as a mesh."""
+    m = _mesh(10 ** 3, 9)
+    D, H, st, perm = _partial_substep(m)
+    assert len(D.ctx.get_active_faces()) == len(st.faces)
+    rng = np.random.default_rng(2)
+    st.bnd[rng.choice(st.np, size=st.np // 3, replace=False)] = G.OUTFLOW
+    want = np.asarray(Oracle("f64", limiter=G.LIMITER_SMOOTH).get_active_faces(st.copy()))
+    assert 0 < len(want) < len(st.faces)
+    P = G.Context(gamma=H.gamma, courant=H.courant, box=st.box, limiter=G.LIMITER_SMOOTH)
+    P.upload_state(st)
+    ref = _lists_and_results(P, st)
+    assert np.array_equal(ref[0], want)
+    flags = np.zeros(m.ncell, np.int32)
+    for some in (0, 1, 0):
+        flags[:5] = some
+        D.ctx.substep_upload("bnd", flags)
+        for a, b in zip(_lists_and_results(D.ctx, st), ref):
+            assert np.array_equal(a, b)
+    P.close()
+    D.ctx.close()

@@ -590,24 +590,32 @@ int build_layout(fvm_ctx *c, unsigned mask, double t_global, int check, int *cou
   int nA = 0, nfl = 0, nI = 0, nref = 0;
   // the flag's copy completes with the scan's own synchronisation
   SCHK(c, hipMemcpyAsync(s.errh, s.err.p, sizeof(int), hipMemcpyDeviceToHost, st));
-  if (fvm::exclusive_scan_flags(c->scan, P<int>(s.act), P<int>(s.apos), n, &nA, st, P<int>(s.perm)))
+  if (fvm::exclusive_scan_flags(c->scan, P<int>(s.act), P<int>(s.apos), n, &nA, st, P<int>(s.oval2)))
     return fvm_fail(c, FVM_EHIP, "substep: scan of active cells failed");
   if (*s.errh & 1) return fvm_fail(c, FVM_ESTATE, "substep: an active cell does not end its step at the current time");
+  // so far the layout before this one is whole (perm, fmark, fpos and the mesh's
+  // arrays are read by its entry points); from here on there is none until the
+  // new one is complete (capacity for the whole mesh was reserved at setup)
+  c->have_mesh = false;
+  c->sub_layout = false;
+  c->nfa = -1;
+  fvm_fast_release(c);
   // the active list in the Scheduler's order: finest rung first, each rung in
   // push order (Scheduler.h pull_active_list)
   if (nA > 1) {
     const unsigned long long base = s.next_seq - (1ull << 32);
-    SLAUNCH(c, nA, k_sub_order_keys, P<int>(s.perm), nA, P<int>(s.rung), P<unsigned long long>(s.seq), base,
+    SLAUNCH(c, nA, k_sub_order_keys, P<int>(s.oval2), nA, P<int>(s.rung), P<unsigned long long>(s.seq), base,
             P<unsigned long long>(s.okey));
     if (nA <= kSmallSort) {
-      SLAUNCH(c, 64LL * nA, k_sub_rank_sort, P<int>(s.perm), P<unsigned long long>(s.okey), nA, P<int>(s.oval2),
+      SLAUNCH(c, 64LL * nA, k_sub_rank_sort, P<int>(s.oval2), P<unsigned long long>(s.okey), nA, P<int>(s.perm),
               P<int>(s.apos));
     } else {
       size_t tb = s.otmp_bytes;
       SCHK(c, rocprim::radix_sort_pairs(s.otmp.p, tb, P<unsigned long long>(s.okey), P<unsigned long long>(s.okey2),
-                                        P<int>(s.perm), P<int>(s.oval2), (unsigned)nA, 0, kKeyBits, st));
-      SLAUNCH(c, nA, k_sub_apos, P<int>(s.oval2), nA, P<int>(s.apos));
+                                        P<int>(s.oval2), P<int>(s.perm), (unsigned)nA, 0, kKeyBits, st));
+      SLAUNCH(c, nA, k_sub_apos, P<int>(s.perm), nA, P<int>(s.apos));
     }
+  } else {
     std::swap(s.perm, s.oval2);
   }
   SLAUNCH(c, nA, k_sub_face_counts, P<int>(s.perm), nA, P<int>(s.goff), P<int>(s.len));
@@ -627,11 +635,6 @@ int build_layout(fvm_ctx *c, unsigned mask, double t_global, int check, int *cou
   nref = c->scan.total_h[1];
   SLAUNCH(c, n, k_sub_g2l, P<int>(s.act), P<int>(s.apos), P<int>(s.iflag), P<int>(s.ipos), n, nA, P<int>(s.g2l));
   const int npl = nA + nI;
-  // the context's mesh (capacity for the whole mesh was reserved at setup);
-  // not valid until the layout is complete
-  c->have_mesh = false;
-  c->sub_layout = true;
-  fvm_fast_release(c);
   SLAUNCH(c, nfl, k_sub_local_faces, P<int>(s.fl), nfl, P<int>(s.gs1), P<int>(s.gs2), P<double>(s.gcn),
           P<double>(s.g[FVM_FIELD_POS]), P<int>(s.act), P<int>(s.g2l), c->prm.domain_size[0], c->prm.domain_size[1],
           c->prm.domain_size[2], P<int>(c->m_s1), P<int>(c->m_s2), P<double>(c->m_cn));
@@ -645,8 +648,8 @@ int build_layout(fvm_ctx *c, unsigned mask, double t_global, int check, int *cou
   c->nimport_loc = nI;
   c->nface = nfl;
   c->nref = nref;
-  c->nfa = -1;
   c->lists_complete = s.complete;  // active cells list all their faces when the global lists are complete
+  c->sub_layout = true;
   c->have_mesh = true;
   c->t_global = t_global;
   // the context's fields, one launch; the whole path follows unless only the

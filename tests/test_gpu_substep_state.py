@@ -74,3 +74,25 @@ def test_layout_with_boundary_flags_lists_its_active_faces():
             assert np.array_equal(a, b)
     P.close()
     D.ctx.close()
+
+
+def test_refused_substep_leaves_the_layout_before_it():
+    """A substep refused because its active cells do not end their step now: the
+    layout of the substep before it still gives its face lists and results (those
+    of a context that was given it as a mesh), and the substeps go on."""
+    m = _mesh(10 ** 3, 9)
+    D, H, st, perm = _partial_substep(m)
+    for every in (0xFFFFFFFF, 1 << D.max_rung()):  # every cell; the cells of the finest rung
+        with pytest.raises(G.FvmError) as e:
+            D.ctx.substep_run(every, -1.0, 0.25, 0, 6)
+        assert e.value.code == G.FVM_ESTATE
+    P = G.Context(gamma=H.gamma, courant=H.courant, box=st.box, limiter=G.LIMITER_SMOOTH)
+    P.upload_state(st)
+    for a, b in zip(_lists_and_results(D.ctx, st), _lists_and_results(P, st)):
+        assert np.array_equal(a, b)
+    B = GpuBackend(H.gamma, H.courant, st.box, limiter=G.LIMITER_SMOOTH)
+    for _ in range(3):
+        assert D.substep() == H.substep(B)
+    assert np.array_equal(D.state("W"), H.W)
+    P.close()
+    D.ctx.close()

@@ -424,9 +424,11 @@ __global__ void k_sub_order_keys(const int *__restrict__ perm, int nA, const int
 }
 
 // The same order for a short list, by ranks: a wavefront counts the keys below
-// one cell's (keys are distinct: the stamps are), four loads in flight; the list
-// in that order and each cell's place in it.  Each trip round the loop costs a
-// load's latency: 2100 keys with 16 lanes a key and one load 32 us, now 5.5.
+// one cell's, four loads in flight; the list in that order and each cell's place
+// in it.  Equal keys (stamps 2^32 apart; stamps a caller's state does not tell
+// apart) keep the order of the list, as in the radix sort of longer ones, so that
+// every rank is taken once.  Each trip round the loop costs a load's latency: 2100
+// keys with 16 lanes a key and one load 32 us, now 5.5.
 // (Bounded to 4096 keys, 16.8 M comparisons; a sort in one workgroup took 48 us.)
 constexpr int kSmallSort = 4096;
 __global__ void k_sub_rank_sort(const int *__restrict__ perm, const unsigned long long *__restrict__ key, int nA,
@@ -441,7 +443,10 @@ __global__ void k_sub_rank_sort(const int *__restrict__ perm, const unsigned lon
 #pragma unroll
     for (int u = 0; u < 4; u++) k[u] = key[min(m0 + 64 * u + l, nA - 1)];
 #pragma unroll
-    for (int u = 0; u < 4; u++) below += m0 + 64 * u + l < nA && k[u] < mine ? 1 : 0;
+    for (int u = 0; u < 4; u++) {
+      const int m = m0 + 64 * u + l;
+      below += m < nA && (k[u] < mine || (k[u] == mine && m < i)) ? 1 : 0;
+    }
   }
   for (int o = 32; o > 0; o >>= 1) below += __shfl_xor(below, o);
   if (l == 0) {
@@ -895,6 +900,10 @@ int fvm_substep_setup(fvm_ctx *c, int ncell, int nface, const fvm_face *faces, c
     }
   }
   SCHK(c, hipMemsetAsync(s.rung.p, 0, 4 * N, c->stream));
+  // every cell pushed in index order, until fvm_substep_init_rungs or for a state
+  // that is uploaded with its rungs
+  SLAUNCH(c, ncell, k_sub_iota64, P<unsigned long long>(s.seq), ncell);
+  s.next_seq = (unsigned long long)ncell;
   SCHK(c, hipStreamSynchronize(c->stream));
   if (nface > 0) {
     // same conversion as the mesh upload

@@ -285,7 +285,9 @@ int fvm_substep_setup(fvm_ctx *ctx, int ncell, int nface, const fvm_face *faces,
                       const int *cell_face, const double *cell_volume);
 /* per-cell fields kept between substeps (W, gradients, Wt, POS, J, TEND, BND,
  * MINMAX_LO/HI, DU, DGRADPSI, DDIVB, U, MESH_VOLUME, TBEG, DT_NEW) and the
- * rungs, host layout [ncell][width] in mesh order */
+ * rungs, host layout [ncell][width] in mesh order.  A state uploaded with its
+ * rungs and times can be run on without fvm_substep_init_rungs: its cells count
+ * as pushed in index order */
 int fvm_substep_upload(fvm_ctx *ctx, int field, const void *host, int ncell);
 int fvm_substep_download(fvm_ctx *ctx, int field, void *host, int ncell);
 /* first rungs from the CFL timestep of every cell (System.cpp:255-300, per cell) */

@@ -5,7 +5,7 @@ import pytest
 
 from fvmhd3d_amd import gpu as G
 from fvmhd3d_amd import mesh as M
-from fvmhd3d_amd.substep import DeviceSubstepper, GpuBackend, Substepper, ic_disk
+from fvmhd3d_amd.substep import DeviceSubstepper, GpuBackend, Substepper, ic_disk, ic_thin_disk
 from oracle.oracle import Oracle
 
 pytestmark = pytest.mark.gpu
@@ -16,12 +16,12 @@ def _mesh(n, seed):
     return M.build_periodic(pos[M.morton_order(pos, (1, 1, 1))])
 
 
-def _partial_substep(m):
+def _partial_substep(m, ic=ic_disk, dtmax=0.25):
     """A device substepper just after a substep with inactive neighbours, the host
     driver of the same substeps, and that substep's layout (state, perm)."""
-    W = ic_disk(m.pos)
-    D = DeviceSubstepper(m, W, dtmax=0.25, limiter=G.LIMITER_SMOOTH)
-    H = Substepper(m, W, dtmax=0.25, limiter=G.LIMITER_SMOOTH)
+    W = ic(m.pos)
+    D = DeviceSubstepper(m, W, dtmax=dtmax, limiter=G.LIMITER_SMOOTH)
+    H = Substepper(m, W, dtmax=dtmax, limiter=G.LIMITER_SMOOTH)
     B = GpuBackend(H.gamma, H.courant, tuple(float(b) for b in m.box), limiter=G.LIMITER_SMOOTH)
     D.init_rungs()
     H.init_rungs(B)
@@ -95,4 +95,38 @@ def test_refused_substep_leaves_the_layout_before_it():
         assert D.substep() == H.substep(B)
     assert np.array_equal(D.state("W"), H.W)
     P.close()
+    D.ctx.close()
+
+
+@pytest.mark.parametrize("case", ["disk_random_12", "thin_disk_lattice_17"])
+def test_uploaded_state_runs_in_index_order(case):
+    """A state taken between two substeps (fields, times and rungs) uploaded into a new
+    context and run on without fvm_substep_init_rungs: its cells count as pushed in
+    index order, and the substeps equal the host driver's with those stamps, bit for
+    bit.  17^3 = 4913 cells: active lists on both sides of 4096 cells, whose orders
+    come from two sorts."""
+    if case == "disk_random_12":
+        m, ic, dtmax = _mesh(12 ** 3, 9), ic_disk, 0.25
+    else:
+        m, ic, dtmax = M.workload_mesh("lattice", 17), ic_thin_disk, 0.125
+    _, H, _, _ = _partial_substep(m, ic, dtmax)
+    H.seq[:] = np.arange(m.ncell)
+    H.next_seq = m.ncell
+    D = DeviceSubstepper(m, H.W, dtmax=dtmax, limiter=G.LIMITER_SMOOTH)
+    for name in ("U", "x", "y", "z", "t", "mm_lo", "mm_hi", "J", "dU", "dgp", "ddivB", "mvol", "bnd", "tbeg", "tend",
+                 "dt_new", "rung"):
+        D.ctx.substep_upload(name, getattr(H, name))
+    D.clock.tsysU, D.clock.min_rung = H.clock.tsysU, H.clock.min_rung
+    D.hist = np.bincount(H.rung, minlength=32).astype(np.int32)
+    B = GpuBackend(H.gamma, H.courant, tuple(float(b) for b in m.box), limiter=G.LIMITER_SMOOTH)
+    nact = []
+    for k in range(32):
+        a, b = H.substep(B), D.substep()
+        assert a == b, k
+        nact.append(a[0])
+    assert np.all(np.isfinite(H.dU))
+    for name in ("W", "U", "dU", "t", "tend", "dt_new"):
+        assert np.array_equal(getattr(H, name), D.state(name).reshape(getattr(H, name).shape)), name
+    assert np.array_equal(H.rung, D.state("rung"))
+    assert m.ncell < 4096 or min(nact) <= 4096 < max(nact)
     D.ctx.close()

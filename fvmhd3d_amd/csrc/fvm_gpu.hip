@@ -2254,6 +2254,19 @@ void flux_stage_out(const FluxBatch &b, size_t f0, size_t n, const FluxStage &s)
   std::memcpy(b.flux + 10 * f0, s.out + 2 * n, 80 * n);
 }
 
+// outputs in memory that holds inputs: such a batch is taken up whole before any of
+// its results come down, where pieces would read what earlier ones have replaced
+bool flux_in_place(const FluxBatch &b, size_t n) {
+  const std::pair<const void *, size_t> in[] = {{b.wij, 24 * n}, {b.Wi, 80 * n}, {b.Wj, 80 * n}, {b.jbnd, 4 * n}, {b.normal, 24 * n}},
+                                        out[] = {{b.psi, 8 * n}, {b.Bn, 8 * n}, {b.flux, 80 * n}};
+  for (const auto &o : out)
+    for (const auto &i : in) {
+      const uintptr_t a = (uintptr_t)o.first, c = (uintptr_t)i.first;
+      if (a < c + i.second && c < a + o.second) return true;
+    }
+  return false;
+}
+
 hipError_t flux_chunk(double gamma, const FluxBatch &b, size_t f0, size_t n, char *h, char *d, hipStream_t st) {
   const FluxStage H = flux_stage(h, n), D = flux_stage(d, n);
   flux_stage_in(b, f0, n, H);
@@ -2329,7 +2342,8 @@ static int flux_batch_staged(fvm_ctx *c, char *base, bool threads, int n, const 
     HIPCHK(c, flux_pinned(c->prm.gamma_gas, b, N, c->pin, c->stream));
     return FVM_OK;
   }
-  if (threads && n >= 2 * FLUX_CHUNK) {
+  const bool whole = !threads || flux_in_place(b, N);
+  if (!whole && n >= 2 * FLUX_CHUNK) {
     hipError_t err = hipSuccess;
     HIPCHK(c, hipStreamSynchronize(c->stream));  // the staging may be in use by work before this call
     if (fvm_xfer_chunks(c, (n + FLUX_CHUNK - 1) / FLUX_CHUNK, [&](int k, char *slot, hipStream_t st) {
@@ -2340,11 +2354,12 @@ static int flux_batch_staged(fvm_ctx *c, char *base, bool threads, int n, const 
       return FVM_OK;
     }
   }
-  if (threads) {
+  if (!whole) {
     HIPCHK(c, flux_pieces(c->prm.gamma_gas, b, N, FLUX_PIN / 2, c->pin, (size_t)1 << 19, c->pin_ev, c->stream));
     return FVM_OK;
   }
-  // fvm_compute_flux_noalloc past the pinned staging: its fixed device array
+  // whole through the device staging: fvm_compute_flux_noalloc past the pinned
+  // staging (its fixed device array), and batches computed in place
   double *d_wij = (double *)base, *d_Wi = d_wij + 3 * N, *d_Wj = d_Wi + 10 * N, *d_n = d_Wj + 10 * N, *d_psi = d_n + 3 * N,
          *d_Bn = d_psi + N, *d_flux = d_Bn + N;
   int *d_jb = (int *)(d_flux + 10 * N);

@@ -165,7 +165,9 @@ int fvm_compute_timestep_limiter(fvm_ctx *ctx);
  * Scheduler's (Scheduler.h:15-25, 94-111) for the dt/128 probe */
 int fvm_compute_predictor(fvm_ctx *ctx, double dtmax, int min_rung);
 /* System::computeFlux for n independent faces (computeFlux.cpp:6-148), host
- * arrays: wij[n][3], Wi/Wj[n][10], jbnd[n], normal[n][3] -> psi[n], Bn[n], flux[n][10] */
+ * arrays: wij[n][3], Wi/Wj[n][10], jbnd[n], normal[n][3] -> psi[n], Bn[n], flux[n][10].
+ * Outputs may lie in the memory of inputs (not of one another): every input is
+ * read before an output is written */
 int fvm_compute_flux(fvm_ctx *ctx, int n, const double *wij, const double *Wi, const double *Wj,
                      const int *jbnd, const double *normal, double *psi, double *Bn, double *flux);
 /* fvm_compute_flux without any device allocation.  No counterpart in the

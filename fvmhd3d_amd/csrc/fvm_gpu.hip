@@ -860,7 +860,7 @@ __global__ void __launch_bounds__(256) k_timestep(Cells<S> C, MeshView M, Phys P
   }
   wave_sync();
   const int i = c0 + lane;
-  double v = REF_HUGE;
+  double v = HUGE_VAL;  // no cell
   if (lane < 4 * R && i < C.nactive) {
     const double g = P.gamma;
     const double Volume = C.mvol[i];
@@ -881,8 +881,9 @@ __global__ void __launch_bounds__(256) k_timestep(Cells<S> C, MeshView M, Phys P
     const double a = arg[wv][lane];
     if (a >= 0.0) dti = smin(dti, h / (csi + dsqrt(a)));
     dti = smin(dti, REF_HUGE);
-    v = dti * P.courant;
-    C.dt_new[i] = v;
+    const double dtn = dti * P.courant;
+    C.dt_new[i] = dtn;
+    if (dtn >= 0.0) v = dtn;  // a cell without a timestep (NaN) leaves the others theirs
   }
   // min over active cells; dt > 0 so the IEEE bit patterns order like the
   // values.  Atomics on one address take their turn (about 10 ns each), so a
@@ -894,7 +895,7 @@ __global__ void __launch_bounds__(256) k_timestep(Cells<S> C, MeshView M, Phys P
   if (threadIdx.x == 0) {
     for (int m = 1; m < 256 / 64; m++) v = smin(v, wmin[m]);
     const unsigned long long bits = (unsigned long long)__double_as_longlong(v);
-    if (c0 < C.nactive && v >= 0.0 && bits < __hip_atomic_load(dtmin_bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+    if (bits < __hip_atomic_load(dtmin_bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
       atomicMin(dtmin_bits, bits);
   }
 }

@@ -1441,7 +1441,17 @@ int fvm_ensure(fvm_ctx *c, DBuf &b, size_t bytes) {
   b.p = nullptr;
   b.bytes = 0;
   if (bytes == 0) bytes = 8;
-  HIPCHK(c, hipMalloc(&b.p, bytes));
+  hipError_t e = hipMalloc(&b.p, bytes);
+  if (e != hipSuccess && &b != &c->crow && c->crow.p) {
+    // the cell rows are optional: their memory goes to what cannot do without
+    (void)hipGetLastError();
+    fvm_release(c->crow);
+    e = hipMalloc(&b.p, bytes);
+  }
+  if (e != hipSuccess) {
+    b.p = nullptr;
+    return fvm_fail(c, FVM_EHIP, std::string("hipMalloc(&b.p, bytes): ") + hipGetErrorString(e));
+  }
   b.bytes = bytes;
   return FVM_OK;
 }

@@ -890,7 +890,6 @@ int fvm_substep_setup(fvm_ctx *c, int ncell, int nface, const fvm_face *faces, c
                            {&c->tmp0, 4 * (std::max(N, R) + 1)}, {&c->tmp1, 4 * (std::max(F, R) + 1)},
                            {&c->tmp2, 4 * (R + 1)}, {&c->rec, 8 * 16 * F} /* 16-double face records */})))
     return rc;
-  (void)fvm_cell_row_space(c, ncell, nface);  // without it the fields serve
   for (int f = 0; f < FVM_NFIELDS; f++) {
     const size_t bytes = (kInt[f] ? 4 : 8) * (size_t)kWidth[f] * N;
     if ((rc = fvm_ensure(c, c->field[f], bytes))) return rc;
@@ -899,6 +898,8 @@ int fvm_substep_setup(fvm_ctx *c, int ncell, int nface, const fvm_face *faces, c
       SCHK(c, hipMemsetAsync(s.g[f].p, 0, bytes, c->stream));
     }
   }
+  // last, from what memory is left: without the rows the fields serve
+  (void)fvm_cell_row_space(c, ncell, nface);
   SCHK(c, hipMemsetAsync(s.rung.p, 0, 4 * N, c->stream));
   // every cell pushed in index order, until fvm_substep_init_rungs or for a state
   // that is uploaded with its rungs

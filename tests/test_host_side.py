@@ -1,0 +1,110 @@
+"""The library's host side without a device: what it allocates and when it waits.
+
+libfvm_gpu.so runs in a process of its own over tests/hip_stub.c, which stands in
+for the HIP runtime (allocations from a budget on the host, kernels that do
+nothing), so device memory can be short at any chosen point."""
+import ctypes
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+ROW = 448  # bytes of a cell's row for the face flux kernel
+
+
+@pytest.fixture(scope="session")
+def stub(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("hip_stub") / "libamdhip64.so")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-O1", "-I/opt/rocm/include", "-Wl,-soname,libamdhip64.so.7", "-o", so,
+                    os.path.join(HERE, "hip_stub.c")], check=True)
+    return so
+
+
+def _apart(stub, case):
+    """Run a function of this file in a process that has the stub for a HIP runtime."""
+    code = (f"import sys; sys.path.insert(0, {ROOT!r})\n"
+            f"from tests import test_host_side as t\n"
+            f"t.{case}(t.Stub({stub!r}))\nprint('case done')\n")
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and r.stdout.endswith("case done\n"), r.stdout + r.stderr
+
+
+class Stub:
+    def __init__(self, so):
+        self.L = ctypes.CDLL(so, mode=ctypes.RTLD_GLOBAL)  # found by its name when the library asks for HIP
+        self.L.stub_used.restype = ctypes.c_size_t
+        self.L.stub_budget.argtypes = [ctypes.c_size_t]
+        self.L.stub_waits.restype = self.L.stub_launches.restype = ctypes.c_long
+
+    def used(self):
+        return self.L.stub_used()
+
+    def budget(self, n=None):
+        self.L.stub_budget(ctypes.c_size_t(-1).value if n is None else n)
+
+    def waits(self):
+        return self.L.stub_waits()
+
+
+def _random_mesh(n, nface, seed=1):
+    """Faces between random pairs of cells (no geometry) and complete cell lists."""
+    from fvmhd3d_amd.mesh import FACE_DTYPE
+    rng = np.random.default_rng(seed)
+    faces = np.zeros(nface, dtype=FACE_DTYPE)
+    assert faces.itemsize == 56
+    faces["s1"] = rng.integers(0, n, nface)
+    faces["s2"] = (faces["s1"] + rng.integers(1, n, nface)) % n
+    cell = np.concatenate([faces["s1"], faces["s2"]])
+    order = np.argsort(cell, kind="stable")
+    off = np.zeros(n + 1, np.int32)
+    off[1:] = np.cumsum(np.bincount(cell, minlength=n))
+    return faces, off, (order % nface).astype(np.int32), np.ones(n)
+
+
+def case_rows_come_last(S):
+    from fvmhd3d_amd import gpu as G
+    n = 20000
+    mesh = _random_mesh(n, 150000)
+
+    def setup(budget=None):
+        S.budget()
+        ctx = G.Context()
+        S.budget(budget)
+        ctx.substep_setup(*mesh)
+        return ctx
+
+    ctx = setup()
+    full = S.used()
+    ctx.close()
+    assert S.used() == 0
+    # room for everything but the rows: the setup goes without them
+    ctx = setup(full - ROW * n)
+    assert S.used() == full - ROW * n
+    ctx.close()
+    with pytest.raises(G.FvmError):
+        setup(full - ROW * n - 1)
+
+
+def case_rows_are_given_back(S):
+    from fvmhd3d_amd import gpu as G
+    n = 20000
+    ctx = G.Context()
+    ctx.substep_setup(*_random_mesh(n, 150000))
+    full = S.used()
+    S.budget(full + (1 << 20))
+    ctx.upload_mesh(n, n, 0, *_random_mesh(n, 150000))  # stages its face records: 56 bytes a face
+    assert abs(S.used() - (full - ROW * n + 56 * 150000)) < 256
+    ctx.close()
+
+
+@pytest.mark.parametrize("case", ["case_rows_come_last", "case_rows_are_given_back"])
+def test_optional_rows_yield_to_what_a_call_needs(stub, case):
+    """The face flux kernel reads its cells from rows where there is memory for them
+    (448 bytes a cell); without them it reads the fields.  fvm_substep_setup needs
+    no more memory than its other buffers, and a later allocation that fails gets
+    the rows' memory."""
+    _apart(stub, case)

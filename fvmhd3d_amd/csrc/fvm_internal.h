@@ -169,6 +169,7 @@ bool fvm_xfer_run(fvm_ctx *c, int n, hipError_t (*chunk)(void *, int, char *, hi
 template <typename F> bool fvm_xfer_chunks(fvm_ctx *c, int n, F chunk, hipError_t *err) {
   return fvm_xfer_run(c, n, [](void *f, int k, char *slot, hipStream_t st) { return (*(F *)f)(k, slot, st); }, &chunk, err);
 }
+// (the caller waits for the stream)
 int fvm_to_device(fvm_ctx *c, void *dst, const void *src, size_t bytes);
 int fvm_to_host(fvm_ctx *c, void *dst, const void *src, size_t bytes);
 

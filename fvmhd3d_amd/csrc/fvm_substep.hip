@@ -973,7 +973,10 @@ int fvm_substep_upload(fvm_ctx *c, int field, const void *host, int ncell) {
     const int *b = (const int *)host;
     s.has_bnd = std::any_of(b, b + ncell, [](int v) { return v != FVM_NO_BOUNDARY; });
   }
-  return fvm_to_device(c, s.g[field].p, host, (kInt[field] ? 4 : 8) * (size_t)kWidth[field] * ncell);
+  const int rc = fvm_to_device(c, s.g[field].p, host, (kInt[field] ? 4 : 8) * (size_t)kWidth[field] * ncell);
+  if (rc) return rc;
+  SCHK(c, hipStreamSynchronize(c->stream));
+  return FVM_OK;
 }
 
 int fvm_substep_download(fvm_ctx *c, int field, void *host, int ncell) {

@@ -108,3 +108,25 @@ def test_optional_rows_yield_to_what_a_call_needs(stub, case):
     no more memory than its other buffers, and a later allocation that fails gets
     the rows' memory."""
     _apart(stub, case)
+
+
+def case_one_wait_a_field(S):
+    from fvmhd3d_amd import gpu as G
+    n = 20000
+    ctx = G.Context()
+    ctx.upload_mesh(n, n, 0, *_random_mesh(n, 150000))
+    ctx.substep_setup(*_random_mesh(n, 150000))
+    for name, (_, width, kind) in G.FIELDS.items():
+        a = np.zeros((n, width), np.int32 if kind == "i" else np.float64)
+        for call in (ctx.upload, ctx.download, ctx.substep_upload):
+            if call == ctx.substep_upload and name not in ("w", "U", "pos", "tend", "bnd"):
+                continue
+            before = S.waits()
+            call(name, a) if call != ctx.download else call(name)
+            assert S.waits() == before + 1, (name, call.__name__)
+    ctx.close()
+
+
+def test_field_transfers_wait_once(stub):
+    """A field of less than 8 MiB goes up or down with one wait for the stream."""
+    _apart(stub, "case_one_wait_a_field")

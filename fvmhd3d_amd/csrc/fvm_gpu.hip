@@ -2278,6 +2278,14 @@ bool flux_in_place(const FluxBatch &b, size_t n) {
   return false;
 }
 
+// every array within reach of the DMA
+bool flux_all_pinned(const FluxBatch &b) {
+  for (const void *p : {(const void *)b.wij, (const void *)b.Wi, (const void *)b.Wj, (const void *)b.jbnd, (const void *)b.normal,
+                        (const void *)b.psi, (const void *)b.Bn, (const void *)b.flux})
+    if (fvm_pageable(p)) return false;
+  return true;
+}
+
 hipError_t flux_chunk(double gamma, const FluxBatch &b, size_t f0, size_t n, char *h, char *d, hipStream_t st) {
   const FluxStage H = flux_stage(h, n), D = flux_stage(d, n);
   flux_stage_in(b, f0, n, H);
@@ -2340,6 +2348,10 @@ hipError_t flux_pieces(double gamma, const FluxBatch &b, size_t n, size_t piece,
 // copies of pageable memory).
 constexpr int FLUX_PIN = (1 << 20) / FVM_FLUX_BYTES_PER_FACE;
 constexpr int FLUX_CHUNK = 16384;
+// Batches in arrays that are pinned themselves go whole from about where the DMA's
+// own copies overtake the host's into the staging (14 000 faces 172 us whole, 166 in
+// pieces; 16 384 182 and 191; 20 000 204 and 231; 60 000 419 and by chunks 480).
+constexpr int FLUX_WHOLE_PINNED = 16384;
 static_assert((size_t)FLUX_CHUNK * FVM_FLUX_BYTES_PER_FACE <= fvm::kXferSlot, "a chunk fits a slot");
 
 // the batched computeFlux through device staging at base (room for n faces:
@@ -2353,7 +2365,7 @@ static int flux_batch_staged(fvm_ctx *c, char *base, bool threads, int n, const 
     HIPCHK(c, flux_pinned(c->prm.gamma_gas, b, N, c->pin, c->stream));
     return FVM_OK;
   }
-  const bool whole = !threads || flux_in_place(b, N);
+  const bool whole = !threads || flux_in_place(b, N) || (n >= FLUX_WHOLE_PINNED && flux_all_pinned(b));
   if (!whole && n >= 2 * FLUX_CHUNK) {
     hipError_t err = hipSuccess;
     HIPCHK(c, hipStreamSynchronize(c->stream));  // the staging may be in use by work before this call
@@ -2370,7 +2382,8 @@ static int flux_batch_staged(fvm_ctx *c, char *base, bool threads, int n, const 
     return FVM_OK;
   }
   // whole through the device staging: fvm_compute_flux_noalloc past the pinned
-  // staging (its fixed device array), and batches computed in place
+  // staging (its fixed device array), batches computed in place and large ones in
+  // pinned arrays
   double *d_wij = (double *)base, *d_Wi = d_wij + 3 * N, *d_Wj = d_Wi + 10 * N, *d_n = d_Wj + 10 * N, *d_psi = d_n + 3 * N,
          *d_Bn = d_psi + N, *d_flux = d_Bn + N;
   int *d_jb = (int *)(d_flux + 10 * N);

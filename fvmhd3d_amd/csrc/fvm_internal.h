@@ -165,6 +165,7 @@ void fvm_release(DBuf &b);
 // host transfers (fvm_xfer.hip)
 void fvm_xfer_ref();
 void fvm_xfer_unref(fvm_ctx *c);
+bool fvm_pageable(const void *p);
 bool fvm_xfer_run(fvm_ctx *c, int n, hipError_t (*chunk)(void *, int, char *, hipStream_t), void *arg, hipError_t *err);
 template <typename F> bool fvm_xfer_chunks(fvm_ctx *c, int n, F chunk, hipError_t *err) {
   return fvm_xfer_run(c, n, [](void *f, int k, char *slot, hipStream_t st) { return (*(F *)f)(k, slot, st); }, &chunk, err);

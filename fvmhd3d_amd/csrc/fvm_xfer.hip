@@ -60,6 +60,16 @@ void fvm_xfer_unref(fvm_ctx *c) {
   }
 }
 
+// Whether the runtime would have to copy p through memory of its own.  The DMA
+// reaches pinned arrays directly, faster than through the slots: 18 MB down 366 us
+// against 544, a computeFlux batch of 500,001 faces 2.8 ms against 3.3.
+bool fvm_pageable(const void *p) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeUnregistered;
+  (void)hipGetLastError();
+  return true;
+}
+
 // chunk(arg, k, slot, stream) for k = 0 .. n - 1 on up to kXferThreads threads, the
 // caller among them; false: the slots are in use or could not be had, nothing
 // was done.  *err receives the first failure.
@@ -107,7 +117,7 @@ bool fvm_xfer_run(fvm_ctx *c, int n, hipError_t (*chunk)(void *, int, char *, hi
 // a 32^3 state 3.91 -> 3.99 ms).
 static int copy_host(fvm_ctx *c, void *dst, const void *src, size_t bytes, bool down) {
   hipError_t err = hipSuccess;
-  if (bytes >= fvm::kXferMin) {
+  if (bytes >= fvm::kXferMin && fvm_pageable(down ? dst : src)) {
     FVM_HIPCHK(c, hipStreamSynchronize(c->stream));
     const int n = (int)((bytes + fvm::kXferSlot - 1) / fvm::kXferSlot);
     const bool done = fvm_xfer_chunks(c, n, [&](int k, char *slot, hipStream_t st) {

@@ -10,12 +10,17 @@
 #include <hip/hip_runtime_api.h>
 
 static size_t used, budget = (size_t)-1;
-static long waits, launches;
+static long waits, launches, copies;
+static struct {
+  char *p;
+  size_t n;
+} pinned[256]; /* live hipHostMalloc blocks */
 
 size_t stub_used(void) { return used; }
 void stub_budget(size_t bytes) { budget = bytes; }
 long stub_waits(void) { return waits; }
 long stub_launches(void) { return launches; }
+long stub_copies(void) { return copies; }
 
 hipError_t hipMalloc(void **p, size_t n) {
   if (n > budget || used > budget - n) return hipErrorOutOfMemory;
@@ -34,18 +39,34 @@ hipError_t hipFree(void *p) {
   return hipSuccess;
 }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned flags) {
-  *p = calloc(1, n);
-  return *p ? hipSuccess : hipErrorOutOfMemory;
+  int i = 0;
+  while (i < 256 && pinned[i].p) i++;
+  if (i == 256 || !(*p = calloc(1, n))) return hipErrorOutOfMemory;
+  pinned[i].p = *p;
+  pinned[i].n = n;
+  return hipSuccess;
 }
 hipError_t hipHostFree(void *p) {
+  for (int i = 0; i < 256; i++)
+    if (pinned[i].p == p) pinned[i].p = 0;
   free(p);
+  return hipSuccess;
+}
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p) {
+  memset(a, 0, sizeof *a);
+  a->type = hipMemoryTypeUnregistered;
+  for (int i = 0; i < 256; i++)
+    if (pinned[i].p && (char *)p >= pinned[i].p && (char *)p < pinned[i].p + pinned[i].n) a->type = hipMemoryTypeHost;
   return hipSuccess;
 }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind k) {
   memcpy(d, s, n);
   return hipSuccess;
 }
-hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t st) { return hipMemcpy(d, s, n, k); }
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t st) {
+  __atomic_add_fetch(&copies, 1, __ATOMIC_RELAXED);
+  return hipMemcpy(d, s, n, k);
+}
 hipError_t hipMemset(void *d, int v, size_t n) {
   memset(d, v, n);
   return hipSuccess;

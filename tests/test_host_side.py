@@ -38,7 +38,8 @@ class Stub:
         self.L = ctypes.CDLL(so, mode=ctypes.RTLD_GLOBAL)  # found by its name when the library asks for HIP
         self.L.stub_used.restype = ctypes.c_size_t
         self.L.stub_budget.argtypes = [ctypes.c_size_t]
-        self.L.stub_waits.restype = self.L.stub_launches.restype = ctypes.c_long
+        self.L.stub_waits.restype = self.L.stub_launches.restype = self.L.stub_copies.restype = ctypes.c_long
+        self.L.hipHostMalloc.argtypes = [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_uint]
 
     def used(self):
         return self.L.stub_used()
@@ -48,6 +49,14 @@ class Stub:
 
     def waits(self):
         return self.L.stub_waits()
+
+    def copies(self):
+        return self.L.stub_copies()
+
+    def pinned(self, shape, dtype=np.float64):
+        n, p = int(np.prod(shape)) * np.dtype(dtype).itemsize, ctypes.c_void_p()
+        assert self.L.hipHostMalloc(ctypes.byref(p), n, 0) == 0
+        return np.frombuffer((ctypes.c_char * n).from_address(p.value), dtype=dtype).reshape(shape)
 
 
 def _random_mesh(n, nface, seed=1):
@@ -130,3 +139,31 @@ def case_one_wait_a_field(S):
 def test_field_transfers_wait_once(stub):
     """A field of less than 8 MiB goes up or down with one wait for the stream."""
     _apart(stub, "case_one_wait_a_field")
+
+
+def case_pinned_arrays_are_not_staged(S):
+    from fvmhd3d_amd import gpu as G
+    n = 120000  # a ten-wide field: 9.6 MB, two slots
+    ctx = G.Context()
+    ctx.upload_mesh(n, n, 0, *_random_mesh(n, 130000))
+    for new, copies in ((np.zeros, 2), (S.pinned, 1)):
+        a = new((n, 10))
+        for call in (ctx.L.fvm_upload_field, ctx.L.fvm_download_field):
+            before = S.copies()
+            ctx._chk(call(ctx.h, G.FIELDS["w"][0], a.ctypes.data, n))
+            assert S.copies() == before + copies
+    n = 40000  # faces: three chunks of three copies each, or the eight arrays
+    shapes = [((n, 3), float), ((n, 10), float), ((n, 10), float), (n, np.int32), ((n, 3), float), (n, float), (n, float),
+              ((n, 10), float)]
+    for new, copies in ((np.zeros, 9), (S.pinned, 8)):
+        arrays = [new(*s) for s in shapes]
+        before = S.copies()
+        ctx._chk(ctx.L.fvm_compute_flux(ctx.h, n, *[a.ctypes.data for a in arrays]))
+        assert S.copies() == before + copies
+    ctx.close()
+
+
+def test_pinned_arrays_are_copied_directly(stub):
+    """Arrays that are pinned themselves go to and from the device in one copy each,
+    not through the pinned slots."""
+    _apart(stub, "case_pinned_arrays_are_not_staged")

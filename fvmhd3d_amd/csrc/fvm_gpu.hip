@@ -2354,10 +2354,12 @@ constexpr int FLUX_CHUNK = 16384;
 constexpr int FLUX_WHOLE_PINNED = 16384;
 static_assert((size_t)FLUX_CHUNK * FVM_FLUX_BYTES_PER_FACE <= fvm::kXferSlot, "a chunk fits a slot");
 
-// the batched computeFlux through device staging at base (room for n faces:
-// FVM_FLUX_BYTES_PER_FACE each), synchronous; threads: the transfer threads may
-// be used (their slots and streams are allocated on first use)
-static int flux_batch_staged(fvm_ctx *c, char *base, bool threads, int n, const double *wij, const double *Wi, const double *Wj,
+// the batched computeFlux, synchronous.  fixed: device staging with room for n faces
+// (FVM_FLUX_BYTES_PER_FACE each), and nothing may be allocated; null: the context's
+// staging, where the route has one (without the memory for it a batch goes in
+// pieces), and the transfer threads, whose slots and streams are allocated on
+// first use
+static int flux_batch_staged(fvm_ctx *c, char *fixed, int n, const double *wij, const double *Wi, const double *Wj,
                              const int *jbnd, const double *normal, double *psi, double *Bn, double *flux) {
   const size_t N = (size_t)n;
   const FluxBatch b{wij, Wi, Wj, jbnd, normal, psi, Bn, flux};
@@ -2365,8 +2367,20 @@ static int flux_batch_staged(fvm_ctx *c, char *base, bool threads, int n, const 
     HIPCHK(c, flux_pinned(c->prm.gamma_gas, b, N, c->pin, c->stream));
     return FVM_OK;
   }
-  const bool whole = !threads || flux_in_place(b, N) || (n >= FLUX_WHOLE_PINNED && flux_all_pinned(b));
-  if (!whole && n >= 2 * FLUX_CHUNK) {
+  const bool in_place = flux_in_place(b, N);
+  bool whole = fixed || in_place || (n >= FLUX_WHOLE_PINNED && flux_all_pinned(b));
+  char *base = fixed;
+  if (!fixed && (whole || n >= 2 * FLUX_CHUNK)) {
+    const int rc = ensure(c, c->stage, (size_t)FVM_FLUX_BYTES_PER_FACE * N);
+    if (rc && in_place) return rc;
+    if (rc) {
+      (void)hipGetLastError();
+      whole = false;
+    } else {
+      base = (char *)c->stage.p;
+    }
+  }
+  if (!whole && base) {
     hipError_t err = hipSuccess;
     HIPCHK(c, hipStreamSynchronize(c->stream));  // the staging may be in use by work before this call
     if (fvm_xfer_chunks(c, (n + FLUX_CHUNK - 1) / FLUX_CHUNK, [&](int k, char *slot, hipStream_t st) {
@@ -2407,9 +2421,7 @@ int fvm_compute_flux(fvm_ctx *c, int n, const double *wij, const double *Wi, con
   if (n == 0) return FVM_OK;
   if (!wij || !Wi || !Wj || !jbnd || !normal || !psi || !Bn || !flux) return fail(c, FVM_EARG, "NULL array");
   (void)hipSetDevice(c->device);
-  int rc = ensure(c, c->stage, (size_t)FVM_FLUX_BYTES_PER_FACE * (size_t)n);
-  if (rc) return rc;
-  return flux_batch_staged(c, (char *)c->stage.p, true, n, wij, Wi, Wj, jbnd, normal, psi, Bn, flux);
+  return flux_batch_staged(c, nullptr, n, wij, Wi, Wj, jbnd, normal, psi, Bn, flux);
 }
 
 int fvm_compute_flux_noalloc(fvm_ctx *c, int n, const double *wij, const double *Wi, const double *Wj,
@@ -2424,7 +2436,7 @@ int fvm_compute_flux_noalloc(fvm_ctx *c, int n, const double *wij, const double 
   (void)hipSetDevice(c->device);
   char *base = (char *)noalloc_scratch(c->device);
   if (!base) return fail(c, FVM_ESTATE, "fvm_compute_flux_noalloc: no staging address for this device");
-  return flux_batch_staged(c, base, false, n, wij, Wi, Wj, jbnd, normal, psi, Bn, flux);
+  return flux_batch_staged(c, base, n, wij, Wi, Wj, jbnd, normal, psi, Bn, flux);
 }
 
 int fvm_get_diagnostics(fvm_ctx *c, long long *out, int n) {

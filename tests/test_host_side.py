@@ -167,3 +167,39 @@ def test_pinned_arrays_are_copied_directly(stub):
     """Arrays that are pinned themselves go to and from the device in one copy each,
     not through the pinned slots."""
     _apart(stub, "case_pinned_arrays_are_not_staged")
+
+
+def case_flux_without_staging(S):
+    from fvmhd3d_amd import gpu as G
+    ctx = G.Context()
+
+    def arrays(n):
+        return [np.zeros((n, 3)), np.zeros((n, 10)), np.zeros((n, 10)), np.zeros(n, np.int32), np.zeros((n, 3)), np.zeros(n),
+                np.zeros(n), np.zeros((n, 10))]
+
+    def run(a):
+        ctx._chk(ctx.L.fvm_compute_flux(ctx.h, len(a[0]), *[x.ctypes.data for x in a]))
+
+    before = S.used()
+    for n in (300, 5000, 32767):
+        run(arrays(n))
+    assert S.used() == before  # these routes have no device staging
+    S.budget(before)
+    for n in (32768, 100000):
+        run(arrays(n))
+    assert S.used() == before
+    a = arrays(40000)
+    a[7] = a[1]  # the flux in Wi
+    with pytest.raises(G.FvmError):
+        run(a)
+    S.budget()
+    run(a)
+    assert S.used() == before + 308 * 40000
+    ctx.close()
+
+
+def test_flux_batches_without_device_memory(stub):
+    """computeFlux allocates device staging for the routes that use it only, and takes
+    a batch in pieces where there is no memory for it; a batch computed in its
+    inputs' memory needs it and is refused."""
+    _apart(stub, "case_flux_without_staging")

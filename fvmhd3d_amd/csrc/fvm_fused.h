@@ -211,7 +211,13 @@ __device__ __forceinline__ void decode_fe(const FaceEndRec<T> &r, FE<T> &g) {
   }
   const T dsh = g.drL[0] * g.nrm[0] + g.drL[1] * g.nrm[1] + g.drL[2] * g.nrm[2];
   const T dsl = T(2.0) * dsh;
-  for (int d = 0; d < 3; d++) g.drR[d] = g.drL[d] - g.nrm[d] * dsl;
+  // FP32: the fused operation spelled out.  With moving generators n dsl is needed
+  // again (face_velocity), and the compiler then fuses it here or not by the code
+  // around it: not in the quad predictor kernel, which put its gradients an ulp off
+  for (int d = 0; d < 3; d++) {
+    if constexpr (std::is_same<T, float>::value) g.drR[d] = __builtin_fmaf(-g.nrm[d], dsl, g.drL[d]);
+    else g.drR[d] = g.drL[d] - g.nrm[d] * dsl;
+  }
   if constexpr (std::is_same<T, double>::value) {
     // the reference's reconstruction geometry (computeReconstruction.cpp:97-123)
     g.area = dabs(r.area);
@@ -1812,7 +1818,9 @@ template <typename T> int fused_setup_t(fvm_ctx *c) {
 int sg_step_launch(fvm_ctx *c, const FusedArgs<float> &A);
 
 template <typename T, bool MOVING, int LIM> int launch_step(fvm_ctx *c, const FusedArgs<T> &A, hipEvent_t *ev) {
-  const bool quads = c->np <= quad_cells<T>();
+  // FVM_FUSED_ONE_LANE set: the one-lane kernels at every size (so that small meshes
+  // exercise them)
+  const bool quads = c->np <= quad_cells<T>() && std::getenv("FVM_FUSED_ONE_LANE") == nullptr;
   const unsigned grid = fused_grid(c->np), qgrid = quads ? fused_grid(4 * c->np) : 0;
   const auto k1 = [&](const FusedArgs<T> &a) {
     if (quads) hipLaunchKernelGGL((k_cfl_predict_recon_quad<T, MOVING, LIM>), dim3(qgrid), dim3(FB), 0, c->stream, a);

@@ -16,9 +16,10 @@
 //                   order in which the previous layer's accumulator tiles land
 //                   in the lanes, so no transpose is needed between layers),
 //                   then gates and assembles the FP64 flux; weights stay in LDS
-//   fallback        every face the gate rejects is appended to a list (wave
-//                   ballot + one atomic per wave) and a second launch runs the
-//                   FP64 computeFlux on it
+//   fallback        every face the gate rejects is appended to a list (gathered
+//                   in LDS, one atomic addition per 128 of a wavefront's and
+//                   one per block) and a second launch runs the FP64
+//                   computeFlux on it
 //
 // Compiled with -ffp-contract=off so the FP64 Dedner terms and the fallback
 // are operation-for-operation the reference's.

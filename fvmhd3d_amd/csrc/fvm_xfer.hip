@@ -5,12 +5,14 @@
 // memory.  Large transfers here go through four pinned slots, one per thread: a
 // thread copies between its slot and the caller's array while the other slots'
 // DMA runs, in both directions at once where a batch is computed chunk by chunk.
-// Measured: a computeFlux batch of 500,001 faces 7.9 -> 4.0 ms (small batches, through
-// the context's own pinned staging: 2048 faces 130 -> 65 us); 20 steps of 128^3
-// cells with their 168 MB of U read back 47.6 -> 39.0 ms.
+// Measured: a computeFlux batch of 500,001 faces 7.9 -> 4.0 ms (smaller batches go
+// through the context's own pinned staging, fvm_gpu.hip); 20 steps of 128^3 cells
+// with their 168 MB of U read back 47.6 -> 39.0 ms.
 //
 // The slots belong to the process (20 MB, allocated on first use, freed with the
-// last context): a transfer that finds them in use takes the runtime's copies.
+// last context).  While they are in use, by one context at a time, other fields
+// take the runtime's copies and other flux batches go in pieces through their
+// context's staging.
 #include <hip/hip_runtime.h>
 
 #include <atomic>

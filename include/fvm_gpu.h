@@ -245,7 +245,8 @@ int fvm_fused_kernel_ms(fvm_ctx *ctx, double *ms, long long *launches, int n);
  * reference. */
 #define FVM_KT_RECONSTRUCTION 0  /* k_reconstruction (computeReconstruction) */
 #define FVM_KT_SLOPE_LIMITER 1   /* k_slope_limiter (slopeLimiter + computeFluidUpdateI) */
-#define FVM_KT_FACE_FLUX 2       /* k_face_flux (computeFluidUpdate, face part) */
+#define FVM_KT_FACE_FLUX 2       /* k_face_flux (computeFluidUpdate, face part); not the launch that
+                                  * writes the rows it reads its cells from (131072 faces and more) */
 #define FVM_KT_SCATTER 3         /* k_scatter (computeFluidUpdate, per-cell sums) */
 #define FVM_KT_PRIMITIVES 4      /* k_primitives (computePrimitives) */
 #define FVM_KT_TIMESTEP 5        /* k_timestep (computeTimestep) */

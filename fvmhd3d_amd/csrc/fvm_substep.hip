@@ -884,9 +884,23 @@ int fvm_substep_setup(fvm_ctx *c, int ncell, int nface, const fvm_face *faces, c
   // the context's mesh, fields and the path's scratch at their largest (every
   // cell local), so that no substep grows a buffer
   const size_t R = (size_t)nref;
-  if ((rc = ensure_all(c, {{&c->m_s1, 4 * F}, {&c->m_s2, 4 * F}, {&c->m_cn, 48 * F}, {&c->m_fpos, 4 * (F + 1)},
-                           {&c->m_coff, 4 * (N + 1)}, {&c->m_cface, 4 * R}, {&c->m_cnbr, 4 * R}, {&c->m_cvol, 8 * N},
-                           {&c->m_soff, 4 * (N + 1)}, {&c->m_sent, 8 * F + 4}, {&c->m_fact, 4 * (F + 1)},
+  const std::initializer_list<std::pair<DBuf *, size_t>> mesh = {
+      {&c->m_s1, 4 * F},        {&c->m_s2, 4 * F},  {&c->m_cn, 48 * F},  {&c->m_coff, 4 * (N + 1)},
+      {&c->m_cface, 4 * R},     {&c->m_cnbr, 4 * R}, {&c->m_cvol, 8 * N}};
+  const std::initializer_list<std::pair<DBuf *, size_t>> lists = {
+      {&c->m_soff, 4 * (N + 1)}, {&c->m_sent, 8 * F + 4}, {&c->m_fact, 4 * (F + 1)}};
+  // a buffer that has to grow loses what the context's mesh, its fields or its
+  // active faces have in it
+  const auto grows = [](const DBuf &b, size_t bytes) { return b.p && b.bytes < bytes; };
+  for (auto &e : lists)
+    if (grows(*e.first, e.second)) c->nfa = -1;
+  for (auto &e : mesh)
+    if (grows(*e.first, e.second)) c->have_mesh = false;
+  for (int f = 0; f < FVM_NFIELDS; f++)
+    if (grows(c->field[f], (kInt[f] ? 4 : 8) * (size_t)kWidth[f] * N)) c->have_mesh = false;
+  if (!c->have_mesh) c->nfa = -1;
+  if ((rc = ensure_all(c, mesh)) || (rc = ensure_all(c, lists)) ||
+      (rc = ensure_all(c, {{&c->m_fpos, 4 * (F + 1)},
                            {&c->tmp0, 4 * (std::max(N, R) + 1)}, {&c->tmp1, 4 * (std::max(F, R) + 1)},
                            {&c->tmp2, 4 * (R + 1)}, {&c->rec, 8 * 16 * F} /* 16-double face records */})))
     return rc;

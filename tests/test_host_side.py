@@ -119,6 +119,37 @@ def test_optional_rows_yield_to_what_a_call_needs(stub, case):
     _apart(stub, case)
 
 
+def case_setup_of_a_larger_mesh(S):
+    from fvmhd3d_amd import gpu as G
+    n = 20000
+    mesh = _random_mesh(n, 150000)
+    ctx = G.Context()
+    ctx.upload_mesh(n, n, 0, *mesh)
+    ctx.substep_setup(*mesh)
+    assert ctx.L.fvm_compute_reconstruction(ctx.h) == G.FVM_OK  # every buffer is where it was
+    before, full = S.used(), None
+    for short in (False, True):
+        c = G.Context()
+        c.upload_mesh(1000, 1000, 0, *_random_mesh(1000, 8000))
+        if short:  # for the last of the buffers that the path cannot do without
+            S.budget(full - ROW * n - 1)
+            with pytest.raises(G.FvmError):
+                c.substep_setup(*mesh)
+        else:
+            c.substep_setup(*mesh)
+            full = S.used()
+        assert c.L.fvm_compute_reconstruction(c.h) == G.FVM_ESTATE
+        c.close()
+        assert S.used() == before
+    ctx.close()
+
+
+def test_setup_of_a_larger_mesh_ends_the_one_before(stub):
+    """fvm_substep_setup makes room for its mesh in the context's buffers: where one of
+    them moves, or cannot be had, the mesh uploaded before is gone."""
+    _apart(stub, "case_setup_of_a_larger_mesh")
+
+
 def case_one_wait_a_field(S):
     from fvmhd3d_amd import gpu as G
     n = 20000
